@@ -615,6 +615,18 @@ int petch_dda_neutral_flux(petch_ctx* ctx, const float* phi, int nx, int ny, int
                            const float* centroids, const float* gas_normals, const float* areas,
                            const float* bare, int F, const petch_dda_params* p, float* m_a,
                            float* m_b);
+/* The two halves of petch_dda_neutral_flux, for callers that solve several coverages on one
+ * surface (the rounds of mc_flux_3d_dda): petch_dda_march marches every face's rays once into
+ * plan, 3 * 2 n_dir + F * (1 + 2 n_dir) 4-byte words (the directions, the sky's share of every
+ * face, every ray's end); petch_dda_reemit runs the re-emission passes over a plan of the same
+ * phi, faces, dx, n_dir and periodic_y. */
+int petch_dda_march(petch_ctx* ctx, const float* phi, int nx, int ny, int nz,
+                    const float* centroids, const float* gas_normals, int F,
+                    const petch_dda_params* p, int* plan);
+int petch_dda_reemit(petch_ctx* ctx, const float* phi, int nx, int ny, int nz,
+                     const float* centroids, const float* gas_normals, const float* areas,
+                     const float* bare, int F, const petch_dda_params* p, const int* plan,
+                     float* m_a, float* m_b);
 
 /* ---------------------------------------------------------------- a21: radiosity -------- */
 /* Form-factor assembly of mc_flux_3d_radiosity (threed.py:956-960) from the petch_trace_ff

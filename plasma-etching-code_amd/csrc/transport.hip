@@ -255,13 +255,13 @@ __device__ __forceinline__ int round_cell(float q, float dx, int n) {
   return c < 0 ? 0 : (c > n - 1 ? n - 1 : c);
 }
 
-// The value one direction ray brings back to origin o (dda.py:44-93, in the reference's float32
-// order, no contraction): from o + 1.01 dx d in steps of dx d, src_top once z >= z_top; at the
-// first point whose trilinear phi (coordinates clamped to [0, n - 1.001]) is > 0 the remit of
-// the first solid rounded cell among six half steps on, else of the point's rounded cell; 0
-// after max_steps. remit may be NULL (all zero).
-__device__ float dda_ray(const DdaGrid& g, float ox, float oy, float oz, float dxv, float dyv,
-                         float dzv, const float* __restrict__ remit, float src_top) {
+// Where one direction ray from origin o ends (dda.py:44-93, in the reference's float32 order, no
+// contraction): from o + 1.01 dx d in steps of dx d, kDdaSky once z >= z_top; at the first point
+// whose trilinear phi (coordinates clamped to [0, n - 1.001]) is > 0 the first solid rounded cell
+// among six half steps on, else the point's rounded cell; kDdaNone after max_steps.
+constexpr int kDdaSky = -1, kDdaNone = -2;
+__device__ int dda_ray(const DdaGrid& g, float ox, float oy, float oz, float dxv, float dyv,
+                       float dzv) {
 #pragma clang fp contract(off)
   const float dx = g.dx;
   float px = ox + dxv * dx * 1.01f;
@@ -270,7 +270,7 @@ __device__ float dda_ray(const DdaGrid& g, float ox, float oy, float oz, float d
   const float sx = dxv * dx, sy = dyv * dx, sz = dzv * dx;
   const float ux = (float)g.nx - 1.001f, uy = (float)g.ny - 1.001f, uz = (float)g.nz - 1.001f;
   for (int s = 0; s < g.max_steps; ++s) {
-    if (pz >= g.z_top) return src_top;
+    if (pz >= g.z_top) return kDdaSky;
     const float u = fminf(fmaxf(px / dx, 0.f), ux);
     const float v = fminf(fmaxf(py / dx, 0.f), uy);
     const float w = fminf(fmaxf(pz / dx, 0.f), uz);
@@ -283,19 +283,18 @@ __device__ float dda_ray(const DdaGrid& g, float ox, float oy, float oz, float d
     const float p11 = node(g, i0, j0 + 1, k0 + 1) * gu + node(g, i0 + 1, j0 + 1, k0 + 1) * fu;
     const float pv = (p00 * gv + p10 * fv) * gw + (p01 * gv + p11 * fv) * fw;
     if (pv > 0.f) {
-      if (!remit) return 0.f;
       float qx = px, qy = py, qz = pz;
       for (int e = 0; e < 6; ++e) {
         const int ix = round_cell(qx, dx, g.nx), iy = round_cell(qy, dx, g.ny),
                   iz = round_cell(qz, dx, g.nz);
-        if (node(g, ix, iy, iz) > 0.f) return remit[((long long)ix * g.ny + iy) * g.nz + iz];
+        if (node(g, ix, iy, iz) > 0.f) return (ix * g.ny + iy) * g.nz + iz;
         qx = qx + sx * 0.5f;
         qy = qy + sy * 0.5f;
         qz = qz + sz * 0.5f;
       }
       const int ix = round_cell(px, dx, g.nx), iy = round_cell(py, dx, g.ny),
                 iz = round_cell(pz, dx, g.nz);
-      return remit[((long long)ix * g.ny + iy) * g.nz + iz];
+      return (ix * g.ny + iy) * g.nz + iz;
     }
     px = px + sx;
     py = py + sy;
@@ -305,46 +304,121 @@ __device__ float dda_ray(const DdaGrid& g, float ox, float oy, float oz, float d
       if (py >= g.Ly) py = py - g.Ly;
     }
   }
-  return 0.f;
+  return kDdaNone;
 }
 
-// One wavefront per face, its lanes over the directions: sum_k acc_k c_k / max(sum_k acc_k,
-// 1e-12), acc_k = max(n . d_k, 0), directions with acc <= 1e-6 not marched (dda.py:36-95).
-// The sums are float64 (the reference's are float32, so the two differ in the last bits).
-__global__ void __launch_bounds__(kBS) k_dda_gather(DdaGrid g, const float* __restrict__ cen,
-                                                    const float* __restrict__ nrm, int F,
-                                                    const float* __restrict__ dirs, int nd,
-                                                    const float* __restrict__ remit,
-                                                    float src_top, float* __restrict__ out) {
+// A face's rays end in the same cells whatever its surface re-emits, so the march runs once per
+// surface and keeps each ray's end (a cell, or kDdaSky / kDdaNone); the passes then only read the
+// field there. One wavefront per face, its lanes over the directions, acc_k = max(n . d_k, 0),
+// directions with acc <= 1e-6 not marched (dda.py:36-95); `direct` is the sky's share
+// sum_sky acc_k / max(sum_k acc_k, 1e-12). The sums over directions are float64 (the reference's
+// are float32, so the two differ in the last bits). 0.36 ms for 17k faces x 128 directions
+// (56x56x96), bound by the chain of dependent steps of a ray; marching again in each of the 25
+// gathers of a call was 33 of the 36 ms of a four-round flux.
+__device__ __forceinline__ float dda_acc(const float* __restrict__ dirs, int k, float nx, float ny,
+                                         float nz) {
+#pragma clang fp contract(off)
+  return fmaxf(nx * dirs[3 * k] + ny * dirs[3 * k + 1] + nz * dirs[3 * k + 2], 0.f);
+}
+
+__device__ __forceinline__ double wave_sum(double v) {
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d, 64);
+  return v;
+}
+
+__global__ void __launch_bounds__(kBS) k_dda_march(DdaGrid g, const float* __restrict__ cen,
+                                                   const float* __restrict__ nrm, int F,
+                                                   const float* __restrict__ dirs, int nd,
+                                                   int* __restrict__ stops,
+                                                   float* __restrict__ direct) {
 #pragma clang fp contract(off)
   const int f = blockIdx.x * (kBS / 64) + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
+  if (f >= F) return;  // whole waves leave together
   double num = 0.0, den = 0.0;
-  if (f < F) {
-    const float ox = cen[3 * f], oy = cen[3 * f + 1], oz = cen[3 * f + 2];
-    const float nx = nrm[3 * f], ny = nrm[3 * f + 1], nz = nrm[3 * f + 2];
-    for (int k = lane; k < nd; k += 64) {
-      const float dxv = dirs[3 * k], dyv = dirs[3 * k + 1], dzv = dirs[3 * k + 2];
-      const float acc = fmaxf(nx * dxv + ny * dyv + nz * dzv, 0.f);
-      den += (double)acc;
-      if (acc > 1.0e-6f) num += (double)acc * (double)dda_ray(g, ox, oy, oz, dxv, dyv, dzv, remit, src_top);
-    }
+  const float ox = cen[3 * f], oy = cen[3 * f + 1], oz = cen[3 * f + 2];
+  const float nx = nrm[3 * f], ny = nrm[3 * f + 1], nz = nrm[3 * f + 2];
+  for (int k = lane; k < nd; k += 64) {
+    const float acc = dda_acc(dirs, k, nx, ny, nz);
+    den += (double)acc;
+    int stop = kDdaNone;
+    if (acc > 1.0e-6f) stop = dda_ray(g, ox, oy, oz, dirs[3 * k], dirs[3 * k + 1], dirs[3 * k + 2]);
+    stops[(long long)f * nd + k] = stop;
+    if (stop == kDdaSky) num += (double)acc;
   }
-#pragma unroll
-  for (int d = 32; d >= 1; d >>= 1) {
-    num += __shfl_xor(num, d, 64);
-    den += __shfl_xor(den, d, 64);
-  }
-  if (f < F && lane == 0) out[f] = (float)(num / fmax(den, 1.0e-12));
+  num = wave_sum(num);
+  den = wave_sum(den);
+  if (lane == 0) direct[f] = (float)(num / fmax(den, 1.0e-12));
 }
 
-__global__ void k_dda_zero(double* __restrict__ a, double* __restrict__ b, uint8_t* __restrict__ c,
-                           long long n) {
+// A face's re-emission into its cell (dda.py:187): A (1 - s) max(vf, 0).
+__device__ __forceinline__ void dda_emit(const float* __restrict__ areas,
+                                         const float* __restrict__ bare, double beta, double vf,
+                                         int f, double* __restrict__ Rc) {
+  const double s = fmin(fmax((double)bare[f] * beta, 0.0), 1.0);
+  const double alpha = fmin(fmax(1.0 - s, 0.0), 1.0);
+  atomicAdd(Rc, fmax((double)areas[f], 1.0e-9) * alpha * fmax(vf, 0.0));
+}
+
+// One re-emission pass of NS species: every face gathers the field at its rays' ends, its new
+// iterate is direct + the gathered value (rounded to float32 as the reference stores it), and
+// that iterate's own re-emission is added to the next pass's sums. The species share the march,
+// so one 8-byte field read serves both. Bound by the scattered field reads, which stay in the L2
+// (2.4 MB at 56x56x96); with the march, update and scatter as launches of their own a pass of
+// one species took 390 us there.
+template <int NS>
+struct DdaPass {
+  double beta[NS];
+  double* vf[NS];  // this pass's iterate
+};
+
+template <int NS>
+__global__ void __launch_bounds__(kBS) k_dda_pass(const float* __restrict__ nrm, int F,
+                                                  const float* __restrict__ dirs, int nd,
+                                                  const int* __restrict__ stops,
+                                                  const float* __restrict__ direct,
+                                                  const float* __restrict__ field,
+                                                  const int* __restrict__ cell,
+                                                  const float* __restrict__ areas,
+                                                  const float* __restrict__ bare, DdaPass<NS> P,
+                                                  double* __restrict__ Rnext) {
+#pragma clang fp contract(off)
+  const int f = blockIdx.x * (kBS / 64) + (threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  if (f >= F) return;  // whole waves leave together
+  const float nx = nrm[3 * f], ny = nrm[3 * f + 1], nz = nrm[3 * f + 2];
+  double num[NS] = {}, den = 0.0;
+  for (int k = lane; k < nd; k += 64) {
+    const int c = stops[(long long)f * nd + k];
+    const float acc = dda_acc(dirs, k, nx, ny, nz);
+    den += (double)acc;
+    if (c >= 0) {
+#pragma unroll
+      for (int s = 0; s < NS; ++s) num[s] += (double)acc * (double)field[(long long)NS * c + s];
+    }
+  }
+  den = wave_sum(den);
+#pragma unroll
+  for (int s = 0; s < NS; ++s) num[s] = wave_sum(num[s]);
+  if (lane != 0) return;
+#pragma unroll
+  for (int s = 0; s < NS; ++s) {
+    const float got = (float)(num[s] / fmax(den, 1.0e-12));
+    const double v = (double)direct[f] + (double)got;
+    P.vf[s][f] = v;
+    if (Rnext) dda_emit(areas, bare, P.beta[s], v, f, Rnext + (long long)NS * cell[f] + s);
+  }
+}
+
+// clears the cells' areas, seeded flags and the first pass's sums
+__global__ void k_dda_zero(double* __restrict__ carea, double* __restrict__ R, int ns,
+                           uint8_t* __restrict__ seeded, long long n) {
   for (long long i = (long long)blockIdx.x * kBS + threadIdx.x; i < n;
        i += (long long)gridDim.x * kBS) {
-    if (a) a[i] = 0.0;
-    if (b) b[i] = 0.0;
-    if (c) c[i] = 0;
+    carea[i] = 0.0;
+    seeded[i] = 0;
+    for (int s = 0; s < ns; ++s) R[ns * i + s] = 0.0;
   }
 }
 
@@ -370,35 +444,39 @@ __global__ void k_dda_cells(const float* __restrict__ cen, const float* __restri
   seeded[c] = 1;
 }
 
-// Per face: its re-emitted intensity A (1 - s) max(vf, 0) into its cell (dda.py:187).
-__global__ void k_dda_scatter(const int* __restrict__ cell, const float* __restrict__ areas,
-                              const float* __restrict__ bare, double beta,
-                              const double* __restrict__ vf, int F, double* __restrict__ R) {
+// The first iterate vf = direct and its re-emission.
+template <int NS>
+__global__ void k_dda_start(const float* __restrict__ direct, const int* __restrict__ cell,
+                            const float* __restrict__ areas, const float* __restrict__ bare, int F,
+                            DdaPass<NS> P, double* __restrict__ R) {
   const int f = blockIdx.x * kBS + threadIdx.x;
   if (f >= F) return;
-  const double s = fmin(fmax((double)bare[f] * beta, 0.0), 1.0);
-  const double alpha = fmin(fmax(1.0 - s, 0.0), 1.0);
-  atomicAdd(R + cell[f], fmax((double)areas[f], 1.0e-9) * alpha * fmax(vf[f], 0.0));
+#pragma unroll
+  for (int s = 0; s < NS; ++s) {
+    const double v = (double)direct[f];
+    P.vf[s][f] = v;
+    dda_emit(areas, bare, P.beta[s], v, f, R + (long long)NS * cell[f] + s);
+  }
 }
 
-// Per cell: R = sum / max(area, 1e-12) (the area-weighted mean of the cell's faces).
-__global__ void k_dda_mean(double* __restrict__ R, const double* __restrict__ carea, long long n) {
-  for (long long i = (long long)blockIdx.x * kBS + threadIdx.x; i < n;
-       i += (long long)gridDim.x * kBS)
-    R[i] = R[i] / fmax(carea[i], 1.0e-12);
-}
-
-// Per cell: the field the march reads (float32). A solid unseeded cell with seeded neighbours
-// (the six, wrapping around the grid) takes their mean, summed in the order -x, +x, -y, +y, -z,
-// +z of the reference's rolls (dda.py:196-207); every other cell keeps R.
+// Per cell: the field a pass reads (float32), from the sums R: the area-weighted mean
+// R / max(area, 1e-12) of the cell's faces; a solid unseeded cell with seeded neighbours (the six,
+// wrapping around the grid) takes their mean, summed in the order -x, +x, -y, +y, -z, +z of the
+// reference's rolls (dda.py:196-207). Rz, the sums the following pass adds into, are cleared.
+template <int NS>
 __global__ void k_dda_fill(const float* __restrict__ phi, const double* __restrict__ R,
-                           const uint8_t* __restrict__ seeded, int nx, int ny, int nz,
-                           float* __restrict__ out) {
+                           const double* __restrict__ carea, const uint8_t* __restrict__ seeded,
+                           int nx, int ny, int nz, float* __restrict__ out,
+                           double* __restrict__ Rz) {
   const long long n = (long long)nx * ny * nz;
   for (long long c = (long long)blockIdx.x * kBS + threadIdx.x; c < n;
        c += (long long)gridDim.x * kBS) {
-    double v = R[c];
-    if (phi[c] > 0.f && !seeded[c]) {
+    double v[NS] = {};
+    if (seeded[c]) {  // an unseeded cell's sums are 0
+      const double a = fmax(carea[c], 1.0e-12);
+#pragma unroll
+      for (int s = 0; s < NS; ++s) v[s] = R[NS * c + s] / a;
+    } else if (phi[c] > 0.f) {
       const int k = (int)(c % nz), j = (int)((c / nz) % ny), i = (int)(c / ((long long)nz * ny));
       const int im = i == 0 ? nx - 1 : i - 1, ip = i == nx - 1 ? 0 : i + 1;
       const int jm = j == 0 ? ny - 1 : j - 1, jp = j == ny - 1 ? 0 : j + 1;
@@ -406,25 +484,25 @@ __global__ void k_dda_fill(const float* __restrict__ phi, const double* __restri
       const long long nb[6] = {((long long)im * ny + j) * nz + k, ((long long)ip * ny + j) * nz + k,
                                ((long long)i * ny + jm) * nz + k, ((long long)i * ny + jp) * nz + k,
                                ((long long)i * ny + j) * nz + km, ((long long)i * ny + j) * nz + kp};
-      double num = 0.0;
       int cnt = 0;
       for (int q = 0; q < 6; ++q) {
-        if (seeded[nb[q]]) {
-          num += R[nb[q]];
-          ++cnt;
-        }
+        if (!seeded[nb[q]]) continue;
+        const double a = fmax(carea[nb[q]], 1.0e-12);
+#pragma unroll
+        for (int s = 0; s < NS; ++s) v[s] += R[NS * nb[q] + s] / a;
+        ++cnt;
       }
-      if (cnt > 0) v = num / (double)cnt;
+      if (cnt > 0) {
+#pragma unroll
+        for (int s = 0; s < NS; ++s) v[s] = v[s] / (double)cnt;
+      }
     }
-    out[c] = (float)v;
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      out[NS * c + s] = (float)v[s];
+      if (Rz) Rz[NS * c + s] = 0.0;
+    }
   }
-}
-
-// vf = direct (+ the gathered re-emission g, when given)
-__global__ void k_dda_update(const float* __restrict__ direct, const float* __restrict__ g,
-                             int F, double* __restrict__ vf) {
-  const int f = blockIdx.x * kBS + threadIdx.x;
-  if (f < F) vf[f] = g ? (double)direct[f] + (double)g[f] : (double)direct[f];
 }
 
 // Aitken on the last three iterates (dda.py:212-218) when there are three, then clip to [0, 8].
@@ -445,6 +523,112 @@ __global__ void k_dda_final(const double* __restrict__ vf, const double* __restr
 unsigned grid_of(long long n) {
   const long long b = (n + kBS - 1) / kBS;
   return (unsigned)(b < 65536 ? (b > 0 ? b : 1) : 65536);
+}
+
+// The plan of a surface's rays, in 4-byte words: the 2 n_dir directions (x, y, z), the direct
+// values of the F faces, every ray's end.
+struct DdaPlan {
+  const float* dirs;
+  const float* direct;
+  const int* stops;
+  DdaPlan(const int* w, int nd, int F)
+      : dirs((const float*)w), direct((const float*)w + 3 * (size_t)nd),
+        stops(w + 3 * (size_t)nd + (size_t)F) {}
+};
+
+size_t dda_plan_words(int nd, int F) { return 3 * (size_t)nd + (size_t)F * (1 + (size_t)nd); }
+
+DdaGrid dda_grid(const float* phi, int nx, int ny, int nz, const petch_dda_params* p) {
+  const double dx = p->dx, z_top = (double)(nz - 1) * dx - 0.5 * dx;
+  DdaGrid g;
+  g.phi = phi; g.nx = nx; g.ny = ny; g.nz = nz;
+  g.dx = (float)dx;
+  g.z_top = (float)z_top;
+  g.Ly = (float)ny * (float)dx;
+  g.max_steps = ((int)(z_top / dx) + 4) * (p->periodic_y ? 3 : 1);
+  g.periodic_y = p->periodic_y ? 1 : 0;
+  return g;
+}
+
+int dda_march(petch_ctx* ctx, const float* phi, int nx, int ny, int nz, const float* centroids,
+              const float* gas_normals, int F, const petch_dda_params* p, int* plan) {
+  const int nd = 2 * p->n_dir;
+  // the direction set (fib_sphere(2 n_dir), dda.py:124-135): float64, handed over as float32
+  std::vector<float> dirs((size_t)nd * 3);
+  const double gold = M_PI * (1.0 + sqrt(5.0));
+  for (int i = 0; i < nd; ++i) {
+    const double t = (double)i + 0.5;
+    const double z = 1.0 - 2.0 * t / (double)nd;
+    const double r = sqrt(fmax(1.0 - z * z, 0.0));
+    const double th = gold * t;
+    dirs[3 * i] = (float)(r * cos(th));
+    dirs[3 * i + 1] = (float)(r * sin(th));
+    dirs[3 * i + 2] = (float)z;
+  }
+  const size_t bytes = dirs.size() * sizeof(float);
+  const void* dd = petch_upload_table(ctx, dirs.data(), bytes);
+  if (!dd) return PETCH_E_HIP;
+  PETCH_HIP(ctx, hipMemcpyAsync(plan, dd, bytes, hipMemcpyDeviceToDevice, ctx->stream));
+  const DdaPlan P(plan, nd, F);
+  hipLaunchKernelGGL(k_dda_march, dim3(petch_blocks(F, kBS / 64)), dim3(kBS), 0, ctx->stream,
+                     dda_grid(phi, nx, ny, nz, p), centroids, gas_normals, F, P.dirs, nd,
+                     (int*)P.stops, (float*)P.direct);
+  PETCH_LAUNCH_CHECK(ctx);
+  return PETCH_OK;
+}
+
+// The re-emission passes of NS species over a plan's rays.
+template <int NS>
+int dda_reemit(petch_ctx* ctx, const float* phi, int nx, int ny, int nz, const float* centroids,
+               const float* gas_normals, const float* areas, const float* bare, int F,
+               const petch_dda_params* p, const DdaPlan& L, float* const out[2]) {
+  const long long N = (long long)nx * ny * nz;
+  const int nd = 2 * p->n_dir;
+  // cells: area, two sets of sums, the field, seeded flags; faces: three iterates, cell
+  char* cw = (char*)petch_scratch(ctx, SCR_RAD_A, (size_t)N * (8 + 2 * 8 * NS + 4 * NS + 1) + 64);
+  char* fw = (char*)petch_scratch(ctx, SCR_RAD_B, (size_t)F * (3 * 8 * NS + 4) + 64);
+  if (!cw || !fw) return PETCH_E_HIP;
+  double* carea = (double*)cw;
+  double* R[2] = {carea + N, carea + N + (size_t)NS * N};
+  float* field = (float*)(R[1] + (size_t)NS * N);
+  uint8_t* seeded = (uint8_t*)(field + (size_t)NS * N);
+  double* it = (double*)fw;
+  int* cell = (int*)(it + (size_t)3 * NS * F);
+  const unsigned gN = grid_of(N), gF = petch_blocks(F, kBS), gW = petch_blocks(F, kBS / 64);
+  hipLaunchKernelGGL(k_dda_zero, dim3(gN), dim3(kBS), 0, ctx->stream, carea, R[0], NS, seeded, N);
+  PETCH_LAUNCH_CHECK(ctx);
+  hipLaunchKernelGGL(k_dda_cells, dim3(gF), dim3(kBS), 0, ctx->stream, centroids, gas_normals,
+                     areas, F, nx, ny, nz, p->dx, cell, carea, seeded);
+  PETCH_LAUNCH_CHECK(ctx);
+  // pass r's iterate of species s is it[(r % 3) NS F + s F ...]: the last three are kept
+  DdaPass<NS> P;
+  auto iterate = [&](int r, int s) { return it + ((size_t)(r % 3) * NS + s) * F; };
+  P.beta[0] = p->beta_a;
+  if (NS > 1) P.beta[NS - 1] = p->beta_b;
+  for (int s = 0; s < NS; ++s) P.vf[s] = iterate(0, s);
+  hipLaunchKernelGGL(k_dda_start<NS>, dim3(gF), dim3(kBS), 0, ctx->stream, L.direct, cell, areas,
+                     bare, F, P, R[0]);
+  PETCH_LAUNCH_CHECK(ctx);
+  const int n_re = p->n_reemit > 1 ? p->n_reemit : 1;
+  for (int r = 1; r <= n_re; ++r) {
+    const bool more = r < n_re;
+    double *cur = R[(r - 1) & 1], *nxt = more ? R[r & 1] : (double*)nullptr;
+    hipLaunchKernelGGL(k_dda_fill<NS>, dim3(gN), dim3(kBS), 0, ctx->stream, phi, cur, carea,
+                       seeded, nx, ny, nz, field, nxt);
+    PETCH_LAUNCH_CHECK(ctx);
+    for (int s = 0; s < NS; ++s) P.vf[s] = iterate(r, s);
+    hipLaunchKernelGGL(k_dda_pass<NS>, dim3(gW), dim3(kBS), 0, ctx->stream, gas_normals, F, L.dirs,
+                       nd, L.stops, L.direct, field, cell, areas, bare, P, nxt);
+    PETCH_LAUNCH_CHECK(ctx);
+  }
+  for (int s = 0; s < NS; ++s) {
+    hipLaunchKernelGGL(k_dda_final, dim3(gF), dim3(kBS), 0, ctx->stream, iterate(n_re, s),
+                       iterate(n_re - 1, s),
+                       n_re >= 2 ? (const double*)iterate(n_re - 2, s) : (const double*)nullptr, F,
+                       out[s]);
+    PETCH_LAUNCH_CHECK(ctx);
+  }
+  return PETCH_OK;
 }
 
 }  // namespace
@@ -496,100 +680,49 @@ extern "C" int petch_knudsen_face_flux(petch_ctx* ctx, const float* phi, int nx,
   return PETCH_OK;
 }
 
+extern "C" int petch_dda_march(petch_ctx* ctx, const float* phi, int nx, int ny, int nz,
+                               const float* centroids, const float* gas_normals, int F,
+                               const petch_dda_params* p, int* plan) {
+  PETCH_ARG(ctx, ctx && phi && p, "dda_march: null pointer");
+  PETCH_ARG(ctx, nx > 1 && ny > 1 && nz > 1 && F >= 0, "dda_march: bad shape");
+  PETCH_ARG(ctx, (long long)nx * ny * nz <= 0x7fffffffLL, "dda_march: more than 2^31-1 nodes");
+  PETCH_ARG(ctx, p->dx > 0.0 && p->n_dir > 0, "dda_march: dx <= 0 or n_dir <= 0");
+  if (F == 0) return PETCH_OK;
+  PETCH_ARG(ctx, centroids && gas_normals && plan, "dda_march: null array");
+  return dda_march(ctx, phi, nx, ny, nz, centroids, gas_normals, F, p, plan);
+}
+
+extern "C" int petch_dda_reemit(petch_ctx* ctx, const float* phi, int nx, int ny, int nz,
+                                const float* centroids, const float* gas_normals,
+                                const float* areas, const float* bare, int F,
+                                const petch_dda_params* p, const int* plan, float* m_a,
+                                float* m_b) {
+  PETCH_ARG(ctx, ctx && phi && p && m_a, "dda_reemit: null pointer");
+  PETCH_ARG(ctx, nx > 1 && ny > 1 && nz > 1 && F >= 0, "dda_reemit: bad shape");
+  PETCH_ARG(ctx, (long long)nx * ny * nz <= 0x7fffffffLL, "dda_reemit: more than 2^31-1 nodes");
+  PETCH_ARG(ctx, p->dx > 0.0 && p->n_dir > 0, "dda_reemit: dx <= 0 or n_dir <= 0");
+  if (F == 0) return PETCH_OK;
+  PETCH_ARG(ctx, centroids && gas_normals && areas && bare && plan, "dda_reemit: null array");
+  const DdaPlan L(plan, 2 * p->n_dir, F);
+  float* const out[2] = {m_a, m_b};
+  if (m_b)
+    return dda_reemit<2>(ctx, phi, nx, ny, nz, centroids, gas_normals, areas, bare, F, p, L, out);
+  return dda_reemit<1>(ctx, phi, nx, ny, nz, centroids, gas_normals, areas, bare, F, p, L, out);
+}
+
 extern "C" int petch_dda_neutral_flux(petch_ctx* ctx, const float* phi, int nx, int ny, int nz,
                                       const float* centroids, const float* gas_normals,
                                       const float* areas, const float* bare, int F,
                                       const petch_dda_params* p, float* m_a, float* m_b) {
   PETCH_ARG(ctx, ctx && phi && p && m_a, "dda_neutral_flux: null pointer");
-  PETCH_ARG(ctx, nx > 1 && ny > 1 && nz > 1 && F >= 0, "dda_neutral_flux: bad shape");
-  PETCH_ARG(ctx, p->dx > 0.0 && p->n_dir > 0, "dda_neutral_flux: dx <= 0 or n_dir <= 0");
-  if (F == 0) return PETCH_OK;
-  PETCH_ARG(ctx, centroids && gas_normals && areas && bare, "dda_neutral_flux: null face array");
-  const long long N = (long long)nx * ny * nz;
-  const int nd = 2 * p->n_dir;
-  // the direction set (fib_sphere(2 n_dir), dda.py:124-135): float64, handed over as float32
-  std::vector<float> dirs((size_t)nd * 3);
-  const double gold = M_PI * (1.0 + sqrt(5.0));
-  for (int i = 0; i < nd; ++i) {
-    const double t = (double)i + 0.5;
-    const double z = 1.0 - 2.0 * t / (double)nd;
-    const double r = sqrt(fmax(1.0 - z * z, 0.0));
-    const double th = gold * t;
-    dirs[3 * i] = (float)(r * cos(th));
-    dirs[3 * i + 1] = (float)(r * sin(th));
-    dirs[3 * i + 2] = (float)z;
+  PETCH_ARG(ctx, F >= 0 && p->n_dir > 0, "dda_neutral_flux: bad shape or n_dir <= 0");
+  int* plan = nullptr;
+  if (F > 0) {
+    plan = (int*)petch_scratch(ctx, SCR_RAD_C, dda_plan_words(2 * p->n_dir, F) * sizeof(int));
+    if (!plan) return PETCH_E_HIP;
   }
-  // cells: area (double), re-emission sum (double), field (float), seeded (u8);
-  // faces: cell, direct and gathered values (float), three iterates per species (double)
-  char* cw = (char*)petch_scratch(ctx, SCR_RAD_A, (size_t)N * (8 + 8 + 4 + 1) + 64);
-  char* fw = (char*)petch_scratch(ctx, SCR_RAD_B, (size_t)F * (4 + 4 + 4 + 6 * 8) + 64);
-  if (!cw || !fw) return PETCH_E_HIP;
-  double* carea = (double*)cw;
-  double* R = carea + N;
-  float* field = (float*)(R + N);
-  uint8_t* seeded = (uint8_t*)(field + N);
-  int* cell = (int*)fw;
-  float* direct = (float*)(cell + F);
-  float* gath = direct + F;
-  double* it = (double*)(((uintptr_t)(gath + F) + 7) & ~(uintptr_t)7);
-  const float* dd = (const float*)petch_upload_table(ctx, dirs.data(), dirs.size() * sizeof(float));
-  if (!dd) return PETCH_E_HIP;
-  const double dx = p->dx;
-  const double z_top = (double)(nz - 1) * dx - 0.5 * dx;
-  DdaGrid g;
-  g.phi = phi; g.nx = nx; g.ny = ny; g.nz = nz;
-  g.dx = (float)dx;
-  g.z_top = (float)z_top;
-  g.Ly = (float)ny * (float)dx;
-  g.max_steps = ((int)(z_top / dx) + 4) * (p->periodic_y ? 3 : 1);
-  g.periodic_y = p->periodic_y ? 1 : 0;
-  const unsigned gN = grid_of(N), gF = petch_blocks(F, kBS), gW = petch_blocks(F, kBS / 64);
-  hipLaunchKernelGGL(k_dda_zero, dim3(gN), dim3(kBS), 0, ctx->stream, carea, (double*)nullptr,
-                     seeded, N);
-  PETCH_LAUNCH_CHECK(ctx);
-  hipLaunchKernelGGL(k_dda_cells, dim3(gF), dim3(kBS), 0, ctx->stream, centroids, gas_normals,
-                     areas, F, nx, ny, nz, dx, cell, carea, seeded);
-  PETCH_LAUNCH_CHECK(ctx);
-  hipLaunchKernelGGL(k_dda_gather, dim3(gW), dim3(kBS), 0, ctx->stream, g, centroids, gas_normals,
-                     F, dd, nd, (const float*)nullptr, 1.0f, direct);
-  PETCH_LAUNCH_CHECK(ctx);
-  const int n_re = p->n_reemit > 1 ? p->n_reemit : 1;
-  for (int s = 0; s < 2; ++s) {
-    float* out = s ? m_b : m_a;
-    if (!out) continue;
-    const double beta = s ? p->beta_b : p->beta_a;
-    double* v[3] = {it + (size_t)3 * s * F, it + (size_t)(3 * s + 1) * F, it + (size_t)(3 * s + 2) * F};
-    // v[0]: current iterate; v[1], v[2]: the two before it
-    hipLaunchKernelGGL(k_dda_update, dim3(gF), dim3(kBS), 0, ctx->stream, direct,
-                       (const float*)nullptr, F, v[0]);
-    PETCH_LAUNCH_CHECK(ctx);
-    int have = 1;
-    for (int r = 0; r < n_re; ++r) {
-      hipLaunchKernelGGL(k_dda_zero, dim3(gN), dim3(kBS), 0, ctx->stream, R, (double*)nullptr,
-                         (uint8_t*)nullptr, N);
-      PETCH_LAUNCH_CHECK(ctx);
-      hipLaunchKernelGGL(k_dda_scatter, dim3(gF), dim3(kBS), 0, ctx->stream, cell, areas, bare,
-                         beta, v[0], F, R);
-      PETCH_LAUNCH_CHECK(ctx);
-      hipLaunchKernelGGL(k_dda_mean, dim3(gN), dim3(kBS), 0, ctx->stream, R, carea, N);
-      PETCH_LAUNCH_CHECK(ctx);
-      hipLaunchKernelGGL(k_dda_fill, dim3(gN), dim3(kBS), 0, ctx->stream, phi, R, seeded, nx, ny,
-                         nz, field);
-      PETCH_LAUNCH_CHECK(ctx);
-      hipLaunchKernelGGL(k_dda_gather, dim3(gW), dim3(kBS), 0, ctx->stream, g, centroids,
-                         gas_normals, F, dd, nd, field, 0.0f, gath);
-      PETCH_LAUNCH_CHECK(ctx);
-      double* t = v[2];
-      v[2] = v[1];
-      v[1] = v[0];
-      v[0] = t;
-      hipLaunchKernelGGL(k_dda_update, dim3(gF), dim3(kBS), 0, ctx->stream, direct, gath, F, v[0]);
-      PETCH_LAUNCH_CHECK(ctx);
-      ++have;
-    }
-    hipLaunchKernelGGL(k_dda_final, dim3(gF), dim3(kBS), 0, ctx->stream, v[0], v[1],
-                       have >= 3 ? v[2] : (double*)nullptr, F, out);
-    PETCH_LAUNCH_CHECK(ctx);
-  }
-  return PETCH_OK;
+  const int rc = petch_dda_march(ctx, phi, nx, ny, nz, centroids, gas_normals, F, p, plan);
+  if (rc) return rc;
+  return petch_dda_reemit(ctx, phi, nx, ny, nz, centroids, gas_normals, areas, bare, F, p, plan,
+                          m_a, m_b);
 }

@@ -238,6 +238,9 @@ SIGNATURES = {
                                 POINTER(KnudsenParams), P, P],
     "petch_dda_neutral_flux": [P, P, c_int, c_int, c_int, P, P, P, P, c_int,
                                POINTER(DdaParams), P, P],
+    "petch_dda_march": [P, P, c_int, c_int, c_int, P, P, c_int, POINTER(DdaParams), P],
+    "petch_dda_reemit": [P, P, c_int, c_int, c_int, P, P, P, P, c_int, POINTER(DdaParams), P, P,
+                         P],
     "petch_belen_coverage_adjoint": [P, P, P, P, P, P, P, POINTER(ChemParams), c_int, P, P, P,
                                      P, P, P],
     "petch_surface_rate": [P, P, P, P, P, P, P, P, P, P, POINTER(MaskGeom),

@@ -344,10 +344,12 @@ def dda_flux(mesh, phi, geo, par, n_ion, seed, flags, n_fp=4):
     betaE, betaO = par.get('betaE', 0.7), par.get('betaO', 1.0)
     n_dir, n_re = int(par.get('dda_n_dir', 64)), int(par.get('dda_n_reemit', 12))
     py = int(par.get('periodic_y', 0))
+    # the surface stands still over the coverage rounds, and with it every ray's end
+    plan = ops.dda_march(phi, dx, mesh.centroids, gn, n_dir, py)
 
     def neutrals(bare):
         return ops.dda_neutral_flux(phi, dx, mesh.centroids, gn, mesh.areas, bare,
-                                    (betaE, betaO), n_dir, n_re, py)
+                                    (betaE, betaO), n_dir, n_re, py, plan)
     return _deterministic_neutrals(mesh, phi, geo, par, n_ion, seed, flags, n_fp, neutrals)
 
 

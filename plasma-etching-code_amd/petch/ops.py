@@ -992,9 +992,10 @@ def knudsen_face_flux(phi, dx, sub_top, trench, centroids, gas_normals, areas, b
 
 
 def dda_neutral_flux(phi, dx, centroids, gas_normals, areas, bare, betas, n_dir=64, n_reemit=12,
-                     periodic_y=0):
+                     periodic_y=0, plan=None):
     """dda_neutral_flux (dda.py:138-220) for the sticking coefficients bare * beta of the one or
-    two betas (petch_dda_neutral_flux): one (F,) float32 multiplier per beta."""
+    two betas (petch_dda_neutral_flux): one (F,) float32 multiplier per beta. plan: dda_march's
+    result for the same surface, when several coverages are solved on it."""
     from ._abi import DdaParams
     nx, ny, nz = _shape3(phi)
     F = int(centroids.shape[0])
@@ -1003,11 +1004,31 @@ def dda_neutral_flux(phi, dx, centroids, gas_normals, areas, bare, betas, n_dir=
         raise ValueError("dda_neutral_flux: one or two betas")
     outs = [torch.empty((F,), dtype=f32, device=phi.device) for _ in betas]
     p = DdaParams(float(dx), int(n_dir), int(n_reemit), int(bool(periodic_y)), float(betas[0]),
+def dda_march(phi, dx, centroids, gas_normals, n_dir=64, periodic_y=0):
+    """The rays of dda_neutral_flux marched once (petch_dda_march), as a plan for any number of
+    its calls on the same phi, dx, faces, n_dir and periodic_y."""
+    from ._abi import DdaParams
+    nx, ny, nz = _shape3(phi)
+    F, nd = int(centroids.shape[0]), 2 * int(n_dir)
+    plan = torch.empty((3 * nd + F * (1 + nd),), dtype=i32, device=phi.device)
+    p = DdaParams(float(dx), int(n_dir), 1, int(bool(periodic_y)), 0.0, 0.0)
+    if F:
+        _ctx(phi).call("petch_dda_march", ptr(phi, f32, "phi"), nx, ny, nz,
+                       ptr(centroids, f32, "centroids"), ptr(gas_normals, f32, "gas_normals"), F,
+                       ctypes_ref(p), ptr(plan))
+    return plan
+
+
                   float(betas[-1]))
     if F:
-        _ctx(phi).call("petch_dda_neutral_flux", ptr(phi, f32, "phi"), nx, ny, nz,
-                       ptr(centroids, f32, "centroids"), ptr(gas_normals, f32, "gas_normals"),
-                       ptr(areas, f32, "areas"), ptr(bare, f32, "bare"), F, ctypes_ref(p),
+        args = [ptr(phi, f32, "phi"), nx, ny, nz, ptr(centroids, f32, "centroids"),
+                ptr(gas_normals, f32, "gas_normals"), ptr(areas, f32, "areas"),
+                ptr(bare, f32, "bare"), F, ctypes_ref(p)]
+        if plan is not None:
+            if plan.numel() != 6 * int(n_dir) + F * (1 + 2 * int(n_dir)):
+                raise ValueError("dda_neutral_flux: the plan is of another surface or n_dir")
+            args.append(ptr(plan, i32, "plan"))
+        _ctx(phi).call("petch_dda_neutral_flux" if plan is None else "petch_dda_reemit", *args,
                        ptr(outs[0]), ptr(outs[1]) if len(outs) > 1 else None)
     return outs
 

@@ -133,3 +133,30 @@ def test_etch_loop_runs_deterministic_transports(nt):
                               flags=fl)
     for m in (m_F, m_O):
         assert m.shape == (len(faces),) and (m >= 0).all() and (m <= 8).all()
+
+
+@pytest.mark.parametrize("n_dir,n_re", [(1, 1), (16, 2), (33, 3), (64, 4)])
+def test_dda_plan_and_species_agree(n_dir, n_re):
+    """The march is shared by the passes, the two species and the calls on one surface: a plan's
+    call, the self-contained call and the single-species calls give the same values (direction
+    counts below, beyond and off the 64 lanes of a face's wavefront). The cells' float64 atomic
+    sums may add in another order: rtol 1e-6 covers a float32 rounding step per iterate, times
+    r / (1 - r) of the Aitken step for the three last iterates (atol, values of order 1)."""
+    import torch
+    from petch import ops
+    dx, nx, ny, nz = 0.25, 21, 19, 30
+    phi, _ = _carved("hole", nx, ny, nz, dx, 5.5, 3.0, 1.1)
+    tphi, cen, area, gn = _surface(phi, dx)
+    F = int(cen.shape[0])
+    bare = torch.from_numpy(np.random.default_rng(5).uniform(0.05, 1.0, F).astype(np.float32)).to(_dev())
+    args = (tphi, dx, cen, gn, area, bare)
+    betas = (0.4, 1.0)
+    own = ops.dda_neutral_flux(*args, betas, n_dir, n_re)
+    plan = ops.dda_march(tphi, dx, cen, gn, n_dir)
+    atol = 1e-6 if n_re < 2 else 1e-4
+    for other in (ops.dda_neutral_flux(*args, betas, n_dir, n_re, plan=plan),
+                  [ops.dda_neutral_flux(*args, (b,), n_dir, n_re)[0] for b in betas]):
+        for a, b in zip(own, other):
+            np.testing.assert_allclose(a.cpu().numpy(), b.cpu().numpy(), rtol=1e-6, atol=atol)
+    with pytest.raises(ValueError, match="plan"):
+        ops.dda_neutral_flux(*args, betas, n_dir + 1, n_re, plan=plan)
