@@ -642,6 +642,11 @@ int petch_radiosity_assemble(petch_ctx* ctx, const int* hitface, int nf, int n_f
 int petch_radiosity_solve(petch_ctx* ctx, const int* row_ptr, const int* col, const double* D,
                           int nf, int n_ff, const float* bare, double beta, int n_iter, double tol,
                           double* G, float* out, int* iters_host);
+/* Two solves over one matrix (the F and O sticking of a coverage round) in the same n_iter > 0
+ * sweeps; each gives what petch_radiosity_solve gives for its beta. */
+int petch_radiosity_solve_pair(petch_ctx* ctx, const int* row_ptr, const int* col, const double* D,
+                               int nf, int n_ff, const float* bare, double beta_a, double beta_b,
+                               int n_iter, double* G_a, float* out_a, double* G_b, float* out_b);
 /* Adjoint of petch_radiosity_solve at its solution G (float64) for the output gradient gm
  * (float32, d loss / d out): the transposed system lambda = gG + diag(q) Aff^T lambda, with
  * q = 1 - clip(bare*beta,0,1) and gG = gm where 0 <= G <= 8, solved by Jacobi from lambda0 = gG

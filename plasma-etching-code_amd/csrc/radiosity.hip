@@ -7,7 +7,7 @@
 //             radix sort of (destination, ray id), so every row lists its sources in ray order
 //             and the float64 row sums are reproducible run to run.
 //   solve     G = D + Aff diag(1 - s) G with s = clip(bare*beta, 0, 1), Jacobi from G0 = D in
-//             float64 (one row per lane), n_iter sweeps (the reference's 40, threed.py:965-969)
+//             float64 (16 lanes per row), n_iter sweeps (the reference's 40, threed.py:965-969)
 //             or until max|dG| <= tol*max|G| (the converged solution the GMRES option of
 //             threed.py:973-982 approximates to 1e-3); output clip(G, 0, 8) (threed.py:985).
 //   adjoint   the implicit (fixed-point) adjoint of the solve, which the reference does not have:
@@ -64,38 +64,82 @@ __global__ void k_rad_escape(const int* __restrict__ hit, int nf, int n_ff,
   D[j] = (double)c / (double)n_ff;
 }
 
-__global__ void k_rad_q(const float* __restrict__ bare, double beta, int nf,
-                        double* __restrict__ q) {
-  int j = blockIdx.x * kBS + threadIdx.x;
+// NS solves of one matrix share its sweeps. The weighted iterates w = q G, q = 1 - clip(bare
+// beta, 0, 1), are kept interleaved (face-major), so a matrix entry costs one col read and one
+// gather of 8 NS bytes.
+template <int NS>
+struct RadSpecies {
+  double beta[NS];
+  double* q;
+  double* G[NS];   // the iterates, then the solutions
+  float* out[NS];  // clip(G, 0, 8)
+};
+
+// q, and the first iterate G = D with its w.
+template <int NS>
+__global__ void k_rad_init(const float* __restrict__ bare, const double* __restrict__ D, int nf,
+                           RadSpecies<NS> S, double* __restrict__ w) {
+  const int j = blockIdx.x * kBS + threadIdx.x;
   if (j >= nf) return;
-  double s = fmin(fmax((double)bare[j] * beta, 0.0), 1.0);
-  q[j] = 1.0 - s;
-}
-
-__global__ void k_rad_jacobi(const int* __restrict__ row_ptr, const int* __restrict__ col,
-                             const double* __restrict__ D, const double* __restrict__ q,
-                             const double* __restrict__ Gin, int nf, double inv_nff,
-                             double* __restrict__ Gout, unsigned long long* __restrict__ red) {
-  int i = blockIdx.x * kBS + threadIdx.x;
-  if (i >= nf) return;
-  double acc = 0.0;
-  for (int k = row_ptr[i], e = row_ptr[i + 1]; k < e; ++k) {
-    int j = col[k];
-    acc += q[j] * Gin[j];
-  }
-  double g = D[i] + inv_nff * acc;
-  Gout[i] = g;
-  if (red) {
-    // non-negative doubles order like their bit patterns
-    atomicMax(red, (unsigned long long)__double_as_longlong(fabs(g - Gin[i])));
-    atomicMax(red + 1, (unsigned long long)__double_as_longlong(fabs(g)));
+#pragma unroll
+  for (int s = 0; s < NS; ++s) {
+    const double q = 1.0 - fmin(fmax((double)bare[j] * S.beta[s], 0.0), 1.0);
+    S.q[(size_t)NS * j + s] = q;
+    S.G[s][j] = D[j];
+    w[(size_t)NS * j + s] = q * D[j];
   }
 }
 
-__global__ void k_rad_out(const double* __restrict__ G, int nf, float* __restrict__ out) {
-  int i = blockIdx.x * kBS + threadIdx.x;
+// One Jacobi sweep, kRadLanes lanes per row: the lanes read consecutive entries of the row and
+// their sums are added in a fixed order, so the row sums are reproducible. A row holds about
+// n_ff = 64 entries, which 16 lanes take in four coalesced reads, four rows to a wavefront; with
+// one lane per row the entries of 64 rows were read scattered, one after another. A row reads no
+// iterate G but its own, so G is updated in place; red, when given, receives max |dG| and max |G|.
+constexpr int kRadLanes = 16;
+
+template <int NS>
+__global__ void __launch_bounds__(kBS) k_rad_jacobi(const int* __restrict__ row_ptr,
+                                                    const int* __restrict__ col,
+                                                    const double* __restrict__ D, int nf,
+                                                    double inv_nff, RadSpecies<NS> S,
+                                                    const double* __restrict__ win,
+                                                    double* __restrict__ wout,
+                                                    unsigned long long* __restrict__ red) {
+  const int i = blockIdx.x * (kBS / kRadLanes) + threadIdx.x / kRadLanes;
+  const int lane = threadIdx.x % kRadLanes;
+  double acc[NS] = {};
+  if (i < nf) {
+    for (int k = row_ptr[i] + lane, e = row_ptr[i + 1]; k < e; k += kRadLanes) {
+      const size_t j = (size_t)NS * col[k];
+#pragma unroll
+      for (int s = 0; s < NS; ++s) acc[s] += win[j + s];
+    }
+  }
+#pragma unroll
+  for (int d = kRadLanes / 2; d >= 1; d >>= 1) {
+#pragma unroll
+    for (int s = 0; s < NS; ++s) acc[s] += __shfl_xor(acc[s], d, kRadLanes);
+  }
+  if (i >= nf || lane != 0) return;
+#pragma unroll
+  for (int s = 0; s < NS; ++s) {
+    const double g = D[i] + inv_nff * acc[s];
+    if (red) {
+      // non-negative doubles order like their bit patterns
+      atomicMax(red, (unsigned long long)__double_as_longlong(fabs(g - S.G[s][i])));
+      atomicMax(red + 1, (unsigned long long)__double_as_longlong(fabs(g)));
+    }
+    S.G[s][i] = g;
+    wout[(size_t)NS * i + s] = S.q[(size_t)NS * i + s] * g;
+  }
+}
+
+template <int NS>
+__global__ void k_rad_out(int nf, RadSpecies<NS> S) {
+  const int i = blockIdx.x * kBS + threadIdx.x;
   if (i >= nf) return;
-  out[i] = (float)fmin(fmax(G[i], 0.0), 8.0);
+#pragma unroll
+  for (int s = 0; s < NS; ++s) S.out[s][i] = (float)fmin(fmax(S.G[s][i], 0.0), 8.0);
 }
 
 // Adjoint set-up: q = 1 - clip(bare beta, 0, 1); gG = gm where 0 <= G <= 8 (the clip passes the
@@ -201,6 +245,33 @@ int jacobi_drive(petch_ctx* ctx, Sweep sweep, double** a, double** c, unsigned l
   return PETCH_OK;
 }
 
+template <int NS>
+int rad_solve(petch_ctx* ctx, const int* row_ptr, const int* col, const double* D, int nf,
+              int n_ff, const float* bare, RadSpecies<NS> S, int n_iter, double tol,
+              int* iters_host) {
+  const size_t n = (size_t)NS * nf;
+  double* w = (double*)petch_scratch(ctx, SCR_RAD_C, 3 * n * sizeof(double) + 64);
+  if (!w) return PETCH_E_HIP;
+  S.q = w;
+  double *a = w + n, *c = w + 2 * n;
+  unsigned long long* red = (unsigned long long*)(w + 3 * n);
+  const dim3 g(petch_blocks(nf, kBS)), gr(petch_blocks(nf, kBS / kRadLanes)), b(kBS);
+  hipLaunchKernelGGL(k_rad_init<NS>, g, b, 0, ctx->stream, bare, D, nf, S, a);
+  PETCH_LAUNCH_CHECK(ctx);
+  const double inv = 1.0 / (double)n_ff;
+  int done = 0;
+  auto sweep = [&](double* in, double* out, unsigned long long* r) {
+    hipLaunchKernelGGL(k_rad_jacobi<NS>, gr, b, 0, ctx->stream, row_ptr, col, D, nf, inv, S, in,
+                       out, r);
+  };
+  const int rc = jacobi_drive(ctx, sweep, &a, &c, red, n_iter, tol, &done);
+  if (rc != PETCH_OK) return rc;
+  hipLaunchKernelGGL(k_rad_out<NS>, g, b, 0, ctx->stream, nf, S);
+  PETCH_LAUNCH_CHECK(ctx);
+  if (iters_host) *iters_host = done;
+  return PETCH_OK;
+}
+
 }  // namespace
 
 extern "C" int petch_radiosity_assemble(petch_ctx* ctx, const int* hitface, int nf, int n_ff,
@@ -246,31 +317,22 @@ extern "C" int petch_radiosity_solve(petch_ctx* ctx, const int* row_ptr, const i
   PETCH_ARG(ctx, nf >= 0 && n_ff > 0, "radiosity_solve: bad size");
   if (iters_host) *iters_host = 0;
   if (nf == 0) return PETCH_OK;
-  double* w = (double*)petch_scratch(ctx, SCR_RAD_C, (size_t)nf * 16 + 64);
-  if (!w) return PETCH_E_HIP;
-  double* q = w;
-  double* G2 = w + nf;
-  unsigned long long* red = (unsigned long long*)(w + 2 * (size_t)nf);
-  dim3 g(petch_blocks(nf, kBS)), b(kBS);
-  hipLaunchKernelGGL(k_rad_q, g, b, 0, ctx->stream, bare, beta, nf, q);
-  PETCH_LAUNCH_CHECK(ctx);
-  PETCH_HIP(ctx, hipMemcpyAsync(G, D, (size_t)nf * 8, hipMemcpyDeviceToDevice, ctx->stream));
-  double inv = 1.0 / (double)n_ff;
-  double* a = G;
-  double* c = G2;
-  int done = 0;
-  auto sweep = [&](double* in, double* out_, unsigned long long* r) {
-    hipLaunchKernelGGL(k_rad_jacobi, g, b, 0, ctx->stream, row_ptr, col, D, q, in, nf, inv, out_,
-                       r);
-  };
-  int rc = jacobi_drive(ctx, sweep, &a, &c, red, n_iter, tol, &done);
-  if (rc != PETCH_OK) return rc;
-  if (a != G)
-    PETCH_HIP(ctx, hipMemcpyAsync(G, a, (size_t)nf * 8, hipMemcpyDeviceToDevice, ctx->stream));
-  hipLaunchKernelGGL(k_rad_out, g, b, 0, ctx->stream, G, nf, out);
-  PETCH_LAUNCH_CHECK(ctx);
-  if (iters_host) *iters_host = done;
-  return PETCH_OK;
+  RadSpecies<1> S{{beta}, nullptr, {G}, {out}};
+  return rad_solve(ctx, row_ptr, col, D, nf, n_ff, bare, S, n_iter, tol, iters_host);
+}
+
+extern "C" int petch_radiosity_solve_pair(petch_ctx* ctx, const int* row_ptr, const int* col,
+                                          const double* D, int nf, int n_ff, const float* bare,
+                                          double beta_a, double beta_b, int n_iter, double* G_a,
+                                          float* out_a, double* G_b, float* out_b) {
+  PETCH_ARG(ctx, ctx && row_ptr && col && D && bare && G_a && out_a && G_b && out_b,
+            "radiosity_solve_pair: null pointer");
+  PETCH_ARG(ctx, nf >= 0 && n_ff > 0 && n_iter > 0, "radiosity_solve_pair: bad size");
+  PETCH_ARG(ctx, G_a != G_b && out_a != out_b,
+            "radiosity_solve_pair: the two solves need distinct outputs");
+  if (nf == 0) return PETCH_OK;
+  RadSpecies<2> S{{beta_a, beta_b}, nullptr, {G_a, G_b}, {out_a, out_b}};
+  return rad_solve(ctx, row_ptr, col, D, nf, n_ff, bare, S, n_iter, 0.0, nullptr);
 }
 
 extern "C" int petch_radiosity_adjoint(petch_ctx* ctx, const int* hitface, int nf, int n_ff,

@@ -370,8 +370,12 @@ def radiosity_flux(mesh, phi, geo, par, n_ion, seed, flags, n_ff=64, n_fp=4):
     bare = torch.ones((F,), dtype=torch.float32, device=mesh.device)
     m_F = m_O = torch.zeros((F,), dtype=torch.float32, device=mesh.device)
     for _ in range(n_fp):
-        m_F = ops.radiosity_solve(row_ptr, col, D, F, n_ff, bare, betaE, n_iter)[0]
-        m_O = ops.radiosity_solve(row_ptr, col, D, F, n_ff, bare, betaO, n_iter)[0]
+        if n_iter > 0:
+            m_F, m_O = ops.radiosity_solve_pair(row_ptr, col, D, F, n_ff, bare, (betaE, betaO),
+                                                n_iter)
+        else:                    # to convergence: each species stops by its own test
+            m_F = ops.radiosity_solve(row_ptr, col, D, F, n_ff, bare, betaE, n_iter)[0]
+            m_O = ops.radiosity_solve(row_ptr, col, D, F, n_ff, bare, betaO, n_iter)[0]
         bare = ops.belen_coverage(m_i, m_F, m_O, cos_i, ion_yield, chem)
     return dict(m_i=m_i, m_F=m_F, m_O=m_O, cos_i=cos_i, bare=bare, ion_yield=ion_yield)
 

@@ -927,6 +927,18 @@ def radiosity_solve(row_ptr, col, D, nf, n_ff, bare, beta, n_iter=40, tol=1e-10)
     return out, G[:nf], it.value
 
 
+def radiosity_solve_pair(row_ptr, col, D, nf, n_ff, bare, betas, n_iter=40):
+    """The two (F,) float32 multipliers radiosity_solve gives for betas = (a, b), from shared
+    sweeps (petch_radiosity_solve_pair)."""
+    G = torch.empty((2, max(nf, 1)), dtype=torch.float64, device=D.device)
+    out = torch.empty((2, nf), dtype=f32, device=D.device)
+    if nf:
+        _ctx(D).call("petch_radiosity_solve_pair", ptr(row_ptr, i32), ptr(col, i32),
+                     ptr(D, torch.float64), int(nf), int(n_ff), ptr(bare, f32), float(betas[0]),
+                     float(betas[1]), int(n_iter), ptr(G[0]), ptr(out[0]), ptr(G[1]), ptr(out[1]))
+    return out[0], out[1]
+
+
 def radiosity_adjoint(hitface, nf, n_ff, G, bare, beta, gm, n_iter=40, tol=1e-10):
     """(gD float64 = d loss / dD, gbare float32 = d loss / d bare, sweeps) for the output gradient
     gm of radiosity_solve at its solution G (petch_radiosity_adjoint)."""
@@ -991,19 +1003,6 @@ def knudsen_face_flux(phi, dx, sub_top, trench, centroids, gas_normals, areas, b
     return outs
 
 
-def dda_neutral_flux(phi, dx, centroids, gas_normals, areas, bare, betas, n_dir=64, n_reemit=12,
-                     periodic_y=0, plan=None):
-    """dda_neutral_flux (dda.py:138-220) for the sticking coefficients bare * beta of the one or
-    two betas (petch_dda_neutral_flux): one (F,) float32 multiplier per beta. plan: dda_march's
-    result for the same surface, when several coverages are solved on it."""
-    from ._abi import DdaParams
-    nx, ny, nz = _shape3(phi)
-    F = int(centroids.shape[0])
-    betas = list(betas)
-    if not 1 <= len(betas) <= 2:
-        raise ValueError("dda_neutral_flux: one or two betas")
-    outs = [torch.empty((F,), dtype=f32, device=phi.device) for _ in betas]
-    p = DdaParams(float(dx), int(n_dir), int(n_reemit), int(bool(periodic_y)), float(betas[0]),
 def dda_march(phi, dx, centroids, gas_normals, n_dir=64, periodic_y=0):
     """The rays of dda_neutral_flux marched once (petch_dda_march), as a plan for any number of
     its calls on the same phi, dx, faces, n_dir and periodic_y."""
@@ -1019,6 +1018,19 @@ def dda_march(phi, dx, centroids, gas_normals, n_dir=64, periodic_y=0):
     return plan
 
 
+def dda_neutral_flux(phi, dx, centroids, gas_normals, areas, bare, betas, n_dir=64, n_reemit=12,
+                     periodic_y=0, plan=None):
+    """dda_neutral_flux (dda.py:138-220) for the sticking coefficients bare * beta of the one or
+    two betas (petch_dda_neutral_flux): one (F,) float32 multiplier per beta. plan: dda_march's
+    result for the same surface, when several coverages are solved on it."""
+    from ._abi import DdaParams
+    nx, ny, nz = _shape3(phi)
+    F = int(centroids.shape[0])
+    betas = list(betas)
+    if not 1 <= len(betas) <= 2:
+        raise ValueError("dda_neutral_flux: one or two betas")
+    outs = [torch.empty((F,), dtype=f32, device=phi.device) for _ in betas]
+    p = DdaParams(float(dx), int(n_dir), int(n_reemit), int(bool(periodic_y)), float(betas[0]),
                   float(betas[-1]))
     if F:
         args = [ptr(phi, f32, "phi"), nx, ny, nz, ptr(centroids, f32, "centroids"),

@@ -614,3 +614,30 @@ def test_batched_ion_finish_equals_the_separate_calls():
     for it, ref in zip(items, refs):
         for j in range(5):
             assert torch.equal(it['out'][j], ref[j]), j
+
+
+@pytest.mark.parametrize("nf,n_ff", [(1, 1), (15, 3), (16, 16), (17, 17), (300, 64), (1025, 5)])
+def test_radiosity_pair_equals_single_solves(nf, n_ff):
+    """Rows of every length about the 16 lanes that share one (empty rows and one row that takes
+    a third of all rays among them): the paired sweeps give the single solves' values to the bit,
+    and both a dense float64 Jacobi's to 1e-13 of the largest value (sums of at most 300 x 64
+    positive terms, 40 sweeps that do not amplify: Aff's column sums are at most 1)."""
+    from petch import ops
+    import torch
+    rng = np.random.default_rng(nf)
+    hit = rng.integers(-1, max(nf // 2, 1), (nf, n_ff)).astype(np.int32)
+    hit[rng.random((nf, n_ff)) < 0.33] = nf - 1
+    row_ptr, col, D = ops.radiosity_assemble(_t(hit.ravel()), nf, n_ff)
+    bare = rng.uniform(0.0, 1.2, nf).astype(np.float32)
+    A = np.zeros((nf, nf))
+    np.add.at(A, (hit[hit >= 0], np.nonzero(hit >= 0)[0]), 1.0 / n_ff)
+    D0 = (hit < 0).mean(axis=1)
+    pair = ops.radiosity_solve_pair(row_ptr, col, D, nf, n_ff, _t(bare), (0.3, 1.0))
+    for beta, m in zip((0.3, 1.0), pair):
+        one, G, _ = ops.radiosity_solve(row_ptr, col, D, nf, n_ff, _t(bare), beta, 40)
+        assert torch.equal(m, one)
+        q = 1.0 - np.clip(bare.astype(np.float64) * beta, 0.0, 1.0)
+        g = D0.copy()
+        for _ in range(40):
+            g = D0 + A @ (q * g)
+        np.testing.assert_allclose(G.cpu().numpy(), g, rtol=0, atol=1e-13 * max(g.max(), 1.0))
