@@ -216,6 +216,15 @@ typedef struct petch_mc_item {
   int* nf_out;
 } petch_mc_item;
 int petch_marching_cubes_batch(petch_ctx* ctx, int n, const petch_mc_item* items);
+/* The same, and what petch_bvh_set_grid needs to know of the cells: cells (may be NULL) receives
+ * nx*ny*nz words, first face << 4 | number of faces of the cell that starts at each node, 0 for
+ * a cell without faces. The batch takes one pointer per item (the array or an entry may be
+ * NULL). */
+int petch_marching_cubes_cells(petch_ctx* ctx, const float* phi, int nx, int ny, int nz, double dx,
+                               float* verts, int* faces, int cap_v, int cap_f, uint32_t* cells,
+                               int* nv_host, int* nf_host);
+int petch_marching_cubes_batch_cells(petch_ctx* ctx, int n, const petch_mc_item* items,
+                                     uint32_t* const* cells);
 
 /* Face centroids (nf,3) = vertex mean, areas (nf) = 0.5|cross|, unit normals (nf,3) (zero for a
  * degenerate face) — threed.py:96-99 and _face_normals_k threed.py:228-234. Any output may be
@@ -268,6 +277,22 @@ int petch_bvh_build_batch(petch_ctx* ctx, int n, petch_bvh* const* bvhs_host,
  * meshes of 32k faces or more and 0 below. A caller that knows its ray budget picks the
  * trade-off (no reference counterpart: wp.Mesh has one builder). */
 int petch_bvh_set_quality(petch_ctx* ctx, petch_bvh* bvh, int quality);
+/* Tells a built BVH that its mesh is the marching-cubes surface of an (nx, ny, nz) grid of spacing
+ * dx: every triangle lies in one cell, whose word in `cells` (petch_marching_cubes_cells, the same
+ * verts and faces) lists it. Ray traces and queries then walk the cells instead of the tree, with the
+ * same hits; point queries keep the tree. The BVH keeps copies of all it needs; a new build
+ * forgets the grid. A triangle outside its cell sets the guard flag (code 4). No reference
+ * counterpart. */
+typedef struct petch_grid_item {
+  petch_bvh* bvh;
+  const float* verts;
+  const int* faces;
+  const uint32_t* cells;
+  int nx, ny, nz;
+  double dx;
+} petch_grid_item;
+int petch_bvh_set_grid(petch_ctx* ctx, const petch_grid_item* item);
+int petch_bvh_set_grid_batch(petch_ctx* ctx, int n, const petch_grid_item* items);
 /* wp.mesh_query_ray(mesh, o, d, tmax) (threed.py:306,366,524,569,629,916): closest two-sided hit
  * with 0 < t < tmax (watertight test); face = -1 and t = -1 on a miss. t may be NULL. */
 int petch_bvh_query_ray(petch_ctx* ctx, const petch_bvh* bvh, const float* orig,

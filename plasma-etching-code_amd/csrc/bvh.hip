@@ -16,8 +16,10 @@
 
 #include <stdlib.h>
 #include "bvh.h"
+#include "gridwalk.h"
 #include "scan.h"
 
+bool petch_grid_view(const petch_bvh* b, petch::GridView* v);
 int petch_radix_sort_pairs(petch_ctx* ctx, uint32_t* keys, uint32_t* vals, uint32_t* ktmp,
                            uint32_t* vtmp, int n, int bits);
 
@@ -794,6 +796,17 @@ __global__ void k_query_ray(BvhView b, const float* __restrict__ o, const float*
   if (tout) tout[i] = h.face >= 0 ? h.t : -1.f;
 }
 
+__global__ void k_query_ray_walk(petch::GridView g, BvhView tree, const float* __restrict__ o,
+                                 const float* __restrict__ d, int n, float tmax,
+                                 int* __restrict__ face, float* __restrict__ tout) {
+  int i = blockIdx.x * kBS + threadIdx.x;
+  if (i >= n) return;
+  petch::Hit h = petch::walk_closest_hit(g, tree, petch::v3(o[3 * i], o[3 * i + 1], o[3 * i + 2]),
+                                         petch::v3(d[3 * i], d[3 * i + 1], d[3 * i + 2]), tmax);
+  face[i] = h.face;
+  if (tout) tout[i] = h.face >= 0 ? h.t : -1.f;
+}
+
 __global__ void k_query_point(BvhView b, const float* __restrict__ p, int n, float maxd,
                               int* __restrict__ face, float* __restrict__ dist) {
   int i = blockIdx.x * kBS + threadIdx.x;
@@ -816,6 +829,8 @@ BvhView petch_bvh_view(const petch_bvh* b) {
   v.root = (b->work && b->nf > 1) ? carve(b->work, b->cap_f).root : nullptr;
   return v;
 }
+
+int* petch_bvh_err(const petch_bvh* b) { return b->work ? carve(b->work, b->cap_f).err : nullptr; }
 
 extern "C" int petch_bvh_create(petch_ctx* ctx, petch_bvh** out) {
   PETCH_ARG(ctx, ctx && out, "bvh_create: null pointer");
@@ -843,6 +858,8 @@ extern "C" int petch_bvh_destroy(petch_ctx* ctx, petch_bvh* b) {
   if (b->tris) (void)hipFree(b->tris);
   if (b->work) (void)hipFree(b->work);
   if (b->aux) (void)hipFree(b->aux);
+  if (b->cells) (void)hipFree(b->cells);
+  if (b->gtris) (void)hipFree(b->gtris);
   free(b);
   return PETCH_OK;
 }
@@ -938,6 +955,7 @@ int build_prepare(petch_ctx* ctx, petch_bvh* b, const float* verts, const int* f
   PETCH_ARG(ctx, nf == 0 || (verts && faces), "bvh_build: null mesh");
   b->nv = nv;
   b->nf = 0;
+  b->grid_n[0] = 0;
   refit->n = 0;
   const int rc0 = ensure_capacity(ctx, b, nf);
   if (rc0 != PETCH_OK) return rc0;
@@ -1040,6 +1058,7 @@ extern "C" int petch_bvh_build_batch(petch_ctx* ctx, int n, petch_bvh* const* bv
     }
     b->nv = nv[t];
     b->nf = 0;
+    b->grid_n[0] = 0;
     const int rc = ensure_capacity(ctx, b, nf[t]);
     if (rc != PETCH_OK) return rc;
     BuildItem it;
@@ -1143,6 +1162,13 @@ extern "C" int petch_bvh_query_ray(petch_ctx* ctx, const petch_bvh* b, const flo
   PETCH_ARG(ctx, ctx && b && orig && dir && face, "bvh_query_ray: null pointer");
   PETCH_ARG(ctx, n >= 0, "bvh_query_ray: n < 0");
   if (n == 0) return PETCH_OK;
+  petch::GridView g;
+  if (petch_grid_view(b, &g)) {
+    hipLaunchKernelGGL(k_query_ray_walk, dim3(petch_blocks(n, kBS)), dim3(kBS), 0, ctx->stream, g,
+                       petch_bvh_view(b), orig, dir, n, tmax, face, t);
+    PETCH_LAUNCH_CHECK(ctx);
+    return PETCH_OK;
+  }
   hipLaunchKernelGGL(k_query_ray, dim3(petch_blocks(n, kBS)), dim3(kBS), 0, ctx->stream,
                      petch_bvh_view(b), orig, dir, n, tmax, face, t);
   PETCH_LAUNCH_CHECK(ctx);

@@ -37,6 +37,7 @@ enum PetchScratch {
   SCR_LS_BRICK,      // batched level-set stages: per-brick activity flags and list counters
   SCR_LS_LIST,       // batched level-set stages: lists of the bricks a launch processes
   SCR_SORT_MANY,     // batched radix sort: per-array digit tables
+  SCR_GRID,          // cell distances of a surface's grid, one axis at a time
   SCR_REDEP,         // redeposition: float64 emission CDF and its workgroup partials
   SCR_COUNT
 };
@@ -77,6 +78,13 @@ struct petch_bvh {
   int quality;             // build quality: -1 by mesh size, 0 Morton + fixed collapse,
                            // 1 Morton + area collapse, 2 clustered (PLOC) + area collapse
   float root_lo[3], root_hi[3];
+  // the cells of the grid the mesh was cut from (petch_bvh_set_grid), for ray walks
+  uint32_t* cells;         // one word per node (gridwalk.h)
+  void* gtris;             // nf triangles in face order, 48 B each
+  size_t cells_cap;        // nodes
+  int gtris_cap;           // faces
+  int grid_n[3];           // nodes per axis; 0 when the mesh has no grid
+  double grid_dx;
 };
 
 int petch_set_error(petch_ctx* ctx, int code, const char* fmt, ...);

@@ -216,7 +216,8 @@ __device__ __forceinline__ int mc_append_cell(bool live, long long n, uint32_t* 
 // grid; the batched launches pass the block's index within its grid).
 __device__ __forceinline__ void mc_count_block(const float* __restrict__ phi, const Grid& g,
                                                long long N, long long blk, int* __restrict__ bv,
-                                               int* __restrict__ bt) {
+                                               int* __restrict__ bt,
+                                               uint32_t* __restrict__ words) {
   __shared__ uint32_t cells[kMcMaxRounds * kMcBS];
   int vc = 0, na = 0;
   for (int r = 0; r < g.rounds; ++r) {
@@ -227,6 +228,7 @@ __device__ __forceinline__ void mc_count_block(const float* __restrict__ phi, co
       node_ijk(g, n, i, j, k);
       vc += __popc(vertex_flags(phi, g, n, i, j, k));
       s = cell_signs(phi, g, n, i, j, k);
+      if (words) words[n] = 0u;
     }
     na = mc_append_cell(s != 0 && s != 255, n, cells, na);
   }
@@ -247,8 +249,9 @@ __device__ __forceinline__ void mc_count_block(const float* __restrict__ phi, co
 
 __global__ void __launch_bounds__(kMcBS) k_mc_count(const float* __restrict__ phi, Grid g,
                                                     long long N, int* __restrict__ bv,
-                                                    int* __restrict__ bt) {
-  mc_count_block(phi, g, N, blockIdx.x, bv, bt);
+                                                    int* __restrict__ bt,
+                                                    uint32_t* __restrict__ words) {
+  mc_count_block(phi, g, N, blockIdx.x, bv, bt, words);
 }
 
 // The emit passes skip a block that holds no vertex (no face): its per-node vertex tables are
@@ -400,7 +403,8 @@ __device__ __forceinline__ void mc_faces_block(const float* __restrict__ phi, co
                                                const int* __restrict__ vbase,
                                                const uint8_t* __restrict__ vflg,
                                                int* __restrict__ faces, int cap_f, long long nb,
-                                               const int* __restrict__ total) {
+                                               const int* __restrict__ total,
+                                               uint32_t* __restrict__ words) {
   if (mc_block_empty(bt, blk, nb, total)) return;
   __shared__ uint32_t cells[kMcMaxRounds * kMcBS];
   int na = 0;
@@ -431,7 +435,11 @@ __device__ __forceinline__ void mc_faces_block(const float* __restrict__ phi, co
     int tot;
     const int tb = base + petch::block_excl_scan<kMcBS>(tc, tot);
     base += tot;
-    if (tc) mc_cell_faces(g, n, f, tb, vbase, vflg, faces, cap_f);
+    if (tc) {
+      // at most 10 faces a cell: 12 crossing edges in one loop
+      if (words) words[n] = ((uint32_t)tb << 4) | (uint32_t)tc;
+      mc_cell_faces(g, n, f, tb, vbase, vflg, faces, cap_f);
+    }
   }
 }
 
@@ -440,8 +448,9 @@ __global__ void __launch_bounds__(kMcBS) k_mc_faces(const float* __restrict__ ph
                                                     const int* __restrict__ vbase,
                                                     const uint8_t* __restrict__ vflg,
                                                     int* __restrict__ faces, int cap_f,
-                                                    long long nb, const int* __restrict__ total) {
-  mc_faces_block(phi, g, N, blockIdx.x, bt, vbase, vflg, faces, cap_f, nb, total);
+                                                    long long nb, const int* __restrict__ total,
+                                                    uint32_t* __restrict__ words) {
+  mc_faces_block(phi, g, N, blockIdx.x, bt, vbase, vflg, faces, cap_f, nb, total, words);
 }
 
 // The passes of many grids (the features of a batched step), one launch each: grid t owns the
@@ -458,6 +467,7 @@ struct McGrid {
   uint8_t* vflg;
   float* verts;
   int* faces;
+  uint32_t* words;  // the cells' words (first face << 4 | faces, 0 without a face), or null
   int cap_v, cap_f;
 };
 
@@ -473,7 +483,7 @@ __device__ __forceinline__ int mc_grid_of(const McGrid* __restrict__ t, int n) {
 
 __global__ void __launch_bounds__(kMcBS) k_mc_count_many(const McGrid* __restrict__ t, int n) {
   const McGrid& m = t[mc_grid_of(t, n)];
-  mc_count_block(m.phi, m.g, m.N, blockIdx.x - m.blk0, m.bv, m.bt);
+  mc_count_block(m.phi, m.g, m.N, blockIdx.x - m.blk0, m.bv, m.bt, m.words);
 }
 
 __global__ void __launch_bounds__(1024) k_mc_scan_many(const McGrid* __restrict__ t) {
@@ -508,7 +518,7 @@ __global__ void __launch_bounds__(kMcBS) k_mc_verts_many(const McGrid* __restric
 __global__ void __launch_bounds__(kMcBS) k_mc_faces_many(const McGrid* __restrict__ t, int n) {
   const McGrid& m = t[mc_grid_of(t, n)];
   mc_faces_block(m.phi, m.g, m.N, blockIdx.x - m.blk0, m.bt, m.vbase, m.vflg, m.faces, m.cap_f,
-                 m.nb, m.totals + 1);
+                 m.nb, m.totals + 1, m.words);
 }
 
 }  // namespace
@@ -516,6 +526,14 @@ __global__ void __launch_bounds__(kMcBS) k_mc_faces_many(const McGrid* __restric
 extern "C" int petch_marching_cubes(petch_ctx* ctx, const float* phi, int nx, int ny, int nz,
                                     double dx, float* verts, int* faces, int cap_v, int cap_f,
                                     int* nv_host, int* nf_host) {
+  return petch_marching_cubes_cells(ctx, phi, nx, ny, nz, dx, verts, faces, cap_v, cap_f, nullptr,
+                                    nv_host, nf_host);
+}
+
+extern "C" int petch_marching_cubes_cells(petch_ctx* ctx, const float* phi, int nx, int ny, int nz,
+                                          double dx, float* verts, int* faces, int cap_v,
+                                          int cap_f, uint32_t* cells, int* nv_host,
+                                          int* nf_host) {
   PETCH_ARG(ctx, ctx && phi && nv_host && nf_host, "marching_cubes: null pointer");
   PETCH_ARG(ctx, nx > 0 && ny > 0 && nz > 0, "marching_cubes: bad shape %d,%d,%d", nx, ny, nz);
   PETCH_ARG(ctx, cap_v >= 0 && cap_f >= 0, "marching_cubes: negative capacity");
@@ -534,7 +552,7 @@ extern "C" int petch_marching_cubes(petch_ctx* ctx, const float* phi, int nx, in
   int* bt = blk + nb;
   int* totals = blk + 2 * nb;
   hipLaunchKernelGGL(k_mc_count, dim3((unsigned)nb), dim3(kMcBS), 0, ctx->stream, phi, g, N, bv,
-                     bt);
+                     bt, cells);
   PETCH_LAUNCH_CHECK(ctx);
   hipLaunchKernelGGL(petch::k_scan_partials2, dim3(1), dim3(1024), 0, ctx->stream, bv, bt,
                      (int)nb, totals);
@@ -559,12 +577,17 @@ extern "C" int petch_marching_cubes(petch_ctx* ctx, const float* phi, int nx, in
                      bv, vbase, vflg, verts, cap_v, nb, totals);
   PETCH_LAUNCH_CHECK(ctx);
   hipLaunchKernelGGL(k_mc_faces, dim3((unsigned)nb), dim3(kMcBS), 0, ctx->stream, phi, g, N, bt,
-                     vbase, vflg, faces, cap_f, nb, totals + 1);
+                     vbase, vflg, faces, cap_f, nb, totals + 1, cells);
   PETCH_LAUNCH_CHECK(ctx);
   return PETCH_OK;
 }
 
 extern "C" int petch_marching_cubes_batch(petch_ctx* ctx, int n, const petch_mc_item* items) {
+  return petch_marching_cubes_batch_cells(ctx, n, items, nullptr);
+}
+
+extern "C" int petch_marching_cubes_batch_cells(petch_ctx* ctx, int n, const petch_mc_item* items,
+                                                uint32_t* const* cells_out) {
   PETCH_ARG(ctx, ctx && n >= 0 && (n == 0 || items), "marching_cubes_batch: null pointer or n < 0");
   if (n == 0) return PETCH_OK;
   // block partial sums of every grid side by side, then the totals of every grid
@@ -589,6 +612,7 @@ extern "C" int petch_marching_cubes_batch(petch_ctx* ctx, int n, const petch_mc_
     m.dx = a.dx;
     m.verts = a.verts;
     m.faces = a.faces;
+    m.words = cells_out ? cells_out[f] : nullptr;
     m.cap_v = a.cap_v;
     m.cap_f = a.cap_f;
     t.push_back(m);

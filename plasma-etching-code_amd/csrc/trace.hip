@@ -15,26 +15,35 @@
 // loop is the hit of the caller's query (the reference repeats the same query), so it is reused.
 #include "common.h"
 #include "bvh.h"
+#include "gridwalk.h"
 #include "rng.h"
 
+#include <type_traits>
 #include <vector>
 
 using petch::BvhView;
+using petch::GridView;
 using petch::Hit;
 using petch::Rng;
 using petch::Vec3;
 using petch::v3;
 
 petch::BvhView petch_bvh_view(const petch_bvh* b);
+bool petch_grid_view(const petch_bvh* b, petch::GridView* v);
 
 namespace {
 
+// Rays that a walk trace leaves to the tree (Ties): at most kMaxTies of a launch, the others keep
+// the walk's own choice.
+constexpr unsigned kMaxTies = 65536;
+
 // Per-context 64-bit hit counters (slot 0 neutral, 1 ion), read by petch_trace_hit_counts;
-// slots 2-3 hold the ray-queue cursor of the persistent trace launches.
+// slots 2-3 hold the ray-queue cursor of the persistent trace launches and the number of their
+// ties, whose list follows.
 unsigned long long* petch_hit_counter(petch_ctx* ctx, int which) {
   bool fresh = ctx->scr_cap[SCR_TRACE] == 0;
   unsigned long long* c =
-      (unsigned long long*)petch_scratch(ctx, SCR_TRACE, 4 * sizeof(unsigned long long));
+      (unsigned long long*)petch_scratch(ctx, SCR_TRACE, (4 + kMaxTies) * sizeof(unsigned long long));
   if (c && fresh && hipMemsetAsync(c, 0, 4 * sizeof(unsigned long long), ctx->stream) != hipSuccess)
     return nullptr;
   return c ? c + which : nullptr;
@@ -163,7 +172,8 @@ constexpr int kMaxWraps = 256;
 // On a trench whose mesh stops one cell short of the periodic faces (the grid spans
 // [0, (n-1) dx], the period n dx), the rays that slip through that strip fall below the floor and
 // would spend the 256 wraps there: over half of all queries of a neutral trace.
-__device__ __forceinline__ bool never_returns(const BvhView& bv, Vec3 o, Vec3 d) {
+template <class V>
+__device__ __forceinline__ bool never_returns(const V& bv, Vec3 o, Vec3 d) {
   if (!bv.root) return false;
   return (o.z < bv.root[2] && d.z <= 0.f) || (o.z > bv.root[5] && d.z >= 0.f);
 }
@@ -186,7 +196,8 @@ __device__ __forceinline__ Hit trace_bc(const BvhView& bv, const Box& b, Vec3& o
   return petch::bvh_closest_hit(bv, o, d, 1.0e6f);
 }
 
-__device__ __forceinline__ Vec3 hit_normal(const BvhView& bv, int slot) {
+template <class V>
+__device__ __forceinline__ Vec3 hit_normal(const V& bv, int slot) {
   float4 q0 = bv.tris[3 * slot], q1 = bv.tris[3 * slot + 1], q2 = bv.tris[3 * slot + 2];
   Vec3 a = v3(q0.x, q0.y, q0.z);
   return petch::normalize(petch::cross(v3(q1.x, q1.y, q1.z) - a, v3(q2.x, q2.y, q2.z) - a));
@@ -197,7 +208,9 @@ __device__ __forceinline__ Vec3 hit_normal(const BvhView& bv, int slot) {
 // do not depend on the order of the adds, so the result is the same whatever the schedule; it is
 // the exact sum of the deposits rounded to 2^-32 (|sum| < 2^31 per face).
 constexpr double kFixScale = 4294967296.0;
-__device__ __forceinline__ void deposit(float* __restrict__ acc, int face, float v, int fixed) {
+__device__ __forceinline__ void deposit(float* __restrict__ acc, int face, float v, int fixed,
+                                        bool on = true) {
+  if (!on) return;
   if (fixed)
     atomicAdd((unsigned long long*)acc + face,
               (unsigned long long)__double2ll_rn((double)v * kFixScale));
@@ -230,6 +243,12 @@ __device__ __forceinline__ void count_hits(unsigned long long* __restrict__ ctr,
 struct RayQueue {
   unsigned* next;
   int n;
+  // the walk traces' share of a wavefront: rays per claim, lanes in use, and the live lanes at or
+  // below which it stops for hits and new rays
+  int chunk, lanes, refill_at;
+  // ties: their number and list (queue id, the ray's earlier hits)
+  unsigned* n_ties;
+  uint2* ties;
 };
 
 constexpr unsigned kRayChunk = 128;  // >= 64, so one chunk always covers a wavefront's refill
@@ -278,6 +297,9 @@ __device__ __forceinline__ bool claim_ray(const RayQueue& q, bool active, bool& 
 // comes from that ray's own Philox stream in a fixed order, so the result does not depend on
 // the schedule.
 constexpr int kRefillAt = 24;
+constexpr int kMinLanes = 8;
+constexpr int kTestsPerPhase = 2, kStepsPerPhase = 3;
+constexpr int kTieBlocks = 4;
 constexpr int kLdsStack = 8;  // traversal stack entries per lane held in LDS (16 KB/workgroup)
 // kMiss: the ray left the domain and the policy replays paths (P::kReplay), so it gets a say
 // (P::miss) before the lane goes idle.
@@ -306,7 +328,7 @@ __device__ __forceinline__ void persistent_trace(const P& pol, const RayQueue& q
       bool emit = false;
       if (st == kHit) {
         ++nh;
-        emit = pol.hit(R, T.h, o, d, e);
+        emit = pol.hit(R, T.h, o, d, e, true);
         st = kIdle;
       }
       if constexpr (P::kReplay) {
@@ -344,6 +366,147 @@ __device__ __forceinline__ void persistent_trace(const P& pol, const RayQueue& q
     }
   }
   count_hits(hits, nh);
+}
+
+// claim_ray for the walk traces: new rays for lanes that want one (`idle`, at most `room` of
+// them), from the wavefront's pool and then from a fresh chunk of any length. `exhausted` is set
+// when the counter has passed the end; the pool may still hold ids then.
+__device__ __forceinline__ bool claim_some(const RayQueue& q, bool idle, int room, bool& exhausted,
+                                           unsigned& pool, unsigned& pool_end, unsigned& ray) {
+  const int lane = threadIdx.x & 63;
+  const unsigned long long mask = __ballot(idle);
+  const unsigned cnt = (unsigned)min(__popcll(mask), room);
+  if (!cnt) return false;
+  const unsigned rank = (unsigned)__popcll(mask & ((1ull << lane) - 1ull));
+  const unsigned left = pool_end - pool, n = (unsigned)q.n, chunk = (unsigned)q.chunk;
+  unsigned id = pool + rank, got = min(left, cnt);
+  pool += got;
+  if (got < cnt && !exhausted) {
+    unsigned base = 0;
+    if (lane == 0) base = atomicAdd(q.next, chunk);
+    base = __shfl(base, 0, 64);
+    exhausted = base >= n || n - base <= chunk;
+    const unsigned end = base >= n ? base : min(base + chunk, n);
+    const unsigned more = min(end - base, cnt - got);
+    if (rank >= got) id = base + (rank - got);
+    got += more;
+    pool = base + more;
+    pool_end = end;
+  }
+  ray = id;
+  return idle && rank < got;
+}
+
+// The trace loop over a marching-cubes surface's cells (gridwalk.h), for the same policies. A
+// lane is between rays (kIdle, kHit, kMiss), stepping from cell to cell (kWalk), testing a cell's
+// triangles (kTri), or about to start a query (kBegin, after a wrap kWrap). Every iteration runs
+// the one of the three phases that most lanes are in, so each phase's instructions are issued for
+// many lanes at once: in the tree's loop a leaf test ran as soon as one lane had reached a leaf,
+// with 5 of 64 lanes active, and took nearly half of the issue slots.
+enum WalkLane {
+  kWIdle = 0,
+  kWWalk = petch::kWalkOn,
+  kWTri = petch::kWalkTri,
+  kWBegin = 3,
+  kWWrap = petch::kWalkMiss,
+  kWHit = petch::kWalkHit,
+  kWMiss = 6
+};
+
+template <class P>
+__device__ __forceinline__ void walk_trace(const P& pol, const RayQueue& q,
+                                           unsigned long long* __restrict__ hits) {
+  petch::Walk T;
+  typename P::Ray R;
+  Vec3 o = v3(0.f, 0.f, 0.f), d = v3(0.f, 0.f, -1.f);
+  petch::WalkRay rp;
+  int wraps = 0, skip = -1;
+  unsigned nh = 0;
+  int st = kWIdle;
+  bool exhausted = false;
+  unsigned pool = 0, pool_end = 0;  // this wavefront's unclaimed queue ids [pool, pool_end)
+  while (true) {
+    unsigned long long mw = __ballot(st == kWWalk), mt = __ballot(st == kWTri),
+                       mb = __ballot(st == kWBegin || st == kWWrap);
+    const int live = __popcll(mw | mt | mb);
+    if (live <= q.refill_at) {
+      const bool ended = st == kWHit || st == kWMiss;
+      if (pool < pool_end || !exhausted || __ballot(ended)) {
+        Emit e;
+        bool emit = false;
+        if (st == kWHit) {
+          ++nh;
+          st = kWIdle;
+          unsigned at = kMaxTies;
+          if (T.tie) at = atomicAdd(q.n_ties, 1u);
+          if (at < kMaxTies) {
+            --nh;
+            q.ties[at] = make_uint2(pol.id(R), pol.earlier(R));
+          } else {
+            emit = pol.hit(R, Hit{T.face, T.face, T.t}, o, d, e, true);
+            // a replayed path starts over from its source, not from this face
+            skip = (!P::kReplay || e.mode == kLobe) ? T.face : -1;
+          }
+        }
+        if constexpr (P::kReplay) {
+          if (st == kWMiss) {
+            emit = pol.miss(R, o, e);
+            skip = -1;
+            st = kWIdle;
+          }
+        }
+        const int busy = live + __popcll(__ballot(emit));
+        unsigned ray;
+        if (claim_some(q, st == kWIdle && !emit, q.lanes - busy, exhausted, pool, pool_end, ray)) {
+          pol.start(R, ray, o, e);
+          skip = -1;
+          emit = true;
+        }
+        if (emit) {
+          d = emit_dir(e);
+          rp = petch::walk_ray(d);
+          wraps = 0;
+          st = kWBegin;
+        }
+        mb = __ballot(st == kWBegin || st == kWWrap);
+      }
+      if (!(mw | mt | mb)) break;
+    }
+    const int nw = __popcll(mw), nt = __popcll(mt), nb = __popcll(mb);
+    const GridView& g = pol.view(R);
+    if (nb >= nw && nb >= nt) {
+      if (st == kWWrap) {
+        const Box& b = pol.box(R);
+        if (b.periodic && wraps < kMaxWraps && !never_returns(g, o, d) &&
+            wrap_ray(b, o, d, rp.inv)) {
+          ++wraps;
+          skip = -1;
+          st = kWBegin;
+        } else {
+          st = P::kReplay ? kWMiss : kWIdle;
+        }
+      }
+      if (st == kWBegin) st = petch::walk_begin(g, T, o, d, rp, 1.0e6f, skip);
+    } else if (nt >= nw) {
+#pragma unroll 1
+      for (int k = 0; k < kTestsPerPhase; ++k)
+        if (st == kWTri) st = petch::walk_test(g, T, o, rp);
+    } else {
+#pragma unroll 1
+      for (int k = 0; k < kStepsPerPhase; ++k)
+        if (st == kWWalk) st = petch::walk_step(g, T, o, d, rp);
+    }
+  }
+  count_hits(hits, nh);
+}
+
+template <class P>
+__device__ __forceinline__ void run_trace(const P& pol, const RayQueue& q,
+                                          unsigned long long* __restrict__ hits) {
+  if constexpr (std::is_same<typename P::View, GridView>::value)
+    walk_trace(pol, q, hits);
+  else
+    persistent_trace(pol, q, hits);
 }
 
 // _trace3d_cov_rr (threed.py:549-596): deposit w at every hit, w *= 1 - bare*beta, Russian
@@ -392,12 +555,13 @@ __device__ __forceinline__ void rr_emit(const Hit& h, Vec3 nn, const uint32_t u[
   o = p + 1.0e-4f * nn;
 }
 
+template <class V>
 __device__ __forceinline__ bool rr_bounce(float& w, int& bounce, uint64_t seed, unsigned ray,
-                                          const BvhView& bv, const Hit& h, float* __restrict__ fl,
-                                          int fixed, float S, Vec3& o, Vec3 d, Emit& e) {
+                                          const V& bv, const Hit& h, float* __restrict__ fl,
+                                          int fixed, float S, Vec3& o, Vec3 d, Emit& e, bool on) {
   Vec3 nn = hit_normal(bv, h.slot);
   if (petch::dot(nn, d) > 0.f) nn = -nn;
-  deposit(fl, h.face, w, fixed);
+  deposit(fl, h.face, w, fixed, on);
   float w2;
   bool reset;
   uint32_t u[4];
@@ -426,9 +590,11 @@ __device__ __forceinline__ void neutral_source(uint64_t seed, unsigned ray, cons
   }
 }
 
+template <class V>
 struct NeutralRR {
+  using View = V;
   static constexpr bool kReplay = false;
-  BvhView bv;
+  V bv;
   Box b;
   Source src;
   const float* __restrict__ bare;
@@ -443,7 +609,9 @@ struct NeutralRR {
     int sp;
     unsigned ray;  // id within the species' stream
   };
-  __device__ __forceinline__ const BvhView& view(const Ray&) const { return bv; }
+  __device__ __forceinline__ const V& view(const Ray&) const { return bv; }
+  __device__ __forceinline__ unsigned id(const Ray& R) const { return R.sp ? R.ray + n0 : R.ray; }
+  __device__ __forceinline__ unsigned earlier(const Ray& R) const { return (unsigned)R.bounce; }
   __device__ __forceinline__ const Box& box(const Ray&) const { return b; }
   __device__ __forceinline__ void start(Ray& R, unsigned ray, Vec3& o, Emit& e) const {
     R.sp = ray >= n0;
@@ -452,10 +620,11 @@ struct NeutralRR {
     R.w = 1.f;
     R.bounce = 0;
   }
-  __device__ __forceinline__ bool hit(Ray& R, const Hit& h, Vec3& o, Vec3 d, Emit& e) const {
+  __device__ __forceinline__ bool hit(Ray& R, const Hit& h, Vec3& o, Vec3 d, Emit& e,
+                                      bool on) const {
     const float S = bare[h.face] * (R.sp ? beta[1] : beta[0]);
     return rr_bounce(R.w, R.bounce, R.sp ? seed[1] : seed[0], R.ray, bv, h,
-                     R.sp ? fl[1] : fl[0], fixed, S, o, d, e);
+                     R.sp ? fl[1] : fl[0], fixed, S, o, d, e, on);
   }
 };
 
@@ -467,9 +636,11 @@ struct NeutralRR {
 // above u * total, u a 53-bit uniform from words 0 and 1 of its block 0, and its lobe from
 // words 2 and 3. With nothing to emit (total <= 0) every ray carries weight 0 and deposits
 // nothing; the result is then zero.
+template <class V>
 struct Redep {
+  using View = V;
   static constexpr bool kReplay = false;
-  BvhView bv;
+  V bv;
   Box b;
   const float* __restrict__ cen;
   const float* __restrict__ gn;
@@ -484,7 +655,9 @@ struct Redep {
     int bounce;
     unsigned ray;
   };
-  __device__ __forceinline__ const BvhView& view(const Ray&) const { return bv; }
+  __device__ __forceinline__ const V& view(const Ray&) const { return bv; }
+  __device__ __forceinline__ unsigned id(const Ray& R) const { return R.ray; }
+  __device__ __forceinline__ unsigned earlier(const Ray& R) const { return (unsigned)R.bounce; }
   __device__ __forceinline__ const Box& box(const Ray&) const { return b; }
   __device__ __forceinline__ void start(Ray& R, unsigned ray, Vec3& o, Emit& e) const {
     uint32_t u[4];
@@ -511,8 +684,9 @@ struct Redep {
     R.bounce = 0;
     R.ray = ray;
   }
-  __device__ __forceinline__ bool hit(Ray& R, const Hit& h, Vec3& o, Vec3 d, Emit& e) const {
-    return rr_bounce(R.w, R.bounce, seed, R.ray, bv, h, fl, fixed, S, o, d, e);
+  __device__ __forceinline__ bool hit(Ray& R, const Hit& h, Vec3& o, Vec3 d, Emit& e,
+                                      bool on) const {
+    return rr_bounce(R.w, R.bounce, seed, R.ray, bv, h, fl, fixed, S, o, d, e, on);
   }
 };
 
@@ -521,9 +695,11 @@ struct Redep {
 // block against S) and stops at the latest after n_reemit re-emissions; otherwise cosine
 // re-emission as in the RR walk. The reference launches it with no boundary handling, so the
 // box never wraps. Streams as NeutralRR's: source from block 0, bounce k from block (k, ray, 1).
+template <class V>
 struct NeutralCap {
+  using View = V;
   static constexpr bool kReplay = false;
-  BvhView bv;
+  V bv;
   Box b;
   Source src;
   const float* __restrict__ bare;
@@ -536,17 +712,20 @@ struct NeutralCap {
     int bounce;
     unsigned ray;
   };
-  __device__ __forceinline__ const BvhView& view(const Ray&) const { return bv; }
+  __device__ __forceinline__ const V& view(const Ray&) const { return bv; }
+  __device__ __forceinline__ unsigned id(const Ray& R) const { return R.ray; }
+  __device__ __forceinline__ unsigned earlier(const Ray& R) const { return (unsigned)R.bounce; }
   __device__ __forceinline__ const Box& box(const Ray&) const { return b; }
   __device__ __forceinline__ void start(Ray& R, unsigned ray, Vec3& o, Emit& e) const {
     neutral_source(seed, ray, b, src, o, e);
     R.bounce = 0;
     R.ray = ray;
   }
-  __device__ __forceinline__ bool hit(Ray& R, const Hit& h, Vec3& o, Vec3 d, Emit& e) const {
+  __device__ __forceinline__ bool hit(Ray& R, const Hit& h, Vec3& o, Vec3 d, Emit& e,
+                                      bool on) const {
     Vec3 nn = hit_normal(bv, h.slot);
     if (petch::dot(nn, d) > 0.f) nn = -nn;
-    deposit(fl, h.face, 1.f, fixed);
+    deposit(fl, h.face, 1.f, fixed, on);
     uint32_t u[4];
     petch::philox_block(seed, R.ray, (uint32_t)R.bounce + 1u, 1u, u);
     if (petch::u24(u[0]) < bare[h.face] * beta || R.bounce >= n_reemit) return false;
@@ -589,9 +768,11 @@ __device__ __forceinline__ int* seg_buf() {
 // Like the trace, one launch can carry the two species of a fixed-point iteration: queue ids
 // [0, n0) are species 0, the rest species 1 with ids from n0, each with its own beta, stream
 // and gfl; both add into the one gbare.
+template <class V>
 struct NeutralRRAdjoint {
+  using View = V;
   static constexpr bool kReplay = true;
-  BvhView bv;
+  V bv;
   Box b;
   Source src;
   const float* __restrict__ bare;
@@ -611,7 +792,10 @@ struct NeutralRRAdjoint {
     Vec3 o0;
     Emit e0;
   };
-  __device__ __forceinline__ const BvhView& view(const Ray&) const { return bv; }
+  __device__ __forceinline__ const V& view(const Ray&) const { return bv; }
+  __device__ __forceinline__ unsigned id(const Ray& R) const { return R.sp ? R.ray + n0 : R.ray; }
+  // a tie comes up in phase 0, before the ray's first deposit
+  __device__ __forceinline__ unsigned earlier(const Ray&) const { return 0u; }
   __device__ __forceinline__ const Box& box(const Ray&) const { return b; }
   __device__ __forceinline__ static void begin_path(Ray& R, const Vec3& o, const Emit& e) {
     R.o0 = o;
@@ -659,7 +843,8 @@ struct NeutralRRAdjoint {
     R.bounce = 0;
     begin_path(R, o, e);
   }
-  __device__ __forceinline__ bool hit(Ray& R, const Hit& h, Vec3& o, Vec3 d, Emit& e) const {
+  __device__ __forceinline__ bool hit(Ray& R, const Hit& h, Vec3& o, Vec3 d, Emit& e,
+                                      bool on) const {
     Vec3 nn = hit_normal(bv, h.slot);
     if (petch::dot(nn, d) > 0.f) nn = -nn;
     const int i = R.bounce;
@@ -719,10 +904,10 @@ struct IonParams {
 // specular direction (returns true with the next ray in o, d). The constants come from F:
 // F.P (IonParams), F.sE (square roots of the three threshold energies) and F.out (sp, ie, ip,
 // arr, ang accumulators).
-template <class Fc>
+template <class Fc, class V>
 __device__ __forceinline__ bool ion_bounce(Rng& r, float& Ein, float& win, int& bounce,
-                                           const BvhView& bv, const Hit& h, const Fc& F, Vec3& o,
-                                           Vec3& d, float E0 = 0.f) {
+                                           const V& bv, const Hit& h, const Fc& F, Vec3& o,
+                                           Vec3& d, bool on, float E0 = 0.f) {
   const IonParams& P = F.P;
   Vec3 nn = hit_normal(bv, h.slot);
   if (petch::dot(nn, d) > 0.f) nn = -nn;
@@ -739,15 +924,15 @@ __device__ __forceinline__ bool ion_bounce(Rng& r, float& Ein, float& win, int& 
     // dE / dE0 = E / E0 along the path, and dE0 / dmeanE = 1 (0 where E0 was clamped to 0,
     // where sqrtE = 0 deposits nothing).
     const float s = w * sqrtE / (2.f * E0);
-    deposit(F.out[0], h.face, sqrtE > F.sE[0] ? P.A_sp * f_sp * s : 0.f);
-    deposit(F.out[1], h.face, sqrtE > F.sE[1] ? P.A_ie * f_ie * s : 0.f);
-    deposit(F.out[2], h.face, sqrtE > F.sE[2] ? P.A_p * f_ie * s : 0.f);
+    deposit(F.out[0], h.face, sqrtE > F.sE[0] ? P.A_sp * f_sp * s : 0.f, 0, on);
+    deposit(F.out[1], h.face, sqrtE > F.sE[1] ? P.A_ie * f_ie * s : 0.f, 0, on);
+    deposit(F.out[2], h.face, sqrtE > F.sE[2] ? P.A_p * f_ie * s : 0.f, 0, on);
   } else {
-    deposit(F.out[0], h.face, P.A_sp * fmaxf(sqrtE - F.sE[0], 0.f) * f_sp * w, F.fixed);
-    deposit(F.out[1], h.face, P.A_ie * fmaxf(sqrtE - F.sE[1], 0.f) * f_ie * w, F.fixed);
-    deposit(F.out[2], h.face, P.A_p * fmaxf(sqrtE - F.sE[2], 0.f) * f_ie * w, F.fixed);
-    deposit(F.out[3], h.face, w, F.fixed);
-    deposit(F.out[4], h.face, cosT * w, F.fixed);
+    deposit(F.out[0], h.face, P.A_sp * fmaxf(sqrtE - F.sE[0], 0.f) * f_sp * w, F.fixed, on);
+    deposit(F.out[1], h.face, P.A_ie * fmaxf(sqrtE - F.sE[1], 0.f) * f_ie * w, F.fixed, on);
+    deposit(F.out[2], h.face, P.A_p * fmaxf(sqrtE - F.sE[2], 0.f) * f_ie * w, F.fixed, on);
+    deposit(F.out[3], h.face, w, F.fixed, on);
+    deposit(F.out[4], h.face, cosT * w, F.fixed, on);
   }
   float stick = 1.f;
   if (incAng > P.thrmin) {
@@ -804,10 +989,12 @@ __device__ __forceinline__ bool ion_bounce(Rng& r, float& Ein, float& win, int& 
   return true;
 }
 
+template <class V>
 struct IonYield {
+  using View = V;
   static constexpr bool kReplay = false;
   static constexpr bool kTangent = false;
-  BvhView bv;
+  V bv;
   Box b;
   Source src;
   IonParams P;
@@ -820,7 +1007,9 @@ struct IonYield {
     int bounce;
     Rng rng;
   };
-  __device__ __forceinline__ const BvhView& view(const Ray&) const { return bv; }
+  __device__ __forceinline__ const V& view(const Ray&) const { return bv; }
+  __device__ __forceinline__ unsigned id(const Ray& R) const { return R.rng.ray; }
+  __device__ __forceinline__ unsigned earlier(const Ray& R) const { return (unsigned)R.bounce; }
   __device__ __forceinline__ const Box& box(const Ray&) const { return b; }
   __device__ __forceinline__ void start(Ray& R, unsigned ray, Vec3& o, Emit& e) const {
     R.rng.init(seed, ray);
@@ -831,10 +1020,11 @@ struct IonYield {
     R.w = 1.f;
     R.bounce = 0;
   }
-  __device__ __forceinline__ bool hit(Ray& R, const Hit& h, Vec3& o, Vec3 d, Emit& e) const {
+  __device__ __forceinline__ bool hit(Ray& R, const Hit& h, Vec3& o, Vec3 d, Emit& e,
+                                      bool on) const {
     e.mode = kDirect;
     e.n = d;
-    return ion_bounce(R.rng, R.E, R.w, R.bounce, bv, h, *this, o, e.n);
+    return ion_bounce(R.rng, R.E, R.w, R.bounce, bv, h, *this, o, e.n, on);
   }
 };
 
@@ -842,10 +1032,12 @@ struct IonYield {
 // counterpart): the same rays, energies, decisions and paths as IonYield with the same seed;
 // out[0..2] receive d (sp, ie, ip) / d meanE per face. The arrival weight and the cosine
 // channel do not depend on the energy.
+template <class V>
 struct IonYieldTangent {
+  using View = V;
   static constexpr bool kReplay = false;
   static constexpr bool kTangent = true;
-  BvhView bv;
+  V bv;
   Box b;
   Source src;
   IonParams P;
@@ -857,7 +1049,9 @@ struct IonYieldTangent {
     int bounce;
     Rng rng;
   };
-  __device__ __forceinline__ const BvhView& view(const Ray&) const { return bv; }
+  __device__ __forceinline__ const V& view(const Ray&) const { return bv; }
+  __device__ __forceinline__ unsigned id(const Ray& R) const { return R.rng.ray; }
+  __device__ __forceinline__ unsigned earlier(const Ray& R) const { return (unsigned)R.bounce; }
   __device__ __forceinline__ const Box& box(const Ray&) const { return b; }
   __device__ __forceinline__ void start(Ray& R, unsigned ray, Vec3& o, Emit& e) const {
     R.rng.init(seed, ray);
@@ -869,10 +1063,11 @@ struct IonYieldTangent {
     R.w = 1.f;
     R.bounce = 0;
   }
-  __device__ __forceinline__ bool hit(Ray& R, const Hit& h, Vec3& o, Vec3 d, Emit& e) const {
+  __device__ __forceinline__ bool hit(Ray& R, const Hit& h, Vec3& o, Vec3 d, Emit& e,
+                                      bool on) const {
     e.mode = kDirect;
     e.n = d;
-    return ion_bounce(R.rng, R.E, R.w, R.bounce, bv, h, *this, o, e.n, R.E0);
+    return ion_bounce(R.rng, R.E, R.w, R.bounce, bv, h, *this, o, e.n, on, R.E0);
   }
 };
 
@@ -883,6 +1078,7 @@ struct IonYieldTangent {
 // the feature's descriptor (a few hundred bytes, cache resident).
 struct NeutralFeature {
   BvhView bv;
+  GridView gv;  // read when every feature of the launch has a grid
   Box b;
   const float* bare;
   float beta[2];
@@ -897,6 +1093,7 @@ struct NeutralFeature {
 struct IonFeature {
   static constexpr bool kTangent = false;
   BvhView bv;
+  GridView gv;  // read when every feature of the launch has a grid
   Box b;
   Source src;
   IonParams P;
@@ -907,6 +1104,12 @@ struct IonFeature {
   int fixed;      // out are int64 fixed-point accumulators (deterministic mode)
   float* dst[5];  // with fixed: the float outputs the accumulators are converted into
 };
+
+template <class V, class Fd>
+__device__ __forceinline__ const V& feature_view(const Fd& F) {
+  if constexpr (std::is_same<V, GridView>::value) return F.gv;
+  else return F.bv;
+}
 
 // first feature whose id range ends after `ray`
 template <class Fd>
@@ -920,7 +1123,9 @@ __device__ __forceinline__ int locate_feature(const Fd* __restrict__ feat, int n
   return lo;
 }
 
+template <class V>
 struct NeutralRRBatch {
+  using View = V;
   static constexpr bool kReplay = false;
   const NeutralFeature* __restrict__ feat;
   int nfeat;
@@ -931,10 +1136,14 @@ struct NeutralRRBatch {
     int sp;
     int f;
     unsigned ray;  // id within the species' stream
-    BvhView bv;
+    V bv;
     Box b;
   };
-  __device__ __forceinline__ const BvhView& view(const Ray& R) const { return R.bv; }
+  __device__ __forceinline__ const V& view(const Ray& R) const { return R.bv; }
+  __device__ __forceinline__ unsigned id(const Ray& R) const {
+    return (R.f ? feat[R.f - 1].end : 0u) + (R.sp ? feat[R.f].n0 : 0u) + R.ray;
+  }
+  __device__ __forceinline__ unsigned earlier(const Ray& R) const { return (unsigned)R.bounce; }
   __device__ __forceinline__ const Box& box(const Ray& R) const { return R.b; }
   __device__ __forceinline__ void start(Ray& R, unsigned ray, Vec3& o, Emit& e) const {
     R.f = locate_feature(feat, nfeat, ray);
@@ -942,21 +1151,24 @@ struct NeutralRRBatch {
     const unsigned local = ray - (R.f ? feat[R.f - 1].end : 0u);
     R.sp = local >= F.n0;
     R.ray = R.sp ? local - F.n0 : local;
-    R.bv = F.bv;
+    R.bv = feature_view<V>(F);
     R.b = F.b;
     neutral_source(R.sp ? F.seed[1] : F.seed[0], R.ray, R.b, src, o, e);
     R.w = 1.f;
     R.bounce = 0;
   }
-  __device__ __forceinline__ bool hit(Ray& R, const Hit& h, Vec3& o, Vec3 d, Emit& e) const {
+  __device__ __forceinline__ bool hit(Ray& R, const Hit& h, Vec3& o, Vec3 d, Emit& e,
+                                      bool on) const {
     const NeutralFeature& F = feat[R.f];
     const float S = F.bare[h.face] * (R.sp ? F.beta[1] : F.beta[0]);
     return rr_bounce(R.w, R.bounce, R.sp ? F.seed[1] : F.seed[0], R.ray, R.bv, h,
-                     R.sp ? F.fl[1] : F.fl[0], F.fixed, S, o, d, e);
+                     R.sp ? F.fl[1] : F.fl[0], F.fixed, S, o, d, e, on);
   }
 };
 
+template <class V>
 struct IonYieldBatch {
+  using View = V;
   static constexpr bool kReplay = false;
   const IonFeature* __restrict__ feat;
   int nfeat;
@@ -965,16 +1177,20 @@ struct IonYieldBatch {
     int bounce;
     int f;
     Rng rng;
-    BvhView bv;
+    V bv;
     Box b;
   };
-  __device__ __forceinline__ const BvhView& view(const Ray& R) const { return R.bv; }
+  __device__ __forceinline__ const V& view(const Ray& R) const { return R.bv; }
+  __device__ __forceinline__ unsigned id(const Ray& R) const {
+    return (R.f ? feat[R.f - 1].end : 0u) + R.rng.ray;
+  }
+  __device__ __forceinline__ unsigned earlier(const Ray& R) const { return (unsigned)R.bounce; }
   __device__ __forceinline__ const Box& box(const Ray& R) const { return R.b; }
   __device__ __forceinline__ void start(Ray& R, unsigned ray, Vec3& o, Emit& e) const {
     R.f = locate_feature(feat, nfeat, ray);
     const IonFeature& F = feat[R.f];
     R.rng.init(F.seed, ray - (R.f ? feat[R.f - 1].end : 0u));
-    R.bv = F.bv;
+    R.bv = feature_view<V>(F);
     R.b = F.b;
     gen_source(R.rng, R.b, F.src, o, e.n);
     e.mode = kDirect;
@@ -983,10 +1199,11 @@ struct IonYieldBatch {
     R.w = 1.f;
     R.bounce = 0;
   }
-  __device__ __forceinline__ bool hit(Ray& R, const Hit& h, Vec3& o, Vec3 d, Emit& e) const {
+  __device__ __forceinline__ bool hit(Ray& R, const Hit& h, Vec3& o, Vec3 d, Emit& e,
+                                      bool on) const {
     e.mode = kDirect;
     e.n = d;
-    return ion_bounce(R.rng, R.E, R.w, R.bounce, R.bv, h, feat[R.f], o, e.n);
+    return ion_bounce(R.rng, R.E, R.w, R.bounce, R.bv, h, feat[R.f], o, e.n, on);
   }
 };
 
@@ -1038,46 +1255,59 @@ __global__ void k_fix_finish_ion_batch(const IonFeature* __restrict__ feat) {
       F.dst[k][i] = fix_to_float(((const unsigned long long*)F.out[k])[i]);
 }
 
-// The neutral loop fits 96 registers without spills, which gives 5 waves per SIMD; the ion
+// The neutral tree loop fits 96 registers without spills, which gives 5 waves per SIMD; the ion
 // loop needs more and runs best at the compiler's own choice (4 waves per SIMD), measured.
+template <class P>
 __global__ void __launch_bounds__(kBS) __attribute__((amdgpu_waves_per_eu(5)))
-k_trace_neutral_rr(NeutralRR pol, RayQueue q, unsigned long long* __restrict__ hits) {
-  persistent_trace(pol, q, hits);
+k_trace5(P pol, RayQueue q, unsigned long long* __restrict__ hits) {
+  run_trace(pol, q, hits);
 }
 
+template <class P>
 __global__ void __launch_bounds__(kBS)
-k_trace_neutral_rr_adjoint(NeutralRRAdjoint pol, RayQueue q, unsigned long long* __restrict__ hits) {
-  persistent_trace(pol, q, hits);
+k_trace(P pol, RayQueue q, unsigned long long* __restrict__ hits) {
+  run_trace(pol, q, hits);
 }
 
+// The rays that a walk trace left to the tree, from their sources again: the same path up to the
+// tie, whose earlier hits are not deposited a second time. A handful per launch at most, so each
+// lane runs its ray to the end.
+template <class P>
 __global__ void __launch_bounds__(kBS)
-k_trace_ion_yield(IonYield pol, RayQueue q, unsigned long long* __restrict__ hits) {
-  persistent_trace(pol, q, hits);
-}
-
-__global__ void __launch_bounds__(kBS)
-k_trace_ion_yield_tangent(IonYieldTangent pol, RayQueue q, unsigned long long* __restrict__ hits) {
-  persistent_trace(pol, q, hits);
-}
-
-__global__ void __launch_bounds__(kBS)
-k_trace_neutral_rr_batch(NeutralRRBatch pol, RayQueue q, unsigned long long* __restrict__ hits) {
-  persistent_trace(pol, q, hits);
-}
-
-__global__ void __launch_bounds__(kBS)
-k_trace_ion_yield_batch(IonYieldBatch pol, RayQueue q, unsigned long long* __restrict__ hits) {
-  persistent_trace(pol, q, hits);
-}
-
-__global__ void __launch_bounds__(kBS) __attribute__((amdgpu_waves_per_eu(5)))
-k_trace_redep(Redep pol, RayQueue q, unsigned long long* __restrict__ hits) {
-  persistent_trace(pol, q, hits);
-}
-
-__global__ void __launch_bounds__(kBS) __attribute__((amdgpu_waves_per_eu(5)))
-k_trace_neutral_cap(NeutralCap pol, RayQueue q, unsigned long long* __restrict__ hits) {
-  persistent_trace(pol, q, hits);
+k_trace_ties(P pol, RayQueue q, unsigned long long* __restrict__ hits) {
+  const unsigned n = min(*q.n_ties, kMaxTies);
+  unsigned nh = 0;
+  for (unsigned i = blockIdx.x * kBS + threadIdx.x; i < n; i += gridDim.x * kBS) {
+    typename P::Ray R;
+    Emit e;
+    Vec3 o;
+    pol.start(R, q.ties[i].x, o, e);
+    unsigned muted = q.ties[i].y;
+    bool go = true;
+    while (go) {
+      const Vec3 d = emit_dir(e);
+      const BvhView& bv = pol.view(R);
+      const Box& b = pol.box(R);
+      petch::RayPre rp = petch::ray_pre(o, d);
+      petch::ScratchStack stk;
+      Hit h = petch::bvh_closest_hit(bv, rp, 1.0e6f, stk);
+      for (int w = 0; h.face < 0 && b.periodic && w < kMaxWraps && !never_returns(bv, o, d) &&
+                      wrap_ray(b, o, d, rp.inv);
+           ++w) {
+        petch::ray_move(rp, o);
+        h = petch::bvh_closest_hit(bv, rp, 1.0e6f, stk);
+      }
+      if (h.face >= 0) {
+        const bool on = muted == 0;
+        if (on) ++nh; else --muted;
+        go = pol.hit(R, h, o, d, e, on);
+      } else {
+        go = false;
+        if constexpr (P::kReplay) go = pol.miss(R, o, e);
+      }
+    }
+  }
+  count_hits(hits, nh);
 }
 
 // Emission weight of a face for redeposition: max(rate * area, 0), a non-finite product as 0.
@@ -1206,18 +1436,14 @@ __global__ void __launch_bounds__(kBS) k_trace_legacy(BvhView bv, Source src, Bo
   }
 }
 
-// n_ff cosine rays per face from centroid + 1e-3 n (threed.py:949-955); hit face or -1.
-__global__ void __launch_bounds__(kBS) k_trace_ff(BvhView bv, Box b,
-                                                  const float* __restrict__ cen,
-                                                  const float* __restrict__ gn, int nf, int n_ff,
-                                                  uint64_t seed, int* __restrict__ hitface) {
-  long long p = (long long)blockIdx.x * kBS + threadIdx.x;
-  if (p >= (long long)nf * n_ff) return;
-  int j = (int)(p / n_ff);
+// n_ff cosine rays per face from centroid + 1e-3 n (threed.py:949-955).
+__device__ __forceinline__ void ff_ray(const float* __restrict__ cen, const float* __restrict__ gn,
+                                       int n_ff, uint64_t seed, unsigned p, Vec3& o, Vec3& d) {
+  int j = (int)(p / (unsigned)n_ff);
   Rng r;
-  r.init(seed, (uint32_t)p);
+  r.init(seed, p);
   Vec3 nn = v3(gn[3 * j], gn[3 * j + 1], gn[3 * j + 2]);
-  Vec3 o = v3(cen[3 * j], cen[3 * j + 1], cen[3 * j + 2]) + 1.0e-3f * nn;
+  o = v3(cen[3 * j], cen[3 * j + 1], cen[3 * j + 2]) + 1.0e-3f * nn;
   // _cosine_dirs (threed.py:1571-1579): t = cross(a, n) / (|cross(a, n)| + 1e-12)
   Vec3 a = (fabsf(nn.x) > 0.9f) ? v3(0.f, 1.f, 0.f) : v3(1.f, 0.f, 0.f);
   Vec3 c = petch::cross(a, nn);
@@ -1225,10 +1451,55 @@ __global__ void __launch_bounds__(kBS) k_trace_ff(BvhView bv, Box b,
   Vec3 bb = petch::cross(nn, t);
   float u1 = r.uniform(), u2 = r.uniform();
   float ct = sqrtf(u1), st = sqrtf(1.f - u1), ph = kTwoPi * u2;
-  Vec3 d = (st * cosf(ph)) * t + (st * sinf(ph)) * bb + ct * nn;
+  d = (st * cosf(ph)) * t + (st * sinf(ph)) * bb + ct * nn;
+}
+
+// First hit of every form-factor ray, -1 for one that escapes, over a surface's tree.
+__global__ void __launch_bounds__(kBS) k_trace_ff(BvhView bv, Box b,
+                                                  const float* __restrict__ cen,
+                                                  const float* __restrict__ gn, int nf, int n_ff,
+                                                  uint64_t seed, int* __restrict__ hitface) {
+  long long p = (long long)blockIdx.x * kBS + threadIdx.x;
+  if (p >= (long long)nf * n_ff) return;
+  Vec3 o, d;
+  ff_ray(cen, gn, n_ff, seed, (unsigned)p, o, d);
   Hit h = trace_bc(bv, b, o, d);
   hitface[p] = h.face;
 }
+
+// The same rays in the walk loop.
+template <class V>
+struct FormFactor {
+  static constexpr bool kReplay = true;  // a ray that leaves is recorded by miss()
+  using View = V;
+  V bv;
+  Box b;
+  const float* __restrict__ cen;
+  const float* __restrict__ gn;
+  int n_ff;
+  uint64_t seed;
+  int* __restrict__ hitface;
+  struct Ray {
+    unsigned ray;
+  };
+  __device__ __forceinline__ const V& view(const Ray&) const { return bv; }
+  __device__ __forceinline__ unsigned id(const Ray& R) const { return R.ray; }
+  __device__ __forceinline__ unsigned earlier(const Ray&) const { return 0u; }
+  __device__ __forceinline__ const Box& box(const Ray&) const { return b; }
+  __device__ __forceinline__ void start(Ray& R, unsigned ray, Vec3& o, Emit& e) const {
+    R.ray = ray;
+    ff_ray(cen, gn, n_ff, seed, ray, o, e.n);
+    e.mode = kDirect;
+  }
+  __device__ __forceinline__ bool hit(Ray& R, const Hit& h, Vec3&, Vec3, Emit&, bool) const {
+    hitface[R.ray] = h.face;
+    return false;
+  }
+  __device__ __forceinline__ bool miss(Ray& R, Vec3&, Emit&) const {
+    hitface[R.ray] = -1;
+    return false;
+  }
+};
 
 __global__ void k_gen_source(Box b, Source src, int n, uint64_t seed, float* __restrict__ origin,
                              float* __restrict__ dir) {
@@ -1275,8 +1546,72 @@ int make_queue(petch_ctx* ctx, int n, RayQueue& q) {
   if (!c) return PETCH_E_HIP;
   q.next = (unsigned*)c;
   q.n = n;
-  PETCH_HIP(ctx, hipMemsetAsync(q.next, 0, sizeof(unsigned), ctx->stream));
+  q.n_ties = (unsigned*)(c + 1);
+  q.ties = (uint2*)(c + 2);
+  PETCH_HIP(ctx, hipMemsetAsync(q.next, 0, 2 * sizeof(unsigned long long), ctx->stream));
   return PETCH_OK;
+}
+
+// The grid of a walk trace and its wavefronts' shares of the rays.
+unsigned walk_share(petch_ctx* ctx, const void* kernel, RayQueue& q) {
+  const unsigned all = persistent_blocks(ctx, kernel, 0x7fffffff);
+  const long long waves = (long long)all * (kBS / 64);
+  const int per = (int)((q.n + waves - 1) / waves);
+  q.lanes = per < kMinLanes ? kMinLanes : (per < 64 ? per : 64);
+  q.chunk = per < 64 ? q.lanes : (per < 512 ? 64 : (int)kRayChunk);
+  q.refill_at = q.lanes * kRefillAt / 64;
+  const long long need = ((long long)q.n + q.lanes * (kBS / 64) - 1) / (q.lanes * (kBS / 64));
+  return (unsigned)(need < all ? need : all);
+}
+
+// Launches a persistent trace of n rays over the surface's tree, by the kernel K (k_trace or
+// k_trace5).
+template <class P>
+int launch_tree(petch_ctx* ctx, void (*kernel)(P, RayQueue, unsigned long long*), const P& pol,
+                int n, unsigned long long* hits) {
+  RayQueue q;
+  const int rc = make_queue(ctx, n, q);
+  if (rc) return rc;
+  const unsigned grid = persistent_blocks(ctx, (const void*)kernel, n);
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(kBS), 0, ctx->stream, pol, q, hits);
+  PETCH_LAUNCH_CHECK(ctx);
+  return PETCH_OK;
+}
+
+// Launches a persistent trace of n rays by walking the surface's grid, then the rays it left to
+// the tree.
+template <class P, class PTree>
+int launch_walk(petch_ctx* ctx, void (*kernel)(P, RayQueue, unsigned long long*), const P& pol,
+                const PTree& tree, int n, unsigned long long* hits) {
+  RayQueue q;
+  const int rc = make_queue(ctx, n, q);
+  if (rc) return rc;
+  const unsigned grid = walk_share(ctx, (const void*)kernel, q);
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(kBS), 0, ctx->stream, pol, q, hits);
+  PETCH_LAUNCH_CHECK(ctx);
+  hipLaunchKernelGGL(k_trace_ties<PTree>, dim3(kTieBlocks), dim3(kBS), 0, ctx->stream, tree, q,
+                     hits);
+  PETCH_LAUNCH_CHECK(ctx);
+  return PETCH_OK;
+}
+
+// Traces n rays on the surface of bvh: by its grid where it has one, else by its tree.
+// make(view) gives the policy for either view; Five picks k_trace5.
+template <bool Five, class Make>
+int trace_surface(petch_ctx* ctx, const petch_bvh* bvh, Make make, int n,
+                  unsigned long long* hits) {
+  const auto tree = make(petch_bvh_view(bvh));
+  GridView g;
+  const bool grid = petch_grid_view(bvh, &g);
+  const auto walk = make(g);
+  using T = std::decay_t<decltype(tree)>;
+  using W = std::decay_t<decltype(walk)>;
+  if constexpr (Five)
+    return grid ? launch_walk(ctx, k_trace5<W>, walk, tree, n, hits)
+                : launch_tree(ctx, k_trace5<T>, tree, n, hits);
+  else
+    return grid ? launch_walk(ctx, k_trace<W>, walk, tree, n, hits)
+                : launch_tree(ctx, k_trace<T>, tree, n, hits);
 }
 
 int zero(petch_ctx* ctx, float* p, int n) {
@@ -1319,15 +1654,11 @@ extern "C" int petch_gen_source(petch_ctx* ctx, const petch_box* box, const petc
 
 namespace {
 
-int launch_neutral(petch_ctx* ctx, const NeutralRR& pol, int n) {
-  RayQueue q;
-  int rc = make_queue(ctx, n, q);
-  if (rc) return rc;
-  const unsigned grid = persistent_blocks(ctx, (const void*)k_trace_neutral_rr, n);
-  hipLaunchKernelGGL(k_trace_neutral_rr, dim3(grid), dim3(kBS), 0, ctx->stream, pol, q,
-                     petch_hit_counter(ctx, 0));
-  PETCH_LAUNCH_CHECK(ctx);
-  return PETCH_OK;
+int launch_neutral(petch_ctx* ctx, const petch_bvh* bvh, const NeutralRR<BvhView>& p, int n) {
+  return trace_surface<true>(ctx, bvh, [&](auto view) {
+    return NeutralRR<decltype(view)>{view, p.b, p.src, p.bare, {p.beta[0], p.beta[1]},
+                                     {p.fl[0], p.fl[1]}, {p.seed[0], p.seed[1]}, p.n0, p.fixed};
+  }, n, petch_hit_counter(ctx, 0));
 }
 
 }  // namespace
@@ -1340,14 +1671,14 @@ extern "C" int petch_trace_neutral_rr(petch_ctx* ctx, const petch_bvh* bvh, cons
   int rc = zero(ctx, fl, bvh->nf);
   if (rc) return rc;
   if (n == 0 || bvh->nf == 0) return PETCH_OK;
-  NeutralRR pol{petch_bvh_view(bvh), make_box(box), make_source(src), bare, {beta, beta},
+  NeutralRR<BvhView> pol{petch_bvh_view(bvh), make_box(box), make_source(src), bare, {beta, beta},
                 {fl, fl}, {seed, seed}, (unsigned)n};
-  if (!ctx->deterministic) return launch_neutral(ctx, pol, n);
+  if (!ctx->deterministic) return launch_neutral(ctx, bvh, pol, n);
   unsigned long long* q = det_accumulators(ctx, 1, bvh->nf);
   if (!q) return PETCH_E_HIP;
   pol.fl[0] = pol.fl[1] = (float*)q;
   pol.fixed = 1;
-  rc = launch_neutral(ctx, pol, n);
+  rc = launch_neutral(ctx, bvh, pol, n);
   if (rc) return rc;
   return det_finish(ctx, q, fl, bvh->nf);
 }
@@ -1364,21 +1695,16 @@ extern "C" int petch_trace_neutral_cap(petch_ctx* ctx, const petch_bvh* bvh,
   if (n == 0 || bvh->nf == 0) return PETCH_OK;
   Box b = make_box(box);
   b.periodic = 0;  // _trace3d_cov applies no boundary condition
-  NeutralCap pol{petch_bvh_view(bvh), b, make_source(src), bare, beta, n_reemit, fl, seed, 0};
   unsigned long long* q = nullptr;
   if (ctx->deterministic) {
     q = det_accumulators(ctx, 1, bvh->nf);
     if (!q) return PETCH_E_HIP;
-    pol.fl = (float*)q;
-    pol.fixed = 1;
   }
-  RayQueue rq;
-  rc = make_queue(ctx, n, rq);
+  rc = trace_surface<true>(ctx, bvh, [&](auto view) {
+    return NeutralCap<decltype(view)>{view, b, make_source(src), bare, beta, n_reemit,
+                                      q ? (float*)q : fl, seed, q ? 1 : 0};
+  }, n, petch_hit_counter(ctx, 0));
   if (rc) return rc;
-  const unsigned grid = persistent_blocks(ctx, (const void*)k_trace_neutral_cap, n);
-  hipLaunchKernelGGL(k_trace_neutral_cap, dim3(grid), dim3(kBS), 0, ctx->stream, pol, rq,
-                     petch_hit_counter(ctx, 0));
-  PETCH_LAUNCH_CHECK(ctx);
   return q ? det_finish(ctx, q, fl, bvh->nf) : PETCH_OK;
 }
 
@@ -1404,22 +1730,16 @@ extern "C" int petch_trace_redeposition(petch_ctx* ctx, const petch_bvh* bvh,
                      cum);
   PETCH_LAUNCH_CHECK(ctx);
   // open box: no lateral wrap (threed.py:1604 passes periodic = 0)
-  Redep pol{petch_bvh_view(bvh), Box{1.f, 1.f, 1.f, 1.f, 0}, centroids, gas_normals, cum, nf,
-            s_redep, out, seed, 0};
   unsigned long long* q = nullptr;
   if (ctx->deterministic) {
     q = det_accumulators(ctx, 1, nf);
     if (!q) return PETCH_E_HIP;
-    pol.fl = (float*)q;
-    pol.fixed = 1;
   }
-  RayQueue rq;
-  rc = make_queue(ctx, n, rq);
+  rc = trace_surface<true>(ctx, bvh, [&](auto view) {
+    return Redep<decltype(view)>{view, Box{1.f, 1.f, 1.f, 1.f, 0}, centroids, gas_normals, cum, nf,
+                                 s_redep, q ? (float*)q : out, seed, q ? 1 : 0};
+  }, n, nullptr);
   if (rc) return rc;
-  const unsigned grid = persistent_blocks(ctx, (const void*)k_trace_redep, n);
-  hipLaunchKernelGGL(k_trace_redep, dim3(grid), dim3(kBS), 0, ctx->stream, pol, rq,
-                     (unsigned long long*)nullptr);
-  PETCH_LAUNCH_CHECK(ctx);
   if (q) {
     rc = det_finish(ctx, q, out, nf);
     if (rc) return rc;
@@ -1432,15 +1752,13 @@ extern "C" int petch_trace_redeposition(petch_ctx* ctx, const petch_bvh* bvh,
 
 namespace {
 
-int launch_neutral_adjoint(petch_ctx* ctx, const NeutralRRAdjoint& pol, int n) {
-  RayQueue q;
-  int rc = make_queue(ctx, n, q);
-  if (rc) return rc;
-  const unsigned grid = persistent_blocks(ctx, (const void*)k_trace_neutral_rr_adjoint, n);
-  hipLaunchKernelGGL(k_trace_neutral_rr_adjoint, dim3(grid), dim3(kBS), 0, ctx->stream, pol, q,
-                     (unsigned long long*)nullptr);
-  PETCH_LAUNCH_CHECK(ctx);
-  return PETCH_OK;
+int launch_neutral_adjoint(petch_ctx* ctx, const petch_bvh* bvh,
+                           const NeutralRRAdjoint<BvhView>& p, int n) {
+  return trace_surface<false>(ctx, bvh, [&](auto view) {
+    return NeutralRRAdjoint<decltype(view)>{view, p.b, p.src, p.bare, {p.gfl_sp[0], p.gfl_sp[1]},
+                                            p.gbare, {p.beta_sp[0], p.beta_sp[1]},
+                                            {p.seed_sp[0], p.seed_sp[1]}, p.n0};
+  }, n, nullptr);
 }
 
 }  // namespace
@@ -1457,9 +1775,9 @@ extern "C" int petch_trace_neutral_rr_adjoint(petch_ctx* ctx, const petch_bvh* b
   int rc = zero(ctx, gbare, bvh->nf);
   if (rc) return rc;
   if (n == 0 || bvh->nf == 0) return PETCH_OK;
-  NeutralRRAdjoint pol{petch_bvh_view(bvh), make_box(box), make_source(src), bare, {gfl, gfl},
+  NeutralRRAdjoint<BvhView> pol{petch_bvh_view(bvh), make_box(box), make_source(src), bare, {gfl, gfl},
                        gbare, {beta, beta}, {seed, seed}, (unsigned)n};
-  return launch_neutral_adjoint(ctx, pol, n);
+  return launch_neutral_adjoint(ctx, bvh, pol, n);
 }
 
 extern "C" int petch_trace_neutral_rr_pair_adjoint(petch_ctx* ctx, const petch_bvh* bvh,
@@ -1479,9 +1797,9 @@ extern "C" int petch_trace_neutral_rr_pair_adjoint(petch_ctx* ctx, const petch_b
   if (rc) return rc;
   const int n = n_a + n_b;
   if (n == 0 || bvh->nf == 0) return PETCH_OK;
-  NeutralRRAdjoint pol{petch_bvh_view(bvh), make_box(box), make_source(src), bare, {gfl_a, gfl_b},
+  NeutralRRAdjoint<BvhView> pol{petch_bvh_view(bvh), make_box(box), make_source(src), bare, {gfl_a, gfl_b},
                        gbare, {beta_a, beta_b}, {seed_a, seed_b}, (unsigned)n_a};
-  return launch_neutral_adjoint(ctx, pol, n);
+  return launch_neutral_adjoint(ctx, bvh, pol, n);
 }
 
 extern "C" int petch_trace_neutral_rr_pair(petch_ctx* ctx, const petch_bvh* bvh,
@@ -1501,16 +1819,16 @@ extern "C" int petch_trace_neutral_rr_pair(petch_ctx* ctx, const petch_bvh* bvh,
   if (rc) return rc;
   const int n = n_a + n_b;
   if (n == 0 || bvh->nf == 0) return PETCH_OK;
-  NeutralRR pol{petch_bvh_view(bvh), make_box(box), make_source(src), bare, {beta_a, beta_b},
+  NeutralRR<BvhView> pol{petch_bvh_view(bvh), make_box(box), make_source(src), bare, {beta_a, beta_b},
                 {fl_a, fl_b}, {seed_a, seed_b}, (unsigned)n_a};
-  if (!ctx->deterministic) return launch_neutral(ctx, pol, n);
+  if (!ctx->deterministic) return launch_neutral(ctx, bvh, pol, n);
   const int nf = bvh->nf;
   unsigned long long* q = det_accumulators(ctx, 2, nf);
   if (!q) return PETCH_E_HIP;
   pol.fl[0] = (float*)q;
   pol.fl[1] = (float*)(q + nf);
   pol.fixed = 1;
-  rc = launch_neutral(ctx, pol, n);
+  rc = launch_neutral(ctx, bvh, pol, n);
   if (!rc) rc = det_finish(ctx, q, fl_a, nf);
   if (!rc) rc = det_finish(ctx, q + nf, fl_b, nf);
   return rc;
@@ -1532,16 +1850,11 @@ extern "C" int petch_trace_ion_yield_tangent(petch_ctx* ctx, const petch_bvh* bv
   IonParams P{ip->meanE,  ip->sigmaE, ip->A_sp,    ip->Eth_sp, ip->B_sp, ip->A_ie,
               ip->Eth_ie, ip->A_p,    ip->Eth_p,   ip->inflect, ip->minang, ip->n_l,
               ip->A_en,   ip->minE,   ip->thrmin,  ip->thrmax};
-  RayQueue q;
-  int rc2 = make_queue(ctx, n, q);
-  if (rc2) return rc2;
-  IonYieldTangent pol{petch_bvh_view(bvh), make_box(box), make_source(src), P,
-                      {sqrtf(P.Eth_sp), sqrtf(P.Eth_ie), sqrtf(P.Eth_p)}, {dsp, die, dip}, seed};
-  const unsigned grid = persistent_blocks(ctx, (const void*)k_trace_ion_yield_tangent, n);
-  hipLaunchKernelGGL(k_trace_ion_yield_tangent, dim3(grid), dim3(kBS), 0, ctx->stream, pol, q,
-                     (unsigned long long*)nullptr);
-  PETCH_LAUNCH_CHECK(ctx);
-  return PETCH_OK;
+  return trace_surface<false>(ctx, bvh, [&](auto view) {
+    return IonYieldTangent<decltype(view)>{view, make_box(box), make_source(src), P,
+                                           {sqrtf(P.Eth_sp), sqrtf(P.Eth_ie), sqrtf(P.Eth_p)},
+                                           {dsp, die, dip}, seed};
+  }, n, nullptr);
 }
 
 extern "C" int petch_trace_ion_yield(petch_ctx* ctx, const petch_bvh* bvh, const petch_box* box,
@@ -1560,24 +1873,20 @@ extern "C" int petch_trace_ion_yield(petch_ctx* ctx, const petch_bvh* bvh, const
   IonParams P{ip->meanE,  ip->sigmaE, ip->A_sp,    ip->Eth_sp, ip->B_sp, ip->A_ie,
               ip->Eth_ie, ip->A_p,    ip->Eth_p,   ip->inflect, ip->minang, ip->n_l,
               ip->A_en,   ip->minE,   ip->thrmin,  ip->thrmax};
-  RayQueue q;
-  int rc2 = make_queue(ctx, n, q);
-  if (rc2) return rc2;
-  IonYield pol{petch_bvh_view(bvh), make_box(box), make_source(src), P,
-               {sqrtf(P.Eth_sp), sqrtf(P.Eth_ie), sqrtf(P.Eth_p)}, {sp, ie, ipass, arr, ang},
-               seed};
   const int nf = bvh->nf;
   unsigned long long* acc = nullptr;
+  float* dep[5] = {sp, ie, ipass, arr, ang};
   if (ctx->deterministic) {
     acc = det_accumulators(ctx, 5, nf);
     if (!acc) return PETCH_E_HIP;
-    for (int k = 0; k < 5; ++k) pol.out[k] = (float*)(acc + (size_t)k * nf);
-    pol.fixed = 1;
+    for (int k = 0; k < 5; ++k) dep[k] = (float*)(acc + (size_t)k * nf);
   }
-  const unsigned grid = persistent_blocks(ctx, (const void*)k_trace_ion_yield, n);
-  hipLaunchKernelGGL(k_trace_ion_yield, dim3(grid), dim3(kBS), 0, ctx->stream, pol, q,
-                     petch_hit_counter(ctx, 1));
-  PETCH_LAUNCH_CHECK(ctx);
+  const int rc2 = trace_surface<false>(ctx, bvh, [&](auto view) {
+    return IonYield<decltype(view)>{view, make_box(box), make_source(src), P,
+                                    {sqrtf(P.Eth_sp), sqrtf(P.Eth_ie), sqrtf(P.Eth_p)},
+                                    {dep[0], dep[1], dep[2], dep[3], dep[4]}, seed, acc ? 1 : 0};
+  }, n, petch_hit_counter(ctx, 1));
+  if (rc2) return rc2;
   if (acc)
     for (int k = 0; k < 5; ++k) {
       const int rc3 = det_finish(ctx, acc + (size_t)k * nf, outs[k], nf);
@@ -1594,6 +1903,7 @@ extern "C" int petch_trace_neutral_rr_batch(petch_ctx* ctx, const petch_source* 
   std::vector<NeutralFeature> t(nfeat);
   long long end = 0;
   int max_nf = 0;
+  bool grids = true;  // every surface has a grid
   for (int f = 0; f < nfeat; ++f) {
     const petch_neutral_feature& a = feats[f];
     PETCH_ARG(ctx, a.bvh, "trace_neutral_rr_batch: feature %d has no BVH", f);
@@ -1605,6 +1915,7 @@ extern "C" int petch_trace_neutral_rr_batch(petch_ctx* ctx, const petch_source* 
     PETCH_ARG(ctx, a.n_a >= 0 && a.n_b >= 0, "trace_neutral_rr_batch: feature %d: n < 0", f);
     NeutralFeature& d = t[f];
     d.bv = petch_bvh_view(a.bvh);
+    if (a.bvh->nf > 0) grids = petch_grid_view(a.bvh, &d.gv) && grids;
     d.b = make_box(&a.box);
     d.bare = a.bare;
     d.beta[0] = a.beta_a;
@@ -1646,15 +1957,13 @@ extern "C" int petch_trace_neutral_rr_batch(petch_ctx* ctx, const petch_source* 
     PETCH_LAUNCH_CHECK(ctx);
   }
   if (end > 0) {
-    RayQueue q;
-    int rc = make_queue(ctx, (int)end, q);
+    const NeutralRRBatch<BvhView> tree{dev, nfeat, make_source(src)};
+    const int rc = grids ? launch_walk(ctx, k_trace<NeutralRRBatch<GridView>>,
+                                       NeutralRRBatch<GridView>{dev, nfeat, make_source(src)}, tree, (int)end,
+                                       petch_hit_counter(ctx, 0))
+                         : launch_tree(ctx, k_trace<NeutralRRBatch<BvhView>>, tree, (int)end,
+                                       petch_hit_counter(ctx, 0));
     if (rc) return rc;
-    NeutralRRBatch pol{dev, nfeat, make_source(src)};
-    const unsigned grid =
-        persistent_blocks(ctx, (const void*)k_trace_neutral_rr_batch, (int)end);
-    hipLaunchKernelGGL(k_trace_neutral_rr_batch, dim3(grid), dim3(kBS), 0, ctx->stream, pol, q,
-                       petch_hit_counter(ctx, 0));
-    PETCH_LAUNCH_CHECK(ctx);
   }
   if (max_nf > 0 && ctx->deterministic) {
     hipLaunchKernelGGL(k_fix_finish_neutral_batch, dim3(gx, nfeat), dim3(kBS), 0, ctx->stream,
@@ -1672,6 +1981,7 @@ extern "C" int petch_trace_ion_yield_batch(petch_ctx* ctx, int nfeat,
   std::vector<IonFeature> t(nfeat);
   long long end = 0;
   int max_nf = 0;
+  bool grids = true;  // every surface has a grid
   for (int f = 0; f < nfeat; ++f) {
     const petch_ion_feature& a = feats[f];
     PETCH_ARG(ctx, a.bvh, "trace_ion_yield_batch: feature %d has no BVH", f);
@@ -1680,6 +1990,7 @@ extern "C" int petch_trace_ion_yield_batch(petch_ctx* ctx, int nfeat,
     PETCH_ARG(ctx, a.n >= 0, "trace_ion_yield_batch: feature %d: n < 0", f);
     IonFeature& d = t[f];
     d.bv = petch_bvh_view(a.bvh);
+    if (a.bvh->nf > 0) grids = petch_grid_view(a.bvh, &d.gv) && grids;
     d.b = make_box(&a.box);
     d.src = make_source(&a.src);
     const petch_ion_params& ip = a.ip;
@@ -1724,15 +2035,13 @@ extern "C" int petch_trace_ion_yield_batch(petch_ctx* ctx, int nfeat,
     PETCH_LAUNCH_CHECK(ctx);
   }
   if (end > 0) {
-    RayQueue q;
-    int rc = make_queue(ctx, (int)end, q);
+    const IonYieldBatch<BvhView> tree{dev, nfeat};
+    const int rc = grids ? launch_walk(ctx, k_trace<IonYieldBatch<GridView>>,
+                                       IonYieldBatch<GridView>{dev, nfeat}, tree, (int)end,
+                                       petch_hit_counter(ctx, 1))
+                         : launch_tree(ctx, k_trace<IonYieldBatch<BvhView>>, tree, (int)end,
+                                       petch_hit_counter(ctx, 1));
     if (rc) return rc;
-    IonYieldBatch pol{dev, nfeat};
-    const unsigned grid =
-        persistent_blocks(ctx, (const void*)k_trace_ion_yield_batch, (int)end);
-    hipLaunchKernelGGL(k_trace_ion_yield_batch, dim3(grid), dim3(kBS), 0, ctx->stream, pol, q,
-                       petch_hit_counter(ctx, 1));
-    PETCH_LAUNCH_CHECK(ctx);
   }
   if (max_nf > 0 && ctx->deterministic) {
     hipLaunchKernelGGL(k_fix_finish_ion_batch, dim3(gx, nfeat), dim3(kBS), 0, ctx->stream, dev);
@@ -1767,6 +2076,12 @@ extern "C" int petch_trace_ff(petch_ctx* ctx, const petch_bvh* bvh, const petch_
   long long n = (long long)nf * n_ff;
   PETCH_ARG(ctx, n < (1LL << 31), "trace_ff: nf*n_ff too large");
   if (n == 0) return PETCH_OK;
+  GridView g;
+  if (petch_grid_view(bvh, &g))
+    return trace_surface<false>(ctx, bvh, [&](auto view) {
+      return FormFactor<decltype(view)>{view, make_box(box), centroids, gas_normals, n_ff, seed,
+                                        hitface};
+    }, (int)n, nullptr);
   hipLaunchKernelGGL(k_trace_ff, dim3(petch_blocks(n, kBS)), dim3(kBS), 0, ctx->stream,
                      petch_bvh_view(bvh), make_box(box), centroids, gas_normals, nf, n_ff, seed,
                      hitface);
@@ -1784,7 +2099,7 @@ extern "C" int petch_set_trace_occupancy(petch_ctx* ctx, int blocks_per_cu) {
 extern "C" int petch_trace_occupancy_limit(petch_ctx* ctx, int* blocks_per_cu) {
   PETCH_ARG(ctx, ctx && blocks_per_cu, "trace_occupancy_limit: null pointer");
   int per_cu = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)k_trace_neutral_rr, kBS,
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)k_trace5<NeutralRR<BvhView>>, kBS,
                                                    0) != hipSuccess)
     return petch_set_error(ctx, PETCH_E_HIP, "trace_occupancy_limit: occupancy query failed");
   *blocks_per_cu = per_cu;

@@ -146,6 +146,12 @@ class DdaParams(ctypes.Structure):
                 ("beta_a", c_double), ("beta_b", c_double)]
 
 
+class GridItem(ctypes.Structure):
+    """petch_grid_item: the grid of one BVH's marching-cubes surface."""
+    _fields_ = [("bvh", c_void_p), ("verts", c_void_p), ("faces", c_void_p), ("cells", c_void_p),
+                ("nx", c_int), ("ny", c_int), ("nz", c_int), ("dx", c_double)]
+
+
 class McItem(ctypes.Structure):
     """petch_mc_item: one grid of a batched marching cubes."""
     _fields_ = [("phi", c_void_p), ("nx", c_int), ("ny", c_int), ("nz", c_int), ("dx", c_double),
@@ -253,6 +259,10 @@ SIGNATURES = {
     "petch_extend_batch": [P, c_int, P],
     "petch_advect_step": [P, P, P, P, P, c_int, c_int, c_int, c_double, c_double, P],
     "petch_advect_adjoint": [P, P, P, P, P, c_int, c_int, c_int, c_double, c_double, P, P],
+    "petch_marching_cubes_cells": [P, P, c_int, c_int, c_int, c_double, P, P, c_int, c_int, P, P, P],
+    "petch_marching_cubes_batch_cells": [P, c_int, P, P],
+    "petch_bvh_set_grid": [P, P],
+    "petch_bvh_set_grid_batch": [P, c_int, P],
     "petch_marching_cubes_batch": [P, c_int, P],
     "petch_nearest_face_value_batch": [P, c_int, P],
     "petch_radiosity_assemble": [P, P, c_int, c_int, P, P, P],

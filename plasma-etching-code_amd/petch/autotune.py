@@ -57,10 +57,10 @@ class TraceTuner:
         stream = torch.cuda.current_stream(dev)
         for q in QUALITIES:
             mesh.bvh.set_quality(q)
-            mesh.bvh.build(mesh.verts, mesh.faces)          # untimed: allocation on first use
+            mesh.build_bvh()          # untimed: allocation on first use
             a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
             a.record(stream)
-            mesh.bvh.build(mesh.verts, mesh.faces)
+            mesh.build_bvh()
             b.record(stream)
             for occ in occs:
                 ops.set_trace_occupancy(occ, dev)
@@ -83,5 +83,5 @@ class TraceTuner:
     def _apply(mesh, quality, occ):
         ops.set_trace_occupancy(occ, mesh.device)
         mesh.bvh.set_quality(quality)
-        mesh.bvh.build(mesh.verts, mesh.faces)
+        mesh.build_bvh()
         return quality, occ

@@ -22,13 +22,16 @@ SEED_MASK = 0xFFFFFFFFFFFFFFFF
 class SurfaceMesh:
     """The triangle surface of phi with everything the flux and extension stages need.
 
+    Its ray traces walk the cells of phi's grid (Bvh.set_grid) and leave the tree the nearest-face
+    queries and the rays that meet two faces at once.
+
     rays_per_step (optional): the rays a step will trace on this surface. A clustered BVH
     (slower build, faster traces) pays off from ~1000 rays per face; below that the fast
     Morton build is used. Without it the BVH picks by mesh size."""
 
     def __init__(self, device, rays_per_step=None):
         self.device = device
-        self.bufs = ops.MeshBuffers(device)
+        self.bufs = ops.MeshBuffers(device, cells=True)
         self.bvh = ops.Bvh(device)
         self.rays_per_step = rays_per_step
         self.quality = None    # a fixed BVH build quality (petch.autotune's choice), or None
@@ -37,15 +40,18 @@ class SurfaceMesh:
         self.nv = 0
 
     def build(self, phi, dx):
-        return self.build_from(*ops.marching_cubes(phi, dx, self.bufs))
+        v, f = ops.marching_cubes(phi, dx, self.bufs)
+        return self.build_from(v, f, grid=self.bufs.grid)
 
-    def build_from(self, v, f, bvh=True, surf=None):
+    def build_from(self, v, f, bvh=True, surf=None, grid=None):
         """Everything after marching cubes, from its (verts, faces) (the batched loop meshes
         all features' grids with one host read, then builds each feature's surface). bvh=False
         leaves the BVH to the caller (the batched loop builds all features' trees together with
         ops.bvh_build_batch over bvh_item()); with a list `surf` the face attributes and
-        adjacency are only allocated and their item appended, for ops.surface_build_batch."""
+        adjacency are only allocated and their item appended, for ops.surface_build_batch. grid:
+        the MeshBuffers.grid of the marching cubes that made v and f, when it wrote the cells."""
         self.verts, self.faces = v, f
+        self.grid = grid
         self.nv, self.nf = int(v.shape[0]), int(f.shape[0])
         if surf is None:
             self.centroids, self.areas, self.normals = ops.mesh_attrs(v, f)
@@ -66,12 +72,16 @@ class SurfaceMesh:
                 self.bvh.set_quality(q)
                 self._quality = q
         if bvh:
-            self.bvh.build(v, f)
+            self.build_bvh()
         return self
 
+    def build_bvh(self):
+        """The BVH of this surface, with its grid."""
+        self.bvh.build(self.verts, self.faces).set_grid(self.verts, self.faces, self.grid)
+
     def bvh_item(self):
-        """(bvh, verts, faces) of this surface for ops.bvh_build_batch."""
-        return (self.bvh, self.verts, self.faces)
+        """(bvh, verts, faces, grid) of this surface for ops.bvh_build_batch."""
+        return (self.bvh, self.verts, self.faces, self.grid)
 
 
 def ion_params(par):

@@ -229,14 +229,29 @@ def slice_gas_area_adjoint(phi, dx, eps, garea):
 
 # ------------------------------------------------------------------ surface mesh
 class MeshBuffers:
-    """Grow-only device buffers for the per-step surface mesh (reused step to step)."""
+    """Grow-only device buffers for the per-step surface mesh (reused step to step). With cells,
+    marching cubes also writes the grid cells' face lists: `grid` then holds (cells, nx, ny, nz, dx)
+    of the last surface, for Bvh.set_grid."""
 
-    def __init__(self, device):
+    def __init__(self, device, cells=False):
         self.device = device
+        self.want_cells = bool(cells)
         self.cap_v = 0
         self.cap_f = 0
         self.verts = None
         self.faces = None
+        self.cells = None
+        self.grid = None
+
+    def ensure_cells(self, nx, ny, nz, dx):
+        n = nx * ny * nz
+        if not self.want_cells or n >= 1 << 30 or nx * ny >= 1 << 24:     # beyond the walks' indices
+            self.grid = None
+            return None
+        if self.cells is None or self.cells.numel() < n:
+            self.cells = torch.empty((n,), dtype=i32, device=self.device)
+        self.grid = (self.cells, nx, ny, nz, float(dx))
+        return self.cells
 
     def ensure(self, nv, nf):
         if nv > self.cap_v:
@@ -257,12 +272,13 @@ def marching_cubes(phi, dx, bufs=None):
     ctx = _ctx(phi)
     nv = ctypes.c_int()
     nf = ctypes.c_int()
+    words = bufs.ensure_cells(nx, ny, nz, dx)
     from ._abi import PetchCapacityError
     for _ in range(2):
         bufs.ensure(1, 1)
         try:
-            ctx.call("petch_marching_cubes", ptr(phi, f32, "phi"), nx, ny, nz, float(dx),
-                     ptr(bufs.verts), ptr(bufs.faces), bufs.cap_v, bufs.cap_f,
+            ctx.call("petch_marching_cubes_cells", ptr(phi, f32, "phi"), nx, ny, nz, float(dx),
+                     ptr(bufs.verts), ptr(bufs.faces), bufs.cap_v, bufs.cap_f, ptr(words),
                      ctypes.byref(nv), ctypes.byref(nf))
             break
         except PetchCapacityError:
@@ -282,6 +298,9 @@ def marching_cubes_batch(items):
         return []
     counts = np.zeros((len(items), 2), np.int32)
     base = counts.ctypes.data
+    words = (ctypes.c_void_p * len(items))()
+    for k, (phi, dx, bufs) in enumerate(items):
+        words[k] = ptr(bufs.ensure_cells(*_shape3(phi), dx)).value
     for _ in range(2):
         arr = (McItem * len(items))()
         for k, (phi, dx, bufs) in enumerate(items):
@@ -290,8 +309,9 @@ def marching_cubes_batch(items):
             arr[k] = McItem(ptr(phi, f32, "phi"), nx, ny, nz, float(dx), ptr(bufs.verts),
                             ptr(bufs.faces), bufs.cap_v, bufs.cap_f, base + 8 * k, base + 8 * k + 4)
         try:
-            _ctx(items[0][0]).call("petch_marching_cubes_batch", len(items),
-                                   ctypes.cast(arr, ctypes.c_void_p))
+            _ctx(items[0][0]).call("petch_marching_cubes_batch_cells", len(items),
+                                   ctypes.cast(arr, ctypes.c_void_p),
+                                   ctypes.cast(words, ctypes.c_void_p))
             break
         except PetchCapacityError:
             for (phi, dx, bufs), (nv, nf) in zip(items, counts.tolist()):
@@ -383,6 +403,13 @@ class Bvh:
         self.nf = int(faces.shape[0])
         self.ctx.call("petch_bvh_build", self.h, ptr(verts, f32, "verts"), ptr(faces, i32, "faces"),
                       int(verts.shape[0]), self.nf)
+        return self
+
+    def set_grid(self, verts, faces, grid):
+        """Ray traces walk the cells of the grid the mesh was cut from (petch_bvh_set_grid):
+        grid is the MeshBuffers.grid of the marching cubes that made verts and faces, or None.
+        After each build()."""
+        bvh_set_grid_batch([(self, verts, faces, grid)])
         return self
 
     def query_ray(self, orig, dirs, tmax=1.0e6):
@@ -872,7 +899,7 @@ def nearest_face_value_batch(items, miss=1.0):
 
 def bvh_build_batch(items):
     """Bvh.build for many meshes with their refits in one launch (petch_bvh_build_batch).
-    items: (Bvh, verts, faces) tuples."""
+    items: (Bvh, verts, faces) tuples, or (Bvh, verts, faces, grid) to follow it with Bvh.set_grid."""
     import ctypes
     if not items:
         return
@@ -882,7 +909,7 @@ def bvh_build_batch(items):
     fs = (ctypes.c_void_p * n)()
     nv = (ctypes.c_int * n)()
     nf = (ctypes.c_int * n)()
-    for k, (bvh, v, f) in enumerate(items):
+    for k, (bvh, v, f, *_) in enumerate(items):
         hs[k] = bvh.h.value
         vs[k] = ptr(v, f32, "verts").value
         fs[k] = ptr(f, i32, "faces").value
@@ -891,6 +918,26 @@ def bvh_build_batch(items):
     items[0][0].ctx.call("petch_bvh_build_batch", n, ctypes.cast(hs, ctypes.c_void_p),
                          ctypes.cast(vs, ctypes.c_void_p), ctypes.cast(fs, ctypes.c_void_p),
                          ctypes.cast(nv, ctypes.c_void_p), ctypes.cast(nf, ctypes.c_void_p))
+    bvh_set_grid_batch([it for it in items if len(it) > 3])
+
+
+def bvh_set_grid_batch(items):
+    """Bvh.set_grid for many surfaces in one launch per stage (petch_bvh_set_grid_batch).
+    items: (Bvh, verts, faces, grid) tuples; a surface without faces or grid is skipped."""
+    import ctypes
+    from ._abi import GridItem
+    items = [it for it in items if it[3] is not None and 0 < int(it[2].shape[0]) < 1 << 28]
+    if not items:
+        return
+    arr = (GridItem * len(items))()
+    for k, (bvh, v, f, (cells, nx, ny, nz, dx)) in enumerate(items):
+        arr[k] = GridItem(bvh.h.value, ptr(v, f32, "verts"), ptr(f, i32, "faces"),
+                          ptr(cells, i32, "cells"), nx, ny, nz, dx)
+    ctx = items[0][0].ctx
+    if len(items) == 1:
+        ctx.call("petch_bvh_set_grid", ctypes.cast(arr, ctypes.c_void_p))
+    else:
+        ctx.call("petch_bvh_set_grid_batch", len(items), ctypes.cast(arr, ctypes.c_void_p))
 
 
 def nearest_face_value(bvh, src, pts, miss=1.0):

@@ -453,7 +453,8 @@ class EtchLoop:
         ops.surface_build_batch over `surf` (the list its item is appended to)."""
         tm = time.time()
         with self.timer.region("mesh"):
-            self.meshes[step % 2].build_from(*mc, bvh=False, surf=surf)
+            mesh = self.meshes[step % 2]
+            mesh.build_from(*mc, bvh=False, surf=surf, grid=mesh.bufs.grid)
         self.timings['mesh'] += time.time() - tm
 
     def begin_mesh(self, step, mc=None, bvh=True, staged=False):
@@ -626,7 +627,7 @@ class EtchLoop:
         V = self._V
         if bvh_err:
             raise RuntimeError(f"step {step}: BVH traversal guard tripped (code {bvh_err}: "
-                               "1 stack overflow, 2 corrupt tree, 3 tree too deep); the flux is "
+                               "1 stack overflow, 2 corrupt tree, 3 tree too deep, 4 surface off its grid); the flux is "
                                "incomplete")
         if nbad:
             warnings.warn(f"step {step}: {nbad} non-finite surface velocities (NaN/inf) zeroed; "
