@@ -811,8 +811,9 @@ __global__ void k_query_point(BvhView b, const float* __restrict__ p, int n, flo
                               int* __restrict__ face, float* __restrict__ dist) {
   int i = blockIdx.x * kBS + threadIdx.x;
   if (i >= n) return;
+  petch::ScratchStack stk;
   petch::PointHit h =
-      petch::bvh_closest_point(b, petch::v3(p[3 * i], p[3 * i + 1], p[3 * i + 2]), maxd);
+      petch::bvh_closest_point(b, petch::v3(p[3 * i], p[3 * i + 1], p[3 * i + 2]), maxd, stk);
   face[i] = h.face;
   if (dist) dist[i] = h.face >= 0 ? sqrtf(h.d2) : -1.f;
 }

@@ -666,28 +666,50 @@ __global__ void k_band_emit(const ExtendItem* __restrict__ it, int n, long long 
   }
 }
 
+// The workgroup's stack of a point query: this lane's column of the LDS part.
+constexpr int kPointLds = 8;
+using PointStack = petch::TravStack<kBS, kPointLds>;
+__device__ __forceinline__ void point_stack(PointStack& s) {
+  __shared__ int lds_n[kPointLds * kBS];
+  __shared__ float lds_t[kPointLds * kBS];
+  s.lds_n = lds_n + threadIdx.x;
+  s.lds_t = lds_t + threadIdx.x;
+}
+
+// Where a band node's nearest face is expected: phi is a distance after each reinit, and the mesh
+// lies within a fraction of a cell of its zero level.
+__device__ __forceinline__ float band_hint(const ExtendItem& e, long long m) {
+  return 1.1f * fabsf(e.phi[m]) + 0.5f * (float)e.dx;
+}
+
 // one nearest-face query per band node, over the list in grid-stride order
-__global__ void k_extend(const ExtendItem* __restrict__ it, int n, const int* __restrict__ idx,
+__global__ void __launch_bounds__(kBS) k_extend(const ExtendItem* __restrict__ it, int n, const int* __restrict__ idx,
                          const int* __restrict__ count) {
+  PointStack stk;
+  point_stack(stk);
   const int cnt = *count;
   for (int i = blockIdx.x * kBS + threadIdx.x; i < cnt; i += gridDim.x * kBS) {
     long long m;
     const ExtendItem& e = it[locate_item(it, n, idx[i], m)];
-    const petch::PointHit h = petch::bvh_closest_point(e.bv, item_node_pos(e, m), 1.0e6f);
+    const petch::PointHit h =
+        petch::bvh_closest_point(e.bv, item_node_pos(e, m), 1.0e6f, stk, band_hint(e, m));
     e.Fs[m] = h.face >= 0 ? e.V[h.face] : 0.f;
   }
 }
 
 // Adjoint of k_extend (one grid): the extension copies V[nearest face] to each band node, so
 // its transpose adds each band node's gFs (read through the item's Fs) to gV[nearest face].
-__global__ void k_extend_adjoint(const ExtendItem* __restrict__ it, int n,
+__global__ void __launch_bounds__(kBS) k_extend_adjoint(const ExtendItem* __restrict__ it, int n,
                                  const int* __restrict__ idx, const int* __restrict__ count,
                                  float* __restrict__ gV) {
+  PointStack stk;
+  point_stack(stk);
   const int cnt = *count;
   for (int i = blockIdx.x * kBS + threadIdx.x; i < cnt; i += gridDim.x * kBS) {
     long long m;
     const ExtendItem& e = it[locate_item(it, n, idx[i], m)];
-    const petch::PointHit h = petch::bvh_closest_point(e.bv, item_node_pos(e, m), 1.0e6f);
+    const petch::PointHit h =
+        petch::bvh_closest_point(e.bv, item_node_pos(e, m), 1.0e6f, stk, band_hint(e, m));
     if (h.face >= 0) atomicAdd(gV + h.face, e.Fs[m]);
   }
 }
@@ -702,7 +724,10 @@ struct NearestItem {
   long long end;
 };
 
-__global__ void k_nearest_batch(const NearestItem* __restrict__ it, int n, long long total) {
+__global__ void __launch_bounds__(kBS) k_nearest_batch(const NearestItem* __restrict__ it, int n,
+                                                       long long total) {
+  PointStack stk;
+  point_stack(stk);
   const long long g = (long long)blockIdx.x * kBS + threadIdx.x;
   if (g >= total) return;
   int lo = 0, hi = n - 1;
@@ -713,7 +738,7 @@ __global__ void k_nearest_batch(const NearestItem* __restrict__ it, int n, long 
   const NearestItem& e = it[lo];
   const long long i = g - (lo ? it[lo - 1].end : 0);
   const petch::PointHit h = petch::bvh_closest_point(
-      e.bv, petch::v3(e.pts[3 * i], e.pts[3 * i + 1], e.pts[3 * i + 2]), 1.0e6f);
+      e.bv, petch::v3(e.pts[3 * i], e.pts[3 * i + 1], e.pts[3 * i + 2]), 1.0e6f, stk);
   e.out[i] = h.face >= 0 ? e.src[h.face] : e.miss;
 }
 

@@ -468,6 +468,25 @@ def test_surface_rate_adjoint_matches_oracle(chem, yields):
     np.testing.assert_allclose(xF.grad.cpu().numpy(), out[0].cpu().numpy(), rtol=0, atol=0)
 
 
+@pytest.mark.parametrize("scale", [1e-3, 0.4, 1.0, 30.0])
+def test_extension_takes_the_nearest_face_whatever_phi_is(scale):
+    """The extension's query starts from a radius taken from |phi|. Where phi isn't a distance (here
+    too small by 1000, a little, and too large) the nearest face is the one that a query without the
+    radius returns, node by node."""
+    from petch import ops
+    phi, v, f = _mesh()
+    dx = 0.25
+    bvh = ops.Bvh(_dev()).build(_t(v), _t(f))
+    V = np.arange(1, len(f) + 1, dtype=np.float32)
+    inb = np.abs(phi.astype(np.float64)) < 4 * dx
+    ph = np.where(inb, phi * np.float32(scale), np.float32(1e6)).astype(np.float32)
+    Fs = ops.extend(bvh, _t(V), _t(ph), dx, 1e5).cpu().numpy()
+    pts = (np.argwhere(inb) * dx).astype(np.float32)
+    gf = bvh.query_point(_t(pts))[0].cpu().numpy()
+    np.testing.assert_array_equal(Fs[inb], V[gf])
+    np.testing.assert_array_equal(Fs[~inb], 0.0)
+
+
 def test_extend_adjoint_is_the_transpose():
     """petch_extend_adjoint sends each band node's gradient to its nearest face: it equals the
     scatter over the GPU's own nearest faces, and <gFs, extend(V)> = <extend_adjoint(gFs), V>
