@@ -4,12 +4,12 @@
 //   morton   30-bit codes of the centroids                -> stable LDS radix sort (sort.hip)
 //   leaves   triangle vertices gathered into Morton order (48 B per leaf)
 //   karras   internal nodes from the sorted codes (Karras, HPG 2012), ties broken by index
-//   refit    leaves climb to the root; at each node the second arriving thread (atomic flag)
-//            unions the two child boxes and continues, so each node is built exactly once
+//   refit    boxes of the nodes inside each 256-leaf tile in LDS, then those of the few nodes that
+//            span tiles from the tiles' prefix, suffix and whole boxes
 //   wide     4-wide nodes at binary-node indices: on large meshes a top-down collapse that
-//            opens the larger-area inner child first (one workgroup, level by level); on small
-//            ones every binary node at even depth (parity from its parent chain) gathers its
-//            grandchildren (one parallel pass)
+//            opens the larger-area inner child first (the top levels in one workgroup, then a
+//            wavefront per subtree); on small ones every binary node at even depth (parity from
+//            its parent chain) gathers its grandchildren (one parallel pass)
 // plus the two query entry points used by the tests (the trace kernels inline the traversal).
 #include "common.h"
 #include <vector>
@@ -31,10 +31,13 @@ namespace {
 
 constexpr int kBS = 256;
 
+enum Hdr { H_COUNT, H_SIDE, H_LEVEL, H_OVER, H_OVER_LEVEL, H_DONE };
+
 struct Work {  // device scratch owned by the BVH, carved from bvh->work
   float4* cen;
   uint32_t *keys, *vals, *ktmp, *vtmp;
-  int *pint, *pleaf, *flags, *err;
+  int *pint, *pleaf, *err;
+  int* hdr;      // device state of the area-driven collapse and of the clustering (Hdr)
   float* part;   // per-block bounds (6 per block)
   float* scene;  // 6 floats
   float* root;   // 6 floats
@@ -42,7 +45,7 @@ struct Work {  // device scratch owned by the BVH, carved from bvh->work
 
 size_t work_bytes(int cap_f) {
   size_t nb = (cap_f + kBS - 1) / kBS;
-  return (size_t)cap_f * 16 + (size_t)cap_f * 4 * 4 + (size_t)cap_f * 4 * 3 + 64 +
+  return (size_t)cap_f * 16 + (size_t)cap_f * 4 * 4 + (size_t)cap_f * 4 * 2 + 64 +
          nb * 6 * 4 + 64 + 64 + 1024;
 }
 
@@ -57,8 +60,8 @@ Work carve(void* base, int cap_f) {
   w.vtmp = (uint32_t*)p; p += (size_t)cap_f * 4;
   w.pint = (int*)p; p += (size_t)cap_f * 4;
   w.pleaf = (int*)p; p += (size_t)cap_f * 4;
-  w.flags = (int*)p; p += (size_t)cap_f * 4;
-  w.err = (int*)p; p += 64;
+  w.err = (int*)p;
+  w.hdr = w.err + 4; p += 64;
   w.part = (float*)p; p += nb * 6 * 4;
   w.scene = (float*)p; p += 64;
   w.root = (float*)p; p += 64;
@@ -221,14 +224,17 @@ __device__ __forceinline__ void bvh_karras_node(const uint32_t* __restrict__ key
   int lo = i < j ? i : j, hi = i < j ? j : i;
   int left = (lo == gamma) ? ~gamma : gamma;
   int right = (hi == gamma + 1) ? ~(gamma + 1) : gamma + 1;
-  nodes[i].d = make_int4(left, right, 0, 0);
+  nodes[i].d = make_int4(left, right, lo, hi);  // children, first and last leaf
   if (left < 0) pleaf[~left] = i; else pint[left] = i;
   if (right < 0) pleaf[~right] = i; else pint[right] = i;
   if (i == 0) pint[0] = -1;
 }
 
+// `done`, here and in the refit: where the clustered tree is complete there is nothing to do.
 __global__ void k_bvh_karras(const uint32_t* __restrict__ keys, int n, BvhNode* __restrict__ nodes,
-                             int* __restrict__ pint, int* __restrict__ pleaf) {
+                             int* __restrict__ pint, int* __restrict__ pleaf,
+                             const int* __restrict__ done) {
+  if (done && *done) return;
   int i = blockIdx.x * kBS + threadIdx.x;
   if (i < n - 1) bvh_karras_node(keys, n, nodes, pint, pleaf, i);
 }
@@ -243,69 +249,220 @@ __device__ __forceinline__ void put_child_box(BvhNode* nd, bool left, const floa
   }
 }
 
-// Leaf s climbs towards the root; at each node the second arriving thread (acq_rel flag at
-// memory scope kScope) writes the node's box from both children and goes on, the first one
-// stops. Threads of the whole grid need agent scope; within one workgroup (all threads on one
-// CU, one L2) workgroup scope suffices and spares the L2 write-back an agent-scope release
-// costs on a chip whose XCDs keep separate L2s.
-template <int kScope = __HIP_MEMORY_SCOPE_AGENT>
-__device__ __forceinline__ void refit_leaf(const float4* __restrict__ tris, BvhNode* nodes,
-                                           const int* __restrict__ pint,
-                                           const int* __restrict__ pleaf, int* flags, int n,
-                                           float* root, int s) {
-  float4 a = tris[3 * s], b = tris[3 * s + 1], c = tris[3 * s + 2];
-  float lo[3] = {fminf(a.x, fminf(b.x, c.x)), fminf(a.y, fminf(b.y, c.y)), fminf(a.z, fminf(b.z, c.z))};
-  float hi[3] = {fmaxf(a.x, fmaxf(b.x, c.x)), fmaxf(a.y, fmaxf(b.y, c.y)), fmaxf(a.z, fmaxf(b.z, c.z))};
-  int child = ~s;
-  int p = pleaf[s];
-  for (int guard = 0; p >= 0 && p < n - 1 && guard < n; ++guard) {
-    BvhNode* nd = nodes + p;
-    bool isleft = nd->d.x == child;
-    put_child_box(nd, isleft, lo, hi);
-    int old = __hip_atomic_fetch_add(flags + p, 1, __ATOMIC_ACQ_REL, kScope);
-    if (old == 0) return;  // the sibling's thread finishes this node
-    const float* q = (const float*)nd;
-    for (int k = 0; k < 3; ++k) {
-      lo[k] = fminf(q[k], q[6 + k]);
-      hi[k] = fmaxf(q[3 + k], q[9 + k]);
-    }
-    child = p;
-    p = pint[p];
+// The refit: every node's two child boxes, from the leaves' triangles. One climb from the leaves
+// with a flag in memory at each node is a chain of dependent global accesses as deep as the tree,
+// each with an agent-scope release (51 us at 8k faces, 237 us at 47k), or with one workgroup a
+// tree, so that workgroup scope is enough, a pass over all leaves by that workgroup (2.55 ms for
+// 32 trees of 8 to 30k faces side by side). Here a workgroup takes a tile of kTile leaves in
+// Morton order and climbs in LDS through the nodes whose leaves lie inside the tile; a node spanning tiles, a few
+// for each tile, is the union of its first tile's suffix box, its last tile's prefix box and the
+// whole tiles between, so no chain runs through memory: 16 us at 8k faces, 113 us for the 32
+// trees. The boxes are the same, minima and maxima of the same numbers.
+constexpr int kTile = kBS;
+
+struct RefitItem {
+  const float4* tris;
+  BvhNode* nodes;
+  const int *pint, *pleaf;
+  float* scr;        // prefix boxes, then suffix boxes, 6 floats a leaf (the wide nodes' memory)
+  float* root;
+  const int* done;   // nothing to refit where this is set
+  int n;
+  long long blk0;    // first tile of this tree in the launch
+};
+
+__device__ __forceinline__ const RefitItem& refit_item(const RefitItem* __restrict__ it, int n) {
+  int lo = 0, hi = n - 1;
+  const long long b = blockIdx.x;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (it[mid].blk0 <= b) lo = mid; else hi = mid - 1;
   }
+  return it[lo];
+}
+
+__device__ __forceinline__ bool in_one_tile(int4 d) { return d.z / kTile == d.w / kTile; }
+
+__device__ __forceinline__ void put_root(float* root, const float lo[3], const float hi[3]) {
   for (int k = 0; k < 3; ++k) {
     root[k] = lo[k];
     root[3 + k] = hi[k];
   }
 }
 
-__global__ void k_bvh_refit(const float4* __restrict__ tris, BvhNode* nodes,
-                            const int* __restrict__ pint, const int* __restrict__ pleaf,
-                            int* flags, int n, float* root) {
-  int s = blockIdx.x * kBS + threadIdx.x;
-  if (s >= n) return;
-  refit_leaf(tris, nodes, pint, pleaf, flags, n, root, s);
+__device__ __forceinline__ void refit_tile(const RefitItem& it, int tile) {
+  __shared__ int4 s_d[kTile];
+  __shared__ int s_par[kTile], s_flag[kTile];
+  __shared__ float s_box[12][kTile];
+  __shared__ float s_pre[kBS / 64][6], s_suf[kBS / 64][6];
+  const int n = it.n, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int base = tile * kTile, i = base + tid;
+  const bool node = i < n - 1, leaf = i < n;
+  if (node) {
+    s_d[tid] = it.nodes[i].d;
+    s_par[tid] = it.pint[i];
+    s_flag[tid] = 0;
+  }
+  float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+  if (leaf) {
+    const float4 a = it.tris[3 * i], b = it.tris[3 * i + 1], c = it.tris[3 * i + 2];
+    lo[0] = fminf(a.x, fminf(b.x, c.x)); hi[0] = fmaxf(a.x, fmaxf(b.x, c.x));
+    lo[1] = fminf(a.y, fminf(b.y, c.y)); hi[1] = fmaxf(a.y, fmaxf(b.y, c.y));
+    lo[2] = fminf(a.z, fminf(b.z, c.z)); hi[2] = fmaxf(a.z, fmaxf(b.z, c.z));
+  }
+  if (n > kTile) {
+    float pre[6], suf[6];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      pre[k] = suf[k] = lo[k];
+      pre[3 + k] = suf[3 + k] = hi[k];
+    }
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+#pragma unroll
+      for (int k = 0; k < 6; ++k) {
+        const float u = __shfl_up(pre[k], d, 64), v = __shfl_down(suf[k], d, 64);
+        if (lane >= d) pre[k] = k < 3 ? fminf(pre[k], u) : fmaxf(pre[k], u);
+        if (lane + d < 64) suf[k] = k < 3 ? fminf(suf[k], v) : fmaxf(suf[k], v);
+      }
+    }
+    if (lane == 63)
+      for (int k = 0; k < 6; ++k) s_pre[w][k] = pre[k];
+    if (lane == 0)
+      for (int k = 0; k < 6; ++k) s_suf[w][k] = suf[k];
+    __syncthreads();
+    for (int q = 0; q < kBS / 64; ++q) {
+#pragma unroll
+      for (int k = 0; k < 6; ++k) {
+        if (q < w) pre[k] = k < 3 ? fminf(pre[k], s_pre[q][k]) : fmaxf(pre[k], s_pre[q][k]);
+        if (q > w) suf[k] = k < 3 ? fminf(suf[k], s_suf[q][k]) : fmaxf(suf[k], s_suf[q][k]);
+      }
+    }
+    if (leaf) {
+      float* o = it.scr + 6LL * i;
+#pragma unroll
+      for (int k = 0; k < 6; ++k) {
+        o[k] = pre[k];
+        o[6LL * n + k] = suf[k];
+      }
+    }
+  }
+  __syncthreads();
+  if (leaf) {
+    int child = ~i, p = it.pleaf[i];
+    while (true) {
+      const int l = p - base;
+      if (l < 0 || l >= kTile || !in_one_tile(s_d[l])) {
+        put_child_box(it.nodes + p, it.nodes[p].d.x == child, lo, hi);
+        break;
+      }
+      const int side = s_d[l].x == child ? 0 : 6;
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        s_box[side + k][l] = lo[k];
+        s_box[side + 3 + k][l] = hi[k];
+      }
+      const int seen =
+          __hip_atomic_fetch_add(s_flag + l, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP);
+      if (seen == 0) break;   // the second child to arrive goes on
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        lo[k] = fminf(s_box[k][l], s_box[6 + k][l]);
+        hi[k] = fmaxf(s_box[3 + k][l], s_box[9 + k][l]);
+      }
+      child = p;
+      p = s_par[l];
+      if (p < 0) {
+        put_root(it.root, lo, hi);
+        break;
+      }
+    }
+  }
+  __syncthreads();
+  if (node && in_one_tile(s_d[tid])) {
+    BvhNode* nd = it.nodes + i;
+    nd->a = make_float4(s_box[0][tid], s_box[1][tid], s_box[2][tid], s_box[3][tid]);
+    nd->b = make_float4(s_box[4][tid], s_box[5][tid], s_box[6][tid], s_box[7][tid]);
+    nd->c = make_float4(s_box[8][tid], s_box[9][tid], s_box[10][tid], s_box[11][tid]);
+  }
 }
 
-// The refits of many BVHs in one launch: the climbs are chains of dependent global accesses
-// (tens of microseconds for one tree however small), so the trees of a batched step refit side
-// by side instead of one after the other.
-struct RefitItem {
-  const float4* tris;
-  BvhNode* nodes;
-  const int *pint, *pleaf;
-  int* flags;
-  float* root;
-  int n;
-};
+// The box of each node of the tile that spans tiles, into its parent's child slot. A long run of
+// whole tiles is read by the wavefront together, a short one by its own lane.
+constexpr int kSpanSerial = 8;
+__device__ __forceinline__ void refit_span(const RefitItem& it, int tile) {
+  const int n = it.n, i = tile * kTile + threadIdx.x, lane = threadIdx.x & 63;
+  const float* suf = it.scr + 6LL * n;
+  int4 d = make_int4(0, 0, 0, 0);
+  if (i < n - 1) d = it.nodes[i].d;
+  const bool span = !in_one_tile(d);
+  const int t0 = d.z / kTile + 1, t1 = d.w / kTile;   // whole tiles t0 .. t1 - 1
+  float box[6];
+  for (int k = 0; k < 6; ++k) box[k] = k < 3 ? INFINITY : -INFINITY;
+  if (span) {
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {
+      const float a = suf[6LL * d.z + k], b = it.scr[6LL * d.w + k];
+      box[k] = k < 3 ? fminf(a, b) : fmaxf(a, b);
+    }
+    if (t1 - t0 <= kSpanSerial) {
+      for (int t = t0; t < t1; ++t) {
+#pragma unroll
+        for (int k = 0; k < 6; ++k) {
+          const float v = suf[6LL * t * kTile + k];
+          box[k] = k < 3 ? fminf(box[k], v) : fmaxf(box[k], v);
+        }
+      }
+    }
+  }
+  unsigned long long todo = __ballot(span && t1 - t0 > kSpanSerial);
+  while (todo) {
+    const int who = __ffsll(todo) - 1;
+    todo &= todo - 1;
+    const int a = __shfl(t0, who, 64), e = __shfl(t1, who, 64);
+    float part[6];
+    for (int k = 0; k < 6; ++k) part[k] = k < 3 ? INFINITY : -INFINITY;
+    for (int t = a + lane; t < e; t += 64) {
+#pragma unroll
+      for (int k = 0; k < 6; ++k) {
+        const float v = suf[6LL * t * kTile + k];
+        part[k] = k < 3 ? fminf(part[k], v) : fmaxf(part[k], v);
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {
+      const float v = k < 3 ? wave_min(part[k]) : wave_max(part[k]);
+      if (lane == who) box[k] = k < 3 ? fminf(box[k], v) : fmaxf(box[k], v);
+    }
+  }
+  if (span) {
+    const int p = it.pint[i];
+    if (p < 0) put_root(it.root, box, box + 3);
+    else put_child_box(it.nodes + p, it.nodes[p].d.x == i, box, box + 3);
+  }
+}
 
-// One workgroup per tree (the trees of a batched build): the workgroup's threads climb from
-// all of the tree's leaves in turn with workgroup-scope flags, and the trees refit side by side.
-constexpr int kRefitWG = 1024;
-__global__ void __launch_bounds__(kRefitWG) k_bvh_refit_wg(const RefitItem* __restrict__ items) {
-  const RefitItem& it = items[blockIdx.x];
-  for (int s = threadIdx.x; s < it.n; s += kRefitWG)
-    refit_leaf<__HIP_MEMORY_SCOPE_WORKGROUP>(it.tris, it.nodes, it.pint, it.pleaf, it.flags, it.n,
-                                             it.root, s);
+__global__ void __launch_bounds__(kBS) k_bvh_refit_tile(RefitItem it) {
+  if (it.done && *it.done) return;
+  refit_tile(it, blockIdx.x);
+}
+
+__global__ void __launch_bounds__(kBS) k_bvh_refit_span(RefitItem it) {
+  if (it.done && *it.done) return;
+  refit_span(it, blockIdx.x);
+}
+
+// the trees of a batched build, one launch a stage
+__global__ void __launch_bounds__(kBS) k_bvh_refit_tile_many(const RefitItem* __restrict__ items,
+                                                             int n) {
+  const RefitItem& it = refit_item(items, n);
+  refit_tile(it, (int)(blockIdx.x - it.blk0));
+}
+
+__global__ void __launch_bounds__(kBS) k_bvh_refit_span_many(const RefitItem* __restrict__ items,
+                                                             int n) {
+  const RefitItem& it = refit_item(items, n);
+  refit_span(it, (int)(blockIdx.x - it.blk0));
 }
 
 __device__ __forceinline__ void bvh_wide_node(const BvhNode* __restrict__ nodes,
@@ -412,13 +569,11 @@ __global__ void k_bvh_morton_many(const BuildItem* __restrict__ items, int n) {
   if (f < it.nf) bvh_morton_face(it.w.cen, it.w.scene, it.w.keys, it.w.vals, f);
 }
 
-// the leaves in Morton order, and the refit flags cleared
+// the leaves in Morton order
 __global__ void k_bvh_leaves_many(const BuildItem* __restrict__ items, int n) {
   const BuildItem& it = items[build_item_of(items, n, false)];
   const int f = (int)(blockIdx.x - it.fblk0) * kBS + threadIdx.x;
-  if (f >= it.nf) return;
-  bvh_leaf(it.verts, it.faces, it.w.vals, it.tris, f);
-  it.w.flags[f] = 0;
+  if (f < it.nf) bvh_leaf(it.verts, it.faces, it.w.vals, it.tris, f);
 }
 
 __global__ void k_bvh_karras_many(const BuildItem* __restrict__ items, int n) {
@@ -442,91 +597,113 @@ __device__ __forceinline__ float box_area(const float* lo, const float* hi) {
 
 constexpr int kWideBS = 1024;
 constexpr int kWideMaxLevels = 96;
-// The area-driven collapse runs in one workgroup (~0.28 ms at 47k faces) and the clustering in
-// ~50 launches (~1 ms); together they save ~7 % of trace time. Unless the caller chose a
-// quality (petch_bvh_set_quality), meshes below this size get the Morton tree and the
-// per-level grandchildren rule (one parallel pass).
+// The clustering and the area-driven collapse add ~0.28 ms to a build of 47k faces and save ~7 %
+// of trace time. Unless the caller chose a quality (petch_bvh_set_quality), meshes below this size
+// get the Morton tree and the per-level grandchildren rule (one parallel pass).
 constexpr int kWideSahMinFaces = 32768;
 
-// Top-down collapse into 4-wide nodes, one workgroup: starting from the root, each wide node
-// takes its binary node's two children and, twice, replaces the inner child of largest surface
-// area by that child's two children (a leaf stays a leaf), so big boxes are split first. The
-// wide node is stored at its binary node's index and its inner children form the next level.
+// The wide node of binary node b: its two children and, twice, the inner child of largest surface
+// area replaced by that child's two children (a leaf stays a leaf), so big boxes are split first.
+// The wide node is stored at its binary node's index; ref: its children; returns their number.
+__device__ __forceinline__ int wide_sah_node(const BvhNode* __restrict__ nodes, int n,
+                                             BvhWide* __restrict__ wide, int b, int ref[4]) {
+  float lo[4][3], hi[4][3];
+  const float* q = (const float*)(nodes + b);
+  for (int side = 0; side < 2; ++side) {
+    for (int k = 0; k < 3; ++k) {
+      lo[side][k] = q[6 * side + k];
+      hi[side][k] = q[6 * side + 3 + k];
+    }
+    ref[side] = side == 0 ? nodes[b].d.x : nodes[b].d.y;
+  }
+  int cnt = 2;
+#pragma unroll
+  for (int grow = 0; grow < 2; ++grow) {
+    int best = -1;
+    float best_a = -1.f;
+#pragma unroll
+    for (int c = 0; c < 2 + grow; ++c) {
+      if (ref[c] < 0 || ref[c] >= n - 1) continue;   // leaves (and bad refs) stay
+      const float a = box_area(lo[c], hi[c]);
+      if (a > best_a) {
+        best_a = a;
+        best = c;
+      }
+    }
+    const int r = best == 0 ? ref[0] : best == 1 ? ref[1] : best == 2 ? ref[2] : -1;
+    const int at = 2 + grow;
+    for (int k = 0; k < 3; ++k) {
+      lo[at][k] = INFINITY;
+      hi[at][k] = INFINITY;
+    }
+    ref[at] = petch::kWideEmpty;
+    if (r >= 0) {
+      const BvhNode g = nodes[r];
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        if (c == best) {
+          lo[c][0] = g.a.x; lo[c][1] = g.a.y; lo[c][2] = g.a.z;
+          hi[c][0] = g.a.w; hi[c][1] = g.b.x; hi[c][2] = g.b.y;
+          ref[c] = g.d.x;
+        }
+      }
+      lo[at][0] = g.b.z; lo[at][1] = g.b.w; lo[at][2] = g.c.x;
+      hi[at][0] = g.c.y; hi[at][1] = g.c.z; hi[at][2] = g.c.w;
+      ref[at] = g.d.y;
+      ++cnt;
+    }
+  }
+  BvhWide w;
+  w.lox = make_float4(lo[0][0], lo[1][0], lo[2][0], lo[3][0]);
+  w.hix = make_float4(hi[0][0], hi[1][0], hi[2][0], hi[3][0]);
+  w.loy = make_float4(lo[0][1], lo[1][1], lo[2][1], lo[3][1]);
+  w.hiy = make_float4(hi[0][1], hi[1][1], hi[2][1], hi[3][1]);
+  w.loz = make_float4(lo[0][2], lo[1][2], lo[2][2], lo[3][2]);
+  w.hiz = make_float4(hi[0][2], hi[1][2], hi[2][2], hi[3][2]);
+  w.ref = make_int4(ref[0], ref[1], ref[2], ref[3]);
+  w.pad = make_int4(0, 0, 0, 0);
+  wide[b] = w;
+  return cnt;
+}
+
+// Top-down collapse into 4-wide nodes, level by level: the inner children of a level's wide nodes
+// form the next level. Each level is a chain of three dependent fetches a node, so one workgroup
+// (330 us for 47k faces) is bound by how many nodes it has in flight. Here it does the levels
+// below kWideSplit nodes (k_wide_levels with first = true); each workgroup of k_wide_subtrees, one
+// wavefront, then takes its share of the next level down to the leaves, with its lists in LDS.
+// What finds no place there goes to a list in memory that a last launch of k_wide_levels works
+// through (empty unless a subtree is very unbalanced). 28 + 13 + 2 us for the 47k faces.
 // A tree deeper than kWideMaxLevels wide levels leaves error flag 3 (never for Morton trees,
 // whose depth is bounded by the code length plus the index tie-break).
-__global__ void __launch_bounds__(kWideBS) k_bvh_wide_sah(const BvhNode* __restrict__ nodes,
-                                                          int n, BvhWide* __restrict__ wide,
-                                                          int* __restrict__ list_a,
-                                                          int* __restrict__ list_b,
-                                                          int* __restrict__ err) {
+constexpr int kWideSplit = 1024;
+constexpr int kWideList = 1024;   // nodes of one subtree level held in LDS
+
+__global__ void __launch_bounds__(kWideBS) k_wide_levels(const BvhNode* __restrict__ nodes,
+                                                         int n, BvhWide* __restrict__ wide,
+                                                         int* __restrict__ list_a,
+                                                         int* __restrict__ list_b,
+                                                         int* __restrict__ hdr,
+                                                         int* __restrict__ err, bool first) {
   __shared__ int cnt_cur, cnt_next;
+  const int side = first ? 0 : hdr[H_SIDE] ^ 1;   // the second launch's list: the overflow
   if (threadIdx.x == 0) {
-    list_a[0] = 0;
-    cnt_cur = 1;
+    if (first) list_a[0] = 0;
+    cnt_cur = first ? 1 : hdr[H_OVER];
     cnt_next = 0;
   }
   __syncthreads();
-  int* cur = list_a;
-  int* nxt = list_b;
-  for (int level = 0; level < kWideMaxLevels; ++level) {
+  int* cur = side ? list_b : list_a;
+  int* nxt = side ? list_a : list_b;
+  int flip = side, level = first ? 0 : hdr[H_OVER_LEVEL];
+  for (; level < kWideMaxLevels; ++level) {
     const int m = cnt_cur;
-    if (m == 0) break;
+    if (m == 0 || (first && m >= kWideSplit)) break;
     for (int t = threadIdx.x; t < m; t += kWideBS) {
-      const int b = cur[t];
-      float lo[4][3], hi[4][3];
       int ref[4];
-      const float* q = (const float*)(nodes + b);
-      for (int side = 0; side < 2; ++side) {
-        for (int k = 0; k < 3; ++k) {
-          lo[side][k] = q[6 * side + k];
-          hi[side][k] = q[6 * side + 3 + k];
-        }
-        ref[side] = side == 0 ? nodes[b].d.x : nodes[b].d.y;
-      }
-      int cnt = 2;
-      while (cnt < 4) {
-        int best = -1;
-        float best_a = -1.f;
-        for (int c = 0; c < cnt; ++c) {
-          if (ref[c] < 0 || ref[c] >= n - 1) continue;   // leaves (and bad refs) stay
-          const float a = box_area(lo[c], hi[c]);
-          if (a > best_a) {
-            best_a = a;
-            best = c;
-          }
-        }
-        if (best < 0) break;
-        const int r = ref[best];
-        const float* g = (const float*)(nodes + r);
-        for (int k = 0; k < 3; ++k) {
-          lo[best][k] = g[k];
-          hi[best][k] = g[3 + k];
-          lo[cnt][k] = g[6 + k];
-          hi[cnt][k] = g[9 + k];
-        }
-        ref[best] = nodes[r].d.x;
-        ref[cnt] = nodes[r].d.y;
-        ++cnt;
-      }
-      for (int c = cnt; c < 4; ++c) {
-        for (int k = 0; k < 3; ++k) {
-          lo[c][k] = INFINITY;
-          hi[c][k] = INFINITY;
-        }
-        ref[c] = petch::kWideEmpty;
-      }
-      BvhWide w;
-      w.lox = make_float4(lo[0][0], lo[1][0], lo[2][0], lo[3][0]);
-      w.hix = make_float4(hi[0][0], hi[1][0], hi[2][0], hi[3][0]);
-      w.loy = make_float4(lo[0][1], lo[1][1], lo[2][1], lo[3][1]);
-      w.hiy = make_float4(hi[0][1], hi[1][1], hi[2][1], hi[3][1]);
-      w.loz = make_float4(lo[0][2], lo[1][2], lo[2][2], lo[3][2]);
-      w.hiz = make_float4(hi[0][2], hi[1][2], hi[2][2], hi[3][2]);
-      w.ref = make_int4(ref[0], ref[1], ref[2], ref[3]);
-      w.pad = make_int4(0, 0, 0, 0);
-      wide[b] = w;
-      for (int c = 0; c < cnt; ++c) {
-        if (ref[c] >= 0 && ref[c] < n - 1) {
+      const int cnt = wide_sah_node(nodes, n, wide, cur[t], ref);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        if (c < cnt && ref[c] >= 0 && ref[c] < n - 1) {
           const int slot = atomicAdd(&cnt_next, 1);
           if (slot < n - 1) nxt[slot] = ref[c];
         }
@@ -541,8 +718,66 @@ __global__ void __launch_bounds__(kWideBS) k_bvh_wide_sah(const BvhNode* __restr
     int* tmp = cur;
     cur = nxt;
     nxt = tmp;
+    flip ^= 1;
   }
-  if (threadIdx.x == 0 && cnt_cur > 0 && err) *err = 3;
+  if (threadIdx.x == 0) {
+    if (first) {
+      hdr[H_COUNT] = cnt_cur;
+      hdr[H_SIDE] = flip;
+      hdr[H_LEVEL] = level;
+      hdr[H_OVER] = 0;
+      hdr[H_OVER_LEVEL] = 0;
+    }
+    if (cnt_cur > 0 && level >= kWideMaxLevels && err) *err = 3;
+  }
+}
+
+__global__ void __launch_bounds__(64) k_wide_subtrees(const BvhNode* __restrict__ nodes, int n,
+                                                      BvhWide* __restrict__ wide,
+                                                      int* __restrict__ list_a,
+                                                      int* __restrict__ list_b,
+                                                      int* __restrict__ hdr,
+                                                      int* __restrict__ err) {
+  __shared__ int lists[2][kWideList];
+  __shared__ int cnt_next;
+  const int total = hdr[H_COUNT], first_level = hdr[H_LEVEL];
+  const int* from = hdr[H_SIDE] ? list_b : list_a;
+  int* over = hdr[H_SIDE] ? list_a : list_b;
+  if (first_level >= kWideMaxLevels) return;
+  // (a level below kWideSplit nodes has fewer than 4 kWideSplit children, a few each workgroup)
+  int m = 0;
+  for (int t = blockIdx.x; t < total && m < kWideList; t += gridDim.x) ++m;
+  for (int t = threadIdx.x; t < m; t += 64) lists[0][t] = from[blockIdx.x + t * gridDim.x];
+  if (threadIdx.x == 0) cnt_next = 0;
+  __syncthreads();
+  int level = first_level;
+  for (; m > 0 && level < kWideMaxLevels; ++level) {
+    const int* cur = lists[(level - first_level) & 1];
+    int* nxt = lists[((level - first_level) & 1) ^ 1];
+    for (int t = threadIdx.x; t < m; t += 64) {
+      int ref[4];
+      const int cnt = wide_sah_node(nodes, n, wide, cur[t], ref);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        if (c < cnt && ref[c] >= 0 && ref[c] < n - 1) {
+          const int slot = atomicAdd(&cnt_next, 1);
+          if (slot < kWideList) {
+            nxt[slot] = ref[c];
+          } else {
+            const int o = atomicAdd(hdr + H_OVER, 1);
+            if (o < n - 1) over[o] = ref[c];
+            atomicMax(hdr + H_OVER_LEVEL, level + 1);
+          }
+        }
+      }
+    }
+    __syncthreads();
+    m = cnt_next < kWideList ? cnt_next : kWideList;
+    __syncthreads();
+    if (threadIdx.x == 0) cnt_next = 0;
+    __syncthreads();
+  }
+  if (threadIdx.x == 0 && m > 0 && err) *err = 3;
 }
 
 // ---------------------------------------------------------------------------- PLOC
@@ -552,38 +787,57 @@ __global__ void __launch_bounds__(kWideBS) k_bvh_wide_sah(const BvhNode* __restr
 // the survivors are compacted in order, and the rounds repeat until one cluster is left. Node
 // indices count down from n-2, so the last merge is the root, node 0, as in the Morton tree.
 // Builds a tree closer to a surface-area-optimal one than the Morton split. The first rounds
-// run as grid-wide launches; the remaining few thousand clusters are finished by one workgroup
-// in a single launch. If the rounds do not get down to one cluster the Morton tree is kept.
+// are one grid-wide launch each; the remaining few thousand clusters are finished by one
+// workgroup with the clusters in LDS. If the rounds do not get down to one cluster the Morton
+// tree is built after all.
 constexpr int kPlocRadius = 16;
-constexpr int kPlocRounds = 6;          // rounds as grid-wide launches (the big early rounds)
+constexpr int kPlocTile = kBS;          // clusters of one workgroup of a grid-wide round
+constexpr int kPlocMaxRounds = 40;      // grid-wide rounds at most
 constexpr int kPlocFinishRounds = 512;  // then one workgroup finishes the (small) rest
+constexpr int kFinBS = 1024;
+constexpr int kFinCap = 2048;           // clusters that the finishing workgroup holds in LDS
 
-struct PlocWork {
-  int *ca, *cb;     // cluster refs (>= 0 node, < 0 leaf ~slot), ping-pong
-  float4 *ba, *bb;  // cluster boxes (lo, hi) as two float4 per cluster, ping-pong
-  int *nn, *valid, *pos;
-  int* cnt;         // cluster counts, one slot per round parity
-  int* alloc;       // merges so far
-  BvhNode* nodes;   // the clustered tree
+// The clusters between two rounds: tile t's survivors, in order, at [t kPlocTile, + cnt[t]), so
+// that no round needs a compaction of its own; sup[u] sums the counts of 256 tiles.
+struct PlocSet {
+  float4 *lo, *hi;  // cluster boxes
+  int* ref;         // >= 0 node, < 0 leaf ~slot
+  int *cnt, *sup;
 };
 
-size_t ploc_bytes(int cap) {
-  return (size_t)cap * (4 + 4 + 32 + 32 + 4 + 4 + 4) + (size_t)cap * sizeof(BvhNode) + 4096;
+struct PlocWork {
+  PlocSet set[2];
+  int* sup;         // the sums of every round, ns each
+  int* nn;
+  int* alloc;       // merges so far
+  int tiles, ns;
+};
+
+size_t ploc_tiles(int nf) { return ((size_t)nf + kPlocTile - 1) / kPlocTile; }
+
+size_t ploc_bytes(int nf) {
+  const size_t t = ploc_tiles(nf), ns = (t + 255) / 256;
+  return t * kPlocTile * (2 * 36 + 4) + 2 * t * 4 + (kPlocMaxRounds + 1) * ns * 4 + 64;
 }
 
-PlocWork ploc_carve(void* base, int cap) {
-  char* p = (char*)base;
+PlocWork ploc_carve(void* base, int nf) {
   PlocWork w;
-  w.ba = (float4*)p; p += (size_t)cap * 32;
-  w.bb = (float4*)p; p += (size_t)cap * 32;
-  w.nodes = (BvhNode*)p; p += (size_t)cap * sizeof(BvhNode);
-  w.ca = (int*)p; p += (size_t)cap * 4;
-  w.cb = (int*)p; p += (size_t)cap * 4;
-  w.nn = (int*)p; p += (size_t)cap * 4;
-  w.valid = (int*)p; p += (size_t)cap * 4;
-  w.pos = (int*)p; p += (size_t)cap * 4;
-  w.cnt = (int*)p; p += 64;
+  const size_t t = ploc_tiles(nf), cap = t * kPlocTile, ns = (t + 255) / 256;
+  char* p = (char*)base;
+  for (PlocSet& q : w.set) {
+    q.lo = (float4*)p; p += cap * 16;
+    q.hi = (float4*)p; p += cap * 16;
+  }
+  for (PlocSet& q : w.set) {
+    q.ref = (int*)p; p += cap * 4;
+    q.cnt = (int*)p; p += t * 4;
+    q.sup = nullptr;
+  }
+  w.nn = (int*)p; p += cap * 4;
+  w.sup = (int*)p; p += (kPlocMaxRounds + 1) * ns * 4;
   w.alloc = (int*)p;
+  w.tiles = (int)t;
+  w.ns = (int)ns;
   return w;
 }
 
@@ -594,196 +848,291 @@ __device__ __forceinline__ float union_area(float4 alo, float4 ahi, float4 blo, 
   return x * y + y * z + z * x;
 }
 
-__global__ void k_ploc_init(const float4* __restrict__ tris, int n, int* __restrict__ ca,
-                            float4* __restrict__ ba, int* __restrict__ cnt,
-                            int* __restrict__ alloc) {
+// The leaves as clusters; sup: the first round's sums, then `rounds` rounds' to be added to.
+__global__ void __launch_bounds__(kBS) k_ploc_init(const float4* __restrict__ tris, int n,
+                                                   PlocSet out, int tiles, int ns, int rounds,
+                                                   int* __restrict__ sup, int* __restrict__ alloc) {
   const int i = blockIdx.x * kBS + threadIdx.x;
-  if (i == 0) {
-    cnt[0] = n;
-    cnt[1] = n;
-    *alloc = 0;
+  if (i == 0) *alloc = 0;
+  for (long long k = i; k < (long long)(rounds + 1) * ns; k += (long long)gridDim.x * kBS) {
+    const long long left = n - k * 256 * kPlocTile;
+    sup[k] = k >= ns ? 0 : (int)(left < 256 * kPlocTile ? left : 256 * kPlocTile);
   }
+  if (i < tiles) out.cnt[i] = n - i * kPlocTile < kPlocTile ? n - i * kPlocTile : kPlocTile;
   if (i >= n) return;
   const float4 a = tris[3 * i], b = tris[3 * i + 1], c = tris[3 * i + 2];
-  ca[i] = ~i;
-  ba[2 * i] = make_float4(fminf(a.x, fminf(b.x, c.x)), fminf(a.y, fminf(b.y, c.y)),
+  out.ref[i] = ~i;
+  out.lo[i] = make_float4(fminf(a.x, fminf(b.x, c.x)), fminf(a.y, fminf(b.y, c.y)),
                           fminf(a.z, fminf(b.z, c.z)), 0.f);
-  ba[2 * i + 1] = make_float4(fmaxf(a.x, fmaxf(b.x, c.x)), fmaxf(a.y, fmaxf(b.y, c.y)),
-                              fmaxf(a.z, fmaxf(b.z, c.z)), 0.f);
+  out.hi[i] = make_float4(fmaxf(a.x, fmaxf(b.x, c.x)), fmaxf(a.y, fmaxf(b.y, c.y)),
+                          fmaxf(a.z, fmaxf(b.z, c.z)), 0.f);
 }
 
-__global__ void k_ploc_nn(const float4* __restrict__ ba, const int* __restrict__ cnt,
-                          int* __restrict__ nn) {
-  const int count = *cnt;
-  const int i = blockIdx.x * kBS + threadIdx.x;
-  if (i >= count || count <= 1) return;
-  const float4 lo = ba[2 * i], hi = ba[2 * i + 1];
+// The nearest cluster of cluster q among [0, count) (lo, hi: cluster `first` onwards), by lane l
+// of the `sub` lanes that share the search; ties keep the smaller index.
+__device__ __forceinline__ int ploc_nearest(const float4* lo, const float4* hi, int first, int q,
+                                            int count, int l, int sub) {
+  const float4 qlo = lo[q - first], qhi = hi[q - first];
   int best = -1;
   float best_a = INFINITY;
-  const int j0 = i - kPlocRadius < 0 ? 0 : i - kPlocRadius;
-  const int j1 = i + kPlocRadius > count - 1 ? count - 1 : i + kPlocRadius;
-  for (int j = j0; j <= j1; ++j) {
-    if (j == i) continue;
-    const float a = union_area(lo, hi, ba[2 * j], ba[2 * j + 1]);
-    if (a < best_a) {  // ties keep the smaller index (j ascends)
+  const int j0 = q - kPlocRadius < 0 ? 0 : q - kPlocRadius;
+  const int j1 = q + kPlocRadius > count - 1 ? count - 1 : q + kPlocRadius;
+#pragma unroll 4
+  for (int j = j0 + l; j <= j1; j += sub) {
+    const float a = union_area(qlo, qhi, lo[j - first], hi[j - first]);
+    if (j != q && a < best_a) {
       best_a = a;
       best = j;
     }
   }
-  nn[i] = best;
-}
-
-__global__ void k_ploc_merge(int* __restrict__ ca, float4* __restrict__ ba,
-                             const int* __restrict__ nn, const int* __restrict__ cnt,
-                             int* __restrict__ valid, int n_max, BvhNode* __restrict__ nodes,
-                             int* __restrict__ alloc, int n) {
-  const int i = blockIdx.x * kBS + threadIdx.x;
-  if (i >= n_max) return;
-  const int count = *cnt;
-  if (i >= count) {
-    valid[i] = 0;
-    return;
-  }
-  if (count <= 1) {
-    valid[i] = 1;
-    return;
-  }
-  const int j = nn[i];
-  if (j < 0 || j >= count || nn[j] != i) {  // not a mutual pair: the cluster survives
-    valid[i] = 1;
-    return;
-  }
-  if (i > j) {  // the smaller index of the pair builds the node and keeps its slot
-    valid[i] = 0;
-    return;
-  }
-  const int node = (n - 2) - atomicAdd(alloc, 1);
-  if (node < 0) {  // more merges than a binary tree has nodes: cannot happen; drop the pair
-    valid[i] = 1;
-    return;
-  }
-  const float4 l0 = ba[2 * i], l1 = ba[2 * i + 1], r0 = ba[2 * j], r1 = ba[2 * j + 1];
-  BvhNode nd;
-  nd.a = make_float4(l0.x, l0.y, l0.z, l1.x);
-  nd.b = make_float4(l1.y, l1.z, r0.x, r0.y);
-  nd.c = make_float4(r0.z, r1.x, r1.y, r1.z);
-  nd.d = make_int4(ca[i], ca[j], 0, 0);
-  nodes[node] = nd;
-  ca[i] = node;
-  ba[2 * i] = make_float4(fminf(l0.x, r0.x), fminf(l0.y, r0.y), fminf(l0.z, r0.z), 0.f);
-  ba[2 * i + 1] = make_float4(fmaxf(l1.x, r1.x), fmaxf(l1.y, r1.y), fmaxf(l1.z, r1.z), 0.f);
-  valid[i] = 1;
-}
-
-__global__ void k_ploc_scatter(const int* __restrict__ ca, const float4* __restrict__ ba,
-                               const int* __restrict__ valid, const int* __restrict__ pos,
-                               const int* __restrict__ cnt, int* __restrict__ cb,
-                               float4* __restrict__ bb) {
-  const int i = blockIdx.x * kBS + threadIdx.x;
-  if (i >= *cnt || !valid[i]) return;
-  const int k = pos[i];
-  cb[k] = ca[i];
-  bb[2 * k] = ba[2 * i];
-  bb[2 * k + 1] = ba[2 * i + 1];
-}
-
-// The remaining rounds in one workgroup: the same nearest-neighbour, merge and in-order
-// compaction steps, separated by workgroup barriers instead of launches.
-constexpr int kFinBS = 1024;
-
-__global__ void __launch_bounds__(kFinBS) k_ploc_finish(int* __restrict__ ca,
-                                                        float4* __restrict__ ba,
-                                                        int* __restrict__ cb,
-                                                        float4* __restrict__ bb,
-                                                        int* __restrict__ nn,
-                                                        int* __restrict__ valid,
-                                                        int* __restrict__ cnt,
-                                                        BvhNode* __restrict__ nodes,
-                                                        int* __restrict__ alloc, int n) {
-  __shared__ int s_count;
-  if (threadIdx.x == 0) s_count = *cnt;
-  __syncthreads();
-  int* A = ca;
-  float4* AB = ba;
-  int* B = cb;
-  float4* BB = bb;
-  for (int round = 0; round < kPlocFinishRounds; ++round) {
-    const int count = s_count;
-    if (count <= 1) break;
-    for (int i = threadIdx.x; i < count; i += kFinBS) {
-      const float4 lo = AB[2 * i], hi = AB[2 * i + 1];
-      int best = -1;
-      float best_a = INFINITY;
-      const int j0 = i - kPlocRadius < 0 ? 0 : i - kPlocRadius;
-      const int j1 = i + kPlocRadius > count - 1 ? count - 1 : i + kPlocRadius;
-      for (int j = j0; j <= j1; ++j) {
-        if (j == i) continue;
-        const float a = union_area(lo, hi, AB[2 * j], AB[2 * j + 1]);
-        if (a < best_a) {
-          best_a = a;
-          best = j;
-        }
-      }
-      nn[i] = best;
+  for (int d = sub >> 1; d >= 1; d >>= 1) {
+    const float oa = __shfl_xor(best_a, d, 64);
+    const int oj = __shfl_xor(best, d, 64);
+    if (oj >= 0 && (best < 0 || oa < best_a || (oa == best_a && oj < best))) {
+      best_a = oa;
+      best = oj;
     }
-    __syncthreads();
-    for (int i = threadIdx.x; i < count; i += kFinBS) {
-      const int j = nn[i];
-      if (j < 0 || j >= count || nn[j] != i) {
-        valid[i] = 1;
-        continue;
-      }
-      if (i > j) {
-        valid[i] = 0;
-        continue;
-      }
-      const int node = (n - 2) - atomicAdd(alloc, 1);
-      if (node < 0) {
-        valid[i] = 1;
-        continue;
-      }
-      const float4 l0 = AB[2 * i], l1 = AB[2 * i + 1], r0 = AB[2 * j], r1 = AB[2 * j + 1];
-      BvhNode nd;
-      nd.a = make_float4(l0.x, l0.y, l0.z, l1.x);
-      nd.b = make_float4(l1.y, l1.z, r0.x, r0.y);
-      nd.c = make_float4(r0.z, r1.x, r1.y, r1.z);
-      nd.d = make_int4(A[i], A[j], 0, 0);
-      nodes[node] = nd;
-      A[i] = node;
-      AB[2 * i] = make_float4(fminf(l0.x, r0.x), fminf(l0.y, r0.y), fminf(l0.z, r0.z), 0.f);
-      AB[2 * i + 1] = make_float4(fmaxf(l1.x, r1.x), fmaxf(l1.y, r1.y), fmaxf(l1.z, r1.z), 0.f);
-      valid[i] = 1;
+  }
+  return best;
+}
+
+__device__ __forceinline__ void ploc_node(BvhNode* nd, float4 l0, float4 l1, float4 r0, float4 r1,
+                                          int left, int right) {
+  nd->a = make_float4(l0.x, l0.y, l0.z, l1.x);
+  nd->b = make_float4(l1.y, l1.z, r0.x, r0.y);
+  nd->c = make_float4(r0.z, r1.x, r1.y, r1.z);
+  nd->d = make_int4(left, right, 0, 0);
+}
+
+__device__ __forceinline__ float4 min4(float4 a, float4 b) {
+  return make_float4(fminf(a.x, b.x), fminf(a.y, b.y), fminf(a.z, b.z), 0.f);
+}
+__device__ __forceinline__ float4 max4(float4 a, float4 b) {
+  return make_float4(fmaxf(a.x, b.x), fmaxf(a.y, b.y), fmaxf(a.z, b.z), 0.f);
+}
+
+// One round, one launch: workgroup b takes the clusters [b kPlocTile, (b + 1) kPlocTile) of all
+// that are left. It finds where they lie from the tiles' counts, stages them with 2 kPlocRadius
+// neighbours each side in LDS, finds the nearest of its own and of kPlocRadius each side (which
+// tells whether its own pairs are mutual), merges, and leaves its survivors packed in its tile.
+// 10 us a round at 47k faces, half of it the chain of fetches that finds the clusters (25 us as
+// nearest, merge, scan and scatter launches through memory).
+// A full tile keeps at least 120 of its 256 (at most 16 go to the tile before it, the others in
+// pairs), so the 320 staged clusters lie in at most 5 tiles.
+constexpr int kPlocWin = kPlocTile + 4 * kPlocRadius;   // and threads: one a staged cluster
+constexpr int kPlocSpan = 8;
+__global__ void __launch_bounds__(kPlocWin) k_ploc_round(PlocSet in, PlocSet out, int tiles, int ns,
+                                                    BvhNode* __restrict__ nodes,
+                                                    int* __restrict__ alloc, int n) {
+  __shared__ float4 s_lo[kPlocWin], s_hi[kPlocWin];
+  __shared__ int s_ref[kPlocWin], s_nn[kPlocTile + 2 * kPlocRadius];
+  __shared__ int s_at[3], s_pre[kPlocSpan + 1];
+  const int tid = threadIdx.x, b0 = blockIdx.x * kPlocTile;
+  const int start = b0 < 2 * kPlocRadius ? 0 : b0 - 2 * kPlocRadius;
+  int total = 0;
+  for (int c = 0; c < ns; c += kPlocWin) {
+    const int v = c + tid < ns ? in.sup[c + tid] : 0;
+    int sum;
+    const int ex = total + petch::block_excl_scan<kPlocWin>(v, sum);
+    if (start >= ex && start < ex + v) {
+      s_at[0] = c + tid;
+      s_at[1] = ex;
+    }
+    total += sum;
+  }
+  if (b0 >= total) {
+    if (tid == 0) out.cnt[blockIdx.x] = 0;
+    return;
+  }
+  __syncthreads();
+  {
+    const int t = s_at[0] * 256 + tid;
+    const int v = tid < 256 && t < tiles ? in.cnt[t] : 0;
+    int sum;
+    const int ex = s_at[1] + petch::block_excl_scan<kPlocWin>(v, sum);
+    if (start >= ex && start < ex + v) {
+      s_at[2] = t;
+      s_pre[0] = ex;
+    }
+  }
+  __syncthreads();
+  const int t0 = s_at[2];
+  if (tid == 0) {
+#pragma unroll
+    for (int k = 0; k < kPlocSpan; ++k)
+      s_pre[k + 1] = s_pre[k] + (t0 + k < tiles ? in.cnt[t0 + k] : 0);
+  }
+  __syncthreads();
+  const int past = b0 + kPlocTile + 2 * kPlocRadius, end = total < past ? total : past;
+  if (const int q = start + tid; q < end) {
+    int k = 0;
+    while (k < kPlocSpan - 1 && q >= s_pre[k + 1]) ++k;
+    const int src = (t0 + k) * kPlocTile + (q - s_pre[k]);
+    if (src < tiles * kPlocTile) {
+      s_lo[q - start] = in.lo[src];
+      s_hi[q - start] = in.hi[src];
+      s_ref[q - start] = in.ref[src];
+    }
+  }
+  __syncthreads();
+  const int n0 = b0 < kPlocRadius ? 0 : b0 - kPlocRadius;
+  const int n1 = total < b0 + kPlocTile + kPlocRadius ? total : b0 + kPlocTile + kPlocRadius;
+  if (const int q = n0 + tid; q < n1)
+    s_nn[q - n0] = ploc_nearest(s_lo, s_hi, start, q, total, 0, 1);
+  __syncthreads();
+  const int i = b0 + tid;
+  const bool own = tid < kPlocTile && i < total;
+  const int j = own ? s_nn[i - n0] : -1;
+  const bool mutual = j >= 0 && s_nn[j - n0] == i;
+  const bool merge = mutual && i < j;                 // the smaller index builds the node
+  const bool keep = own && !(mutual && i > j);  // and keeps its place
+  int sum;
+  const int ex = petch::block_excl_scan<kPlocWin>((keep ? 1 : 0) | (merge ? 0x10000 : 0), sum);
+  if (tid == 0) {
+    out.cnt[blockIdx.x] = sum & 0xffff;
+    atomicAdd(out.sup + (blockIdx.x >> 8), sum & 0xffff);
+    s_at[0] = atomicAdd(alloc, sum >> 16);
+  }
+  __syncthreads();
+  if (!keep) return;
+  float4 lo = s_lo[i - start], hi = s_hi[i - start];
+  int ref = s_ref[i - start];
+  if (merge) {
+    const int node = (n - 2) - (s_at[0] + (ex >> 16));
+    const float4 rlo = s_lo[j - start], rhi = s_hi[j - start];
+    if (node >= 0) ploc_node(nodes + node, lo, hi, rlo, rhi, ref, s_ref[j - start]);
+    lo = min4(lo, rlo);
+    hi = max4(hi, rhi);
+    ref = node;
+  }
+  const int o = b0 + (ex & 0xffff);   // at most 256 kept: within the tile
+  out.lo[o] = lo;
+  out.hi[o] = hi;
+  out.ref[o] = ref;
+}
+
+// Rounds of one workgroup over clusters [0, count) at lo, hi, ref, compacted in place, until at
+// most `stop` are left or `rounds` is spent. With few clusters several lanes share a search.
+__device__ __forceinline__ void ploc_rounds(float4* lo, float4* hi, int* ref, int* nn, int& count,
+                                            int stop, int& rounds, int& merged, BvhNode* nodes,
+                                            int n) {
+  const int tid = threadIdx.x;
+  for (; rounds > 0 && count > stop; --rounds) {
+    int sub = 16;
+    while (sub > 1 && count * sub > kFinBS) sub >>= 1;
+    for (int i = tid / sub; i < count; i += kFinBS / sub) {
+      const int j = ploc_nearest(lo, hi, 0, i, count, tid % sub, sub);
+      if (tid % sub == 0) nn[i] = j;
     }
     __syncthreads();
     int carry = 0;
     for (int base = 0; base < count; base += kFinBS) {
-      const int i = base + threadIdx.x;
-      const int v = i < count ? valid[i] : 0;
-      int tot;
-      const int ex = petch::block_excl_scan<kFinBS>(v, tot);
-      if (v) {
-        const int k = carry + ex;
-        B[k] = A[i];
-        BB[2 * k] = AB[2 * i];
-        BB[2 * k + 1] = AB[2 * i + 1];
+      const int i = base + tid;
+      const int j = i < count ? nn[i] : -1;
+      const bool mutual = j >= 0 && nn[j] == i;
+      const bool merge = mutual && i < j;
+      const bool keep = i < count && !(mutual && i > j);
+      float4 l0, l1, r0, r1;
+      int ri = 0, rj = 0;
+      if (keep) {
+        l0 = lo[i];
+        l1 = hi[i];
+        ri = ref[i];
       }
-      carry += tot;
+      if (merge) {
+        r0 = lo[j];
+        r1 = hi[j];
+        rj = ref[j];
+      }
+      // (the scan's barriers part these reads from the writes below, which stay below base +
+      // kFinBS: nothing that a later pass reads)
+      int sum;
+      const int ex = petch::block_excl_scan<kFinBS>((keep ? 1 : 0) | (merge ? 0x10000 : 0), sum);
+      if (merge) {
+        const int node = (n - 2) - (merged + (ex >> 16));
+        if (node >= 0) ploc_node(nodes + node, l0, l1, r0, r1, ri, rj);
+        l0 = min4(l0, r0);
+        l1 = max4(l1, r1);
+        ri = node;
+      }
+      if (keep) {
+        const int k = carry + (ex & 0xffff);
+        lo[k] = l0;
+        hi[k] = l1;
+        ref[k] = ri;
+      }
+      carry += sum & 0xffff;
+      merged += sum >> 16;
     }
     __syncthreads();
-    if (threadIdx.x == 0) s_count = carry;
-    __syncthreads();
-    int* ti = A; A = B; B = ti;
-    float4* tf = AB; AB = BB; BB = tf;
+    count = carry;
   }
-  if (threadIdx.x == 0) *cnt = s_count;
 }
 
-// Adopts the clustered tree when it is complete (one cluster left after n-1 merges).
-__global__ void k_ploc_commit(const BvhNode* __restrict__ src, const int* __restrict__ cnt,
-                              const int* __restrict__ alloc, int n,
-                              BvhNode* __restrict__ dst) {
-  if (*cnt != 1 || *alloc != n - 1) return;
-  for (int k = blockIdx.x * kBS + threadIdx.x; k < n - 1; k += gridDim.x * kBS) dst[k] = src[k];
+// The remaining rounds in one workgroup, the clusters packed into LDS (through memory, at buf,
+// while there are more than fit). Its 27 rounds are bound by LDS latency and barriers: 93 us for
+// 47k faces (685 through memory, from 9k clusters on). *done: the tree is complete, and root its
+// box.
+__global__ void __launch_bounds__(kFinBS) k_ploc_finish(PlocSet in, PlocSet buf, int tiles, int ns,
+                                                        int* __restrict__ nn,
+                                                        BvhNode* __restrict__ nodes,
+                                                        const int* __restrict__ alloc, int n,
+                                                        int* __restrict__ done,
+                                                        float* __restrict__ root) {
+  __shared__ float4 s_lo[kFinCap], s_hi[kFinCap];
+  __shared__ int s_ref[kFinCap], s_nn[kFinCap];
+  __shared__ int s_pre[kFinBS], s_cnt[kFinBS];
+  const int tid = threadIdx.x;
+  int count = 0;
+  for (int k = tid; k < ns; k += kFinBS) count += in.sup[k];
+  count = petch::block_sum<kFinBS>(count);
+  const bool fits = count <= kFinCap;
+  int carry = 0;
+  for (int c = 0; c < tiles && carry < count; c += kFinBS) {
+    const int v = c + tid < tiles ? in.cnt[c + tid] : 0;
+    int sum;
+    s_pre[tid] = carry + petch::block_excl_scan<kFinBS>(v, sum);
+    s_cnt[tid] = v;
+    carry += sum;
+    __syncthreads();
+    for (int t = tid / kPlocTile; t < kFinBS && s_pre[t] < carry; t += kFinBS / kPlocTile) {
+      const int k = tid % kPlocTile;
+      if (k < s_cnt[t]) {
+        const int src = (c + t) * kPlocTile + k, o = s_pre[t] + k;
+        if (fits) {
+          s_lo[o] = in.lo[src];
+          s_hi[o] = in.hi[src];
+          s_ref[o] = in.ref[src];
+        } else {
+          buf.lo[o] = in.lo[src];
+          buf.hi[o] = in.hi[src];
+          buf.ref[o] = in.ref[src];
+        }
+      }
+    }
+    __syncthreads();
+  }
+  int rounds = kPlocFinishRounds, merged = *alloc;
+  if (!fits) {
+    ploc_rounds(buf.lo, buf.hi, buf.ref, nn, count, kFinCap, rounds, merged, nodes, n);
+    if (count <= kFinCap) {
+      for (int k = tid; k < count; k += kFinBS) {
+        s_lo[k] = buf.lo[k];
+        s_hi[k] = buf.hi[k];
+        s_ref[k] = buf.ref[k];
+      }
+    }
+    __syncthreads();
+  }
+  if (count <= kFinCap) ploc_rounds(s_lo, s_hi, s_ref, s_nn, count, 1, rounds, merged, nodes, n);
+  if (tid == 0) {
+    const bool whole = count == 1 && merged == n - 1;
+    *done = whole;
+    if (whole) {
+      root[0] = s_lo[0].x; root[1] = s_lo[0].y; root[2] = s_lo[0].z;
+      root[3] = s_hi[0].x; root[4] = s_hi[0].y; root[5] = s_hi[0].z;
+    }
+  }
 }
 
 __global__ void k_query_ray(BvhView b, const float* __restrict__ o, const float* __restrict__ d,
@@ -867,9 +1216,9 @@ extern "C" int petch_bvh_destroy(petch_ctx* ctx, petch_bvh* b) {
 
 namespace {
 
-// PLOC rounds over the leaves of b (tris already in Morton order); the result replaces b's
-// Morton tree only when it is complete.
-int ploc_build(petch_ctx* ctx, petch_bvh* b, int nf) {
+// PLOC rounds over the leaves of b (tris already in Morton order) into b->nodes; *done, on the
+// device, tells whether they hold a complete tree.
+int ploc_build(petch_ctx* ctx, petch_bvh* b, int nf, int* done, float* root) {
   const size_t need = ploc_bytes(nf);
   if (b->aux_cap < need) {
     PETCH_HIP(ctx, hipStreamSynchronize(ctx->stream));
@@ -881,34 +1230,25 @@ int ploc_build(petch_ctx* ctx, petch_bvh* b, int nf) {
     b->aux_cap = want;
   }
   PlocWork p = ploc_carve(b->aux, nf);
-  const unsigned g = petch_blocks(nf, kBS);
+  // the first round keeps about 0.57 of its clusters (most leaves pair up), each later one 0.81:
+  // as many as bring them into the finishing workgroup's LDS
+  int rounds = nf > kFinCap ? 1 : 0;
+  for (long long c = nf * 9LL / 16; c > kFinCap && rounds < kPlocMaxRounds; c -= c * 3 / 16)
+    ++rounds;
+  const unsigned g = (unsigned)p.tiles;
+  p.set[0].sup = p.sup;
   hipLaunchKernelGGL(k_ploc_init, dim3(g), dim3(kBS), 0, ctx->stream, (const float4*)b->tris, nf,
-                     p.ca, p.ba, p.cnt, p.alloc);
+                     p.set[0], p.tiles, p.ns, rounds, p.sup, p.alloc);
   PETCH_LAUNCH_CHECK(ctx);
-  int *ca = p.ca, *cb = p.cb;
-  float4 *ba = p.ba, *bb = p.bb;
-  for (int r = 0; r < kPlocRounds; ++r) {
-    int* cur = p.cnt + (r & 1);
-    int* nxt = p.cnt + ((r + 1) & 1);
-    hipLaunchKernelGGL(k_ploc_nn, dim3(g), dim3(kBS), 0, ctx->stream, ba, cur, p.nn);
+  for (int r = 0; r < rounds; ++r) {
+    p.set[(r + 1) & 1].sup = p.sup + (size_t)(r + 1) * p.ns;
+    hipLaunchKernelGGL(k_ploc_round, dim3(g), dim3(kPlocWin), 0, ctx->stream, p.set[r & 1],
+                       p.set[(r + 1) & 1], p.tiles, p.ns, (BvhNode*)b->nodes, p.alloc, nf);
     PETCH_LAUNCH_CHECK(ctx);
-    hipLaunchKernelGGL(k_ploc_merge, dim3(g), dim3(kBS), 0, ctx->stream, ca, ba, p.nn, cur,
-                       p.valid, nf, p.nodes, p.alloc, nf);
-    PETCH_LAUNCH_CHECK(ctx);
-    int rc = petch_exclusive_scan(ctx, p.valid, p.pos, nf, nxt);
-    if (rc != PETCH_OK) return rc;
-    hipLaunchKernelGGL(k_ploc_scatter, dim3(g), dim3(kBS), 0, ctx->stream, ca, ba, p.valid,
-                       p.pos, cur, cb, bb);
-    PETCH_LAUNCH_CHECK(ctx);
-    int* ti = ca; ca = cb; cb = ti;
-    float4* tf = ba; ba = bb; bb = tf;
   }
-  int* cnt = p.cnt + (kPlocRounds & 1);
-  hipLaunchKernelGGL(k_ploc_finish, dim3(1), dim3(kFinBS), 0, ctx->stream, ca, ba, cb, bb, p.nn,
-                     p.valid, cnt, p.nodes, p.alloc, nf);
-  PETCH_LAUNCH_CHECK(ctx);
-  hipLaunchKernelGGL(k_ploc_commit, dim3(g < 256 ? g : 256), dim3(kBS), 0, ctx->stream, p.nodes,
-                     cnt, p.alloc, nf, (BvhNode*)b->nodes);
+  hipLaunchKernelGGL(k_ploc_finish, dim3(1), dim3(kFinBS), 0, ctx->stream, p.set[rounds & 1],
+                     p.set[(rounds + 1) & 1], p.tiles, p.ns, p.nn, (BvhNode*)b->nodes, p.alloc, nf,
+                     done, root);
   PETCH_LAUNCH_CHECK(ctx);
   return PETCH_OK;
 }
@@ -947,8 +1287,14 @@ int ensure_capacity(petch_ctx* ctx, petch_bvh* b, int nf) {
   return PETCH_OK;
 }
 
-// Everything of a build up to the refit: buffers, centroids, Morton sort, leaves, Karras nodes
-// and the cleared refit flags. Returns the refit's item (n = nf; nothing to refit when nf < 2).
+// The quality a build of nf faces gets.
+int build_quality(const petch_bvh* b, int nf) {
+  return b->quality >= 0 ? b->quality : (nf >= kWideSahMinFaces ? 2 : 0);
+}
+
+// Everything of a build up to the refit: buffers, centroids, Morton sort, leaves, then the
+// clustered tree where the quality asks for it and the Morton tree's nodes where that one isn't
+// complete. Returns the refit's item (n = nf; nothing to refit when nf < 2).
 int build_prepare(petch_ctx* ctx, petch_bvh* b, const float* verts, const int* faces, int nv,
                   int nf, RefitItem* refit) {
   PETCH_ARG(ctx, ctx && b, "bvh_build: null pointer");
@@ -978,30 +1324,49 @@ int build_prepare(petch_ctx* ctx, petch_bvh* b, const float* verts, const int* f
                      (float4*)b->tris);
   PETCH_LAUNCH_CHECK(ctx);
   if (nf > 1) {
+    const int* done = nullptr;
+    if (build_quality(b, nf) >= 2) {
+      rc = ploc_build(ctx, b, nf, w.hdr + H_DONE, w.root);
+      if (rc != PETCH_OK) return rc;
+      done = w.hdr + H_DONE;
+    }
     hipLaunchKernelGGL(k_bvh_karras, dim3(petch_blocks(nf - 1, kBS)), dim3(kBS), 0, ctx->stream,
-                       w.keys, nf, (BvhNode*)b->nodes, w.pint, w.pleaf);
+                       w.keys, nf, (BvhNode*)b->nodes, w.pint, w.pleaf, done);
     PETCH_LAUNCH_CHECK(ctx);
-    PETCH_HIP(ctx, hipMemsetAsync(w.flags, 0, (size_t)nf * sizeof(int), ctx->stream));
-    *refit = RefitItem{(const float4*)b->tris, (BvhNode*)b->nodes, w.pint, w.pleaf, w.flags,
-                       w.root, nf};
+    *refit = RefitItem{(const float4*)b->tris, (BvhNode*)b->nodes, w.pint, w.pleaf,
+                       (float*)b->wide, w.root, done, nf, 0};
   }
   return PETCH_OK;
 }
 
-// The rest of a build after the refit: the clustered tree where the quality asks for it, then
-// the 4-wide nodes the ray queries walk.
+int build_refit(petch_ctx* ctx, const RefitItem& r) {
+  if (r.n < 2) return PETCH_OK;
+  const unsigned g = petch_blocks(r.n, kTile);
+  hipLaunchKernelGGL(k_bvh_refit_tile, dim3(g), dim3(kBS), 0, ctx->stream, r);
+  PETCH_LAUNCH_CHECK(ctx);
+  if (g > 1) {
+    hipLaunchKernelGGL(k_bvh_refit_span, dim3(g), dim3(kBS), 0, ctx->stream, r);
+    PETCH_LAUNCH_CHECK(ctx);
+  }
+  return PETCH_OK;
+}
+
+// The rest of a build after the refit: the 4-wide nodes that the queries walk.
 int build_finish(petch_ctx* ctx, petch_bvh* b, int nf) {
   if (nf > 1) {
     Work w = carve(b->work, b->cap_f);
-    const int q = b->quality >= 0 ? b->quality : (nf >= kWideSahMinFaces ? 2 : 0);
-    if (q >= 2) {
-      int rc2 = ploc_build(ctx, b, nf);
-      if (rc2 != PETCH_OK) return rc2;
-    }
-    if (q >= 1) {
-      hipLaunchKernelGGL(k_bvh_wide_sah, dim3(1), dim3(kWideBS), 0, ctx->stream,
-                         (const BvhNode*)b->nodes, nf, (BvhWide*)b->wide, (int*)w.ktmp,
-                         (int*)w.vtmp, w.err);
+    if (build_quality(b, nf) >= 1) {
+      int *la = (int*)w.ktmp, *lb = (int*)w.vtmp;
+      const BvhNode* nodes = (const BvhNode*)b->nodes;
+      BvhWide* wide = (BvhWide*)b->wide;
+      hipLaunchKernelGGL(k_wide_levels, dim3(1), dim3(kWideBS), 0, ctx->stream, nodes, nf, wide,
+                         la, lb, w.hdr, w.err, true);
+      PETCH_LAUNCH_CHECK(ctx);
+      hipLaunchKernelGGL(k_wide_subtrees, dim3(kWideSplit), dim3(64), 0, ctx->stream, nodes, nf,
+                         wide, la, lb, w.hdr, w.err);
+      PETCH_LAUNCH_CHECK(ctx);
+      hipLaunchKernelGGL(k_wide_levels, dim3(1), dim3(kWideBS), 0, ctx->stream, nodes, nf, wide,
+                         la, lb, w.hdr, w.err, false);
     } else {
       hipLaunchKernelGGL(k_bvh_wide, dim3(petch_blocks(nf - 1, kBS)), dim3(kBS), 0, ctx->stream,
                          (const BvhNode*)b->nodes, w.pint, nf, (BvhWide*)b->wide);
@@ -1019,11 +1384,8 @@ extern "C" int petch_bvh_build(petch_ctx* ctx, petch_bvh* b, const float* verts,
   RefitItem r;
   int rc = build_prepare(ctx, b, verts, faces, nv, nf, &r);
   if (rc != PETCH_OK) return rc;
-  if (r.n > 1) {
-    hipLaunchKernelGGL(k_bvh_refit, dim3(petch_blocks(r.n, kBS)), dim3(kBS), 0, ctx->stream,
-                       r.tris, r.nodes, r.pint, r.pleaf, r.flags, r.n, r.root);
-    PETCH_LAUNCH_CHECK(ctx);
-  }
+  rc = build_refit(ctx, r);
+  if (rc != PETCH_OK) return rc;
   return build_finish(ctx, b, nf);
 }
 
@@ -1049,12 +1411,11 @@ extern "C" int petch_bvh_build_batch(petch_ctx* ctx, int n, petch_bvh* const* bv
   long long fb = 0, nb = 0, tiles = 0, tab = 0;
   for (int t = 0; t < n; ++t) {
     petch_bvh* b = bvhs[t];
-    const int q = b->quality >= 0 ? b->quality : (nf[t] >= kWideSahMinFaces ? 2 : 0);
-    if (q != 0 || nf[t] < 2) {
+    if (build_quality(b, nf[t]) != 0 || nf[t] < 2) {
       RefitItem r;
-      const int rc = build_prepare(ctx, b, verts[t], faces[t], nv[t], nf[t], &r);
+      int rc = build_prepare(ctx, b, verts[t], faces[t], nv[t], nf[t], &r);
+      if (rc == PETCH_OK) rc = build_refit(ctx, r);
       if (rc != PETCH_OK) return rc;
-      if (r.n > 1) refit.push_back(r);
       continue;
     }
     b->nv = nv[t];
@@ -1089,8 +1450,8 @@ extern "C" int petch_bvh_build_batch(petch_ctx* ctx, int n, petch_bvh* const* bv
     fast.push_back(it);
     sorts.push_back(si);
     fast_t.push_back(t);
-    refit.push_back(RefitItem{it.tris, it.nodes, it.w.pint, it.w.pleaf, it.w.flags, it.w.root,
-                              it.nf});
+    refit.push_back(RefitItem{it.tris, it.nodes, it.w.pint, it.w.pleaf, (float*)it.wide, it.w.root,
+                              nullptr, it.nf, it.fblk0});
   }
   PETCH_ARG(ctx, fb <= 0x7fffffffLL && tiles <= 0x7fffffffLL,
             "bvh_build_batch: too many faces for one launch");
@@ -1139,10 +1500,11 @@ extern "C" int petch_bvh_build_batch(petch_ctx* ctx, int n, petch_bvh* const* bv
     hipLaunchKernelGGL(k_bvh_karras_many, dim3((unsigned)nb), dim3(kBS), 0, ctx->stream, db, m);
     PETCH_LAUNCH_CHECK(ctx);
   }
-  hipLaunchKernelGGL(k_bvh_refit_wg, dim3((unsigned)refit.size()), dim3(kRefitWG), 0, ctx->stream,
-                     dr);
-  PETCH_LAUNCH_CHECK(ctx);
   if (m > 0) {
+    hipLaunchKernelGGL(k_bvh_refit_tile_many, dim3((unsigned)fb), dim3(kBS), 0, ctx->stream, dr, m);
+    PETCH_LAUNCH_CHECK(ctx);
+    hipLaunchKernelGGL(k_bvh_refit_span_many, dim3((unsigned)fb), dim3(kBS), 0, ctx->stream, dr, m);
+    PETCH_LAUNCH_CHECK(ctx);
     hipLaunchKernelGGL(k_bvh_wide_many, dim3((unsigned)nb), dim3(kBS), 0, ctx->stream, db, m);
     PETCH_LAUNCH_CHECK(ctx);
     for (int k = 0; k < m; ++k) bvhs[fast_t[k]]->nf = nf[fast_t[k]];

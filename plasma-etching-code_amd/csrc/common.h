@@ -71,8 +71,8 @@ struct petch_bvh {
   void* nodes;             // (nf-1) internal nodes, 64 B each: child AABBs + child refs
   void* wide;              // 4-wide nodes, 128 B each, at the indices of the binary nodes they replace
   void* tris;              // nf triangles in leaf order, 48 B each (v0, v1, v2 as float4)
-  void* work;              // build scratch: morton keys/values, parents, flags
-  void* aux;               // clustering scratch and tree of the large-mesh build
+  void* work;              // build scratch: morton keys/values, parents
+  void* aux;               // clustering scratch of the large-mesh build
   size_t aux_cap;
   size_t work_cap;
   int quality;             // build quality: -1 by mesh size, 0 Morton + fixed collapse,

@@ -148,3 +148,45 @@ def test_batched_build_equals_single_builds():
         pa, da = a.query_point(to)
         pb, db = b.query_point(to)
         assert torch.equal(pa, pb) and torch.equal(da, db)
+
+
+def _soup(nf, kind):
+    """Small triangles far apart for their size, so a triangle's centroid is nearest to itself."""
+    rng = np.random.default_rng(nf)
+    c = rng.uniform(-100, 100, (nf, 3))
+    size = np.full((nf, 1), 1e-3)
+    if kind == "cluster":          # three quarters inside one cell of the others' tree
+        k = 3 * nf // 4
+        d = rng.normal(size=(k, 3))
+        c[:k] = d / np.linalg.norm(d, axis=1, keepdims=True) * 0.5 * rng.uniform(size=(k, 1)) ** (1 / 3)
+        size[:k] = 2e-5
+    v = c[:, None] + size[:, None] * np.array([[1, 0, 0], [0, 1, 0], [0, 0, 1.0]])
+    return v.reshape(-1, 3).astype(np.float32), np.arange(3 * nf, dtype=np.int32).reshape(-1, 3)
+
+
+@pytest.mark.parametrize("quality", [0, 1, 2])
+@pytest.mark.parametrize("nf,kind", [(2, "even"), (3, "even"), (255, "even"), (256, "even"),
+                                     (257, "even"), (512, "even"), (513, "even"), (2048, "even"),
+                                     (2049, "even"), (4000, "cluster"), (66000, "even"),
+                                     (80000, "cluster")])
+def test_every_leaf_is_reached_at_the_edges_of_the_build_tiles(nf, kind, quality):
+    """Sizes at the edges of the refit's and the clustering's 256-leaf tiles and of the 2048
+    clusters that one workgroup finishes, and a dense cluster among spread-out triangles, whose
+    subtree outgrows one wavefront's list. The nearest face to a triangle's centroid is that
+    triangle, and the root box is the vertices' (single and batched builds)."""
+    import torch
+    from petch import ops
+    v, f = _soup(nf, kind)
+    dev = _dev()
+    tv, tf = torch.from_numpy(v).to(dev), torch.from_numpy(f).to(dev)
+    one = ops.Bvh(dev).set_quality(quality).build(tv, tf)
+    many = [ops.Bvh(dev).set_quality(quality) for _ in range(2)]
+    ops.bvh_build_batch([(b, tv, tf) for b in many])
+    pts = v.reshape(-1, 3, 3).astype(np.float64).mean(1).astype(np.float32)
+    for b in [one] + many:
+        face, _ = b.query_point(torch.from_numpy(pts).to(dev))
+        np.testing.assert_array_equal(face.cpu().numpy(), np.arange(nf))
+        assert b.status() == 0
+        lohi = b.root_bounds()
+        np.testing.assert_array_equal(lohi[:3], v.min(0))
+        np.testing.assert_array_equal(lohi[3:], v.max(0))
