@@ -210,6 +210,35 @@ def test_profile_area_and_its_adjoint_match_the_oracle():
     assert np.abs(got).max() > 0
 
 
+@pytest.mark.parametrize("shape", [(8, 8, 16), (9, 7, 17), (1, 1, 40), (3, 20, 1), (17, 16, 31),
+                                   (24, 25, 33)])
+def test_single_grid_sweeps_equal_brick_sweeps(shape):
+    """The last sweep of a single grid's reinit writes phi itself (none with no sweep), the batched
+    one's a pass after it; thin grids and every small number of substeps and sweeps give the same
+    bits."""
+    import torch
+    from petch import ops
+    rng = np.random.default_rng(sum(shape))
+    dx = 0.2
+    X = np.stack(np.meshgrid(*[np.arange(n) * dx for n in shape], indexing="ij"))
+    c = np.array(shape).reshape(3, 1, 1, 1) * dx / 2
+    phi = np.sqrt(((X - c) ** 2).sum(0)) - 0.3 * max(shape) * dx
+    phi = (phi * (1 + 0.3 * rng.random(shape))).astype(np.float32)
+    t = [torch.from_numpy(a).to(_dev()) for a in (
+        phi, rng.uniform(0, 1.5, shape).astype(np.float32),
+        (rng.random(shape) < 0.1).astype(np.uint8),
+        (phi + 0.1 * dx * (rng.random(shape) < 0.5)).astype(np.float32))]
+    for n in range(8):
+        a, b = t[0].clone(), t[0].clone()
+        ops.advect(a, t[1], t[2], t[3], dx, 0.3 * dx, n)
+        ops.advect_batch([(b, torch.full_like(b, float("nan")), t[1], t[2], t[3], dx, 0.3 * dx, n)])
+        assert torch.equal(a, b), n
+        a, b = t[0].clone(), t[0].clone()
+        ops.reinit_fsm(a, dx, 6 * dx, n)
+        ops.reinit_fsm_batch([(b, dx, 6 * dx, n)])
+        assert torch.equal(a, b), n
+
+
 def test_batched_advection_and_reinit_equal_single_calls():
     """petch_advect_batch and petch_reinit_fsm_batch (one launch per substep / sweep for many
     grids, bricks that provably do not change skipped) give exactly what petch_advect and
