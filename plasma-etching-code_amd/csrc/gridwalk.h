@@ -22,13 +22,13 @@
 //
 // Rounding. A plane crossing or a position is exact to a few ulps of the coordinates, 3e-5 of a
 // cell at 260 cells, and a triangle's vertices lie within as much of its cell; eps, 1e-4 of a cell
-// plus 1e-6 of the grid's length in cells, bounds what adds up. From cell to cell the walk goes by
-// the order of the crossings, so only near a cell edge, where two crossings come within eps of
-// each other, can it take the two cells beside the edge in the wrong order; the one it passes over
-// is then tested too. A leap lands in the cell its position says; cells whose border lies within
-// eps of it (along the ray, the crossing's own error) are tested too, and so are those around a
-// ray's start. Each step leaves its cell through a plane ahead, and a leap sets the other axes
-// back by less than it gains, so a walk ends after at most nx + ny + nz steps.
+// plus 1e-6 of the grid's length in cells, bounds what adds up. Within eps of a plane either side
+// may hold the hit, and a ray nearly along a plane stays beside it for many cells: the cells beside
+// the ray are tested too wherever it starts, wherever it enters a cell within eps (and the
+// crossing's own error along the ray) of a second plane, ahead or just left behind, and where it
+// ends just before a plane. (The check of each entry costs 1 to 3 % of a flux.) Each step leaves
+// its cell through a plane ahead, and a leap sets the other axes back by less than it gains, so a
+// walk ends after at most nx + ny + nz steps.
 #pragma once
 #include "bvh.h"
 
@@ -124,10 +124,13 @@ __device__ __forceinline__ int grid_side(float q, float eps) {
   return f < eps ? 1 : (f > 1.f - eps ? 2 : 0);
 }
 
-// The coordinate p in cells, within the m cells of its axis (a ray may run along the outer plane
-// of the last one).
+// The coordinate q in cells, within the m cells of its axis and no nearer than half a cell to its
+// ends (a ray may run along the outer planes; no neighbour lies across them).
+__device__ __forceinline__ float grid_clamp(float q, int m) {
+  return fminf(fmaxf(q, 0.5f), (float)m - 0.5f);
+}
 __device__ __forceinline__ float grid_coord(const GridView& g, float p, int m) {
-  return fminf(fmaxf(p * g.inv_dx, 0.f), (float)m - 0.5f);
+  return grid_clamp(p * g.inv_dx, m);
 }
 
 // Takes up the cell just entered, whose word is w.
@@ -187,11 +190,35 @@ __device__ __forceinline__ float plane_t(const GridView& g, int c, float o, floa
   return fabsf(inv) < 1.0e20f ? t : 1.0e30f;
 }
 
+// The side (as grid_side) on which the coordinate q, in cells, lies within tol of the border of
+// cell c or beyond it.
+__device__ __forceinline__ int cell_side(float q, int c, float tol) {
+  const float r = q - ((float)c + 0.5f);
+  return fabsf(r) > 0.5f - tol ? (r > 0.f ? 2 : 1) : 0;
+}
+
+// Ends a query whose end (its best hit, or the bound on t) lies beside a plane ahead: the cell of
+// that point and its neighbours within eps have their test first. D = 0 says that nothing else is
+// owed then.
+__device__ __forceinline__ WalkState walk_end(const GridView& g, Walk& T, Vec3 o, Vec3 d) {
+  const float qx = grid_coord(g, __builtin_fmaf(T.t, d.x, o.x), g.mx),
+              qy = grid_coord(g, __builtin_fmaf(T.t, d.y, o.y), g.my),
+              qz = grid_coord(g, __builtin_fmaf(T.t, d.z, o.z), g.mz);
+  T.cx = (int)qx;
+  T.cy = (int)qy;
+  T.cz = (int)qz;
+  walk_enter(T, grid_word(g, T.cx, T.cy, T.cz), 0);
+  T.amb = grid_side(qx, g.eps) | (grid_side(qy, g.eps) << 2) | (grid_side(qz, g.eps) << 4);
+  T.D = 0;
+  return kWalkTri;
+}
+
 // Leaves the current cell (or the empty cube around it) for the next.
 __device__ __forceinline__ WalkState walk_step(const GridView& g, Walk& T, Vec3 o, Vec3 d,
                                                const WalkRay& r) {
-  const bool px = r.inv.x >= 0.f, py = r.inv.y >= 0.f, pz = r.inv.z >= 0.f;
   const int D = T.D, E = 1 - D;
+  if (D == 0) return T.face >= 0 ? kWalkHit : kWalkMiss;
+  const bool px = r.inv.x >= 0.f, py = r.inv.y >= 0.f, pz = r.inv.z >= 0.f;
   // the planes the ray leaves through
   const int wx = T.cx + (px ? D : E), wy = T.cy + (py ? D : E), wz = T.cz + (pz ? D : E);
   const float tx = plane_t(g, wx, o.x, r.inv.x);
@@ -199,43 +226,35 @@ __device__ __forceinline__ WalkState walk_step(const GridView& g, Walk& T, Vec3 
   const float tz = plane_t(g, wz, o.z, r.inv.z);
   const float te = fminf(fminf(tx, ty), tz);
   const bool ax = tx <= te, ay = !ax && ty <= te, az = !ax && !ay;
-  const int ex = px ? wx : wx - 1, ey = py ? wy : wy - 1, ez = pz ? wz : wz - 1;
-  // how far a crossing of each axis may be off along the ray
-  const float bx = g.slack * fabsf(r.inv.x), by = g.slack * fabsf(r.inv.y),
-              bz = g.slack * fabsf(r.inv.z);
-  const float be = ax ? bx : (ay ? by : bz);
-  if (T.t <= te - 2.f * be) return T.face >= 0 ? kWalkHit : kWalkMiss;
+  // how far the crossing may be off along the ray
+  const float be = g.slack * fabsf(ax ? r.inv.x : (ay ? r.inv.y : r.inv.z));
+  if (T.t <= te - 2.f * be) {
+    const float s2 = 2.f * g.slack;
+    if (T.t > fminf(fminf(tx - s2 * fabsf(r.inv.x), ty - s2 * fabsf(r.inv.y)),
+                    tz - s2 * fabsf(r.inv.z)))
+      return walk_end(g, T, o, d);
+    return T.face >= 0 ? kWalkHit : kWalkMiss;
+  }
+  // the cell entered: across the plane left, on the other axes the cell held (one step) or the
+  // one that the position says (a leap)
+  const float qx = __builtin_fmaf(te, d.x, o.x) * g.inv_dx,
+              qy = __builtin_fmaf(te, d.y, o.y) * g.inv_dx,
+              qz = __builtin_fmaf(te, d.z, o.z) * g.inv_dx;
+  T.cx = ax ? (px ? wx : wx - 1) : (D == 1 ? T.cx : (int)grid_clamp(qx, g.mx));
+  T.cy = ay ? (py ? wy : wy - 1) : (D == 1 ? T.cy : (int)grid_clamp(qy, g.my));
+  T.cz = az ? (pz ? wz : wz - 1) : (D == 1 ? T.cz : (int)grid_clamp(qz, g.mz));
+  // Where the ray comes within tol of a second plane, ahead or just left behind, the cells beside
+  // the one entered have their test too: across that plane, with those back over the plane it came
+  // through. (The distances to the nearest plane of each axis; that of the plane left is about 0.)
+  const float tol = g.eps + 2.f * be * g.inv_dx * fmaxf(fmaxf(fabsf(d.x), fabsf(d.y)), fabsf(d.z));
   int amb = 0;
-  if (D == 1) {
-    const bool sx = !ax && tx - te < 2.f * (bx + be), sy = !ay && ty - te < 2.f * (by + be),
-               sz = !az && tz - te < 2.f * (bz + be);
-    if (sx || sy || sz) {
-      // the cells across the edge from the one entered: back over the plane left, on over the
-      // plane that is as near
-      amb = (sx ? (px ? 2 : 1) : (ax ? (px ? 1 : 2) : 0)) |
-            (sy ? (py ? 2 : 1) : (ay ? (py ? 1 : 2) : 0)) << 2 |
-            (sz ? (pz ? 2 : 1) : (az ? (pz ? 1 : 2) : 0)) << 4;
-    }
-    if (fmaxf(fmaxf(fabsf(r.inv.x), fabsf(r.inv.y)), fabsf(r.inv.z)) >= 1.0e20f) {
-      // a ray along a plane stays with both sides of it
-      if (fabsf(r.inv.x) >= 1.0e20f) amb |= grid_side(o.x * g.inv_dx, g.eps);
-      if (fabsf(r.inv.y) >= 1.0e20f) amb |= grid_side(o.y * g.inv_dx, g.eps) << 2;
-      if (fabsf(r.inv.z) >= 1.0e20f) amb |= grid_side(o.z * g.inv_dx, g.eps) << 4;
-    }
-    T.cx = ax ? ex : T.cx;
-    T.cy = ay ? ey : T.cy;
-    T.cz = az ? ez : T.cz;
-  } else {
-    const float qx = grid_coord(g, __builtin_fmaf(te, d.x, o.x), g.mx),
-                qy = grid_coord(g, __builtin_fmaf(te, d.y, o.y), g.my),
-                qz = grid_coord(g, __builtin_fmaf(te, d.z, o.z), g.mz);
-    T.cx = ax ? ex : (int)qx;
-    T.cy = ay ? ey : (int)qy;
-    T.cz = az ? ez : (int)qz;
-    const float k = 2.f * be * g.inv_dx;
-    amb = (ax ? 0 : grid_side(qx, g.eps + k * fabsf(d.x))) |
-          (ay ? 0 : grid_side(qy, g.eps + k * fabsf(d.y)) << 2) |
-          (az ? 0 : grid_side(qz, g.eps + k * fabsf(d.z)) << 4);
+  if (__builtin_amdgcn_fmed3f(fabsf(qx - rintf(qx)), fabsf(qy - rintf(qy)),
+                              fabsf(qz - rintf(qz))) < tol) {
+    const int sx = ax ? 0 : cell_side(grid_clamp(qx, g.mx), T.cx, tol),
+              sy = ay ? 0 : cell_side(grid_clamp(qy, g.my), T.cy, tol),
+              sz = az ? 0 : cell_side(grid_clamp(qz, g.mz), T.cz, tol);
+    if (sx | sy | sz)
+      amb = (ax ? (px ? 1 : 2) : sx) | (ay ? (py ? 1 : 2) : sy) << 2 | (az ? (pz ? 1 : 2) : sz) << 4;
   }
   if ((unsigned)T.cx >= (unsigned)g.mx || (unsigned)T.cy >= (unsigned)g.my ||
       (unsigned)T.cz >= (unsigned)g.mz) {

@@ -175,3 +175,48 @@ def test_walk_answers_ray_queries_as_the_tree(name):
         assert int(other.sum()) <= 2
         assert bool(((fa >= 0) == (fb >= 0)).all())
         assert float((ta - tb).abs().max()) <= 2e-6 * float(tb.max())
+
+
+def _aimed_rays(mesh, phi, dx, kind, n, gen):
+    """Rays at vertices and edges of the surface, or that run nearly along a grid plane into one."""
+    import torch
+    v, f = mesh.verts.cpu(), mesh.faces.cpu().long()
+    L = torch.tensor([s * dx for s in phi.shape])
+    q = f[torch.randint(0, mesh.nf, (n,), generator=gen)]
+    a, b = v[q[:, 0]], v[q[:, 1]]
+    u = torch.rand((n, 1), generator=gen)
+    target = a + u * (b - a) if kind == "edge" else a
+    if kind == "beside":
+        # components 1e-2 to 1e-7 of the others on one axis, on half of the rays on two
+        d = torch.randn((n, 3), generator=gen)
+        ax = torch.randint(0, 3, (n,), generator=gen)
+        two = (torch.rand(n, generator=gen) < 0.5).float()
+        rows = torch.arange(n)
+        d[rows, ax] *= 10 ** (-2 - 5 * torch.rand(n, generator=gen))
+        d[rows, (ax + 1) % 3] *= 10 ** (-two * (1 + 5 * torch.rand(n, generator=gen)))
+        d = d / d.norm(dim=1, keepdim=True)
+        o = target - torch.rand((n, 1), generator=gen) * 0.7 * float(L.max()) * d
+    else:
+        o = (torch.rand((n, 3), generator=gen) * 1.2 - 0.1) * L
+        d = target - o
+        d = d / d.norm(dim=1, keepdim=True)
+    return o.contiguous(), (d + 0.0).contiguous()
+
+
+@pytest.mark.parametrize("kind", ["vertex", "edge", "beside"])
+@pytest.mark.parametrize("name", NAMES)
+def test_rays_at_vertices_edges_and_beside_planes_hit_as_on_the_tree(name, kind):
+    """Where two cells meet, a ray can lie on either side of the plane between them by rounding, and
+    one nearly along the plane stays there: both cells have to be looked into. The walk's distances
+    are the tree's to the bit (one triangle test, one query of the tree for a ray that meets two
+    faces at once), and so are the faces."""
+    import torch
+    from petch import ops
+    mesh, phi, dx, box, dev = _surface(name)
+    tree = ops.Bvh(dev).build(mesh.verts, mesh.faces)
+    o, d = _aimed_rays(mesh, phi, dx, kind, 400000, torch.Generator().manual_seed(2))
+    fa, ta = mesh.bvh.query_ray(o.to(dev), d.to(dev))
+    fb, tb = tree.query_ray(o.to(dev), d.to(dev))
+    assert int((fb >= 0).sum()) > 100000
+    print(name, kind, int((fa != fb).sum()), int((ta != tb).sum()), flush=True)
+    assert torch.equal(fa, fb) and torch.equal(ta, tb)
