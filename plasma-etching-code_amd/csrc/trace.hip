@@ -33,9 +33,12 @@ bool petch_grid_view(const petch_bvh* b, petch::GridView* v);
 
 namespace {
 
-// Rays that a walk trace leaves to the tree (Ties): at most kMaxTies of a launch, the others keep
-// the walk's own choice.
-constexpr unsigned kMaxTies = 65536;
+// Places in a launch's list of the rays that a walk trace leaves to the tree. The tie number
+// RayQueue::tie_stop, after which the rays held by all wavefronts still fit, ends the queue for the
+// walk (its cursor goes to kQueueCut), and the tree traces what was not taken: the list never runs
+// over, and no ray's hits depend on the schedule.
+constexpr unsigned kTieList = 1u << 20;
+constexpr unsigned kQueueCut = 0xc0000000u;
 
 // Per-context 64-bit hit counters (slot 0 neutral, 1 ion), read by petch_trace_hit_counts;
 // slots 2-3 hold the ray-queue cursor of the persistent trace launches and the number of their
@@ -43,7 +46,7 @@ constexpr unsigned kMaxTies = 65536;
 unsigned long long* petch_hit_counter(petch_ctx* ctx, int which) {
   bool fresh = ctx->scr_cap[SCR_TRACE] == 0;
   unsigned long long* c =
-      (unsigned long long*)petch_scratch(ctx, SCR_TRACE, (4 + kMaxTies) * sizeof(unsigned long long));
+      (unsigned long long*)petch_scratch(ctx, SCR_TRACE, (4 + kTieList) * sizeof(unsigned long long));
   if (c && fresh && hipMemsetAsync(c, 0, 4 * sizeof(unsigned long long), ctx->stream) != hipSuccess)
     return nullptr;
   return c ? c + which : nullptr;
@@ -246,8 +249,10 @@ struct RayQueue {
   // the walk traces' share of a wavefront: rays per claim, lanes in use, and the live lanes at or
   // below which it stops for hits and new rays
   int chunk, lanes, refill_at;
-  // ties: their number and list (queue id, the ray's earlier hits)
+  // ties: their number (n_ties[0]; [1]: 1 + the cursor when they ended the queue, else 0), the
+  // number that ends it, and their list (queue id, the ray's earlier hits)
   unsigned* n_ties;
+  unsigned tie_stop;
   uint2* ties;
 };
 
@@ -299,7 +304,7 @@ __device__ __forceinline__ bool claim_ray(const RayQueue& q, bool active, bool& 
 constexpr int kRefillAt = 24;
 constexpr int kMinLanes = 8;
 constexpr int kTestsPerPhase = 2, kStepsPerPhase = 3;
-constexpr int kTieBlocks = 4;
+constexpr int kTieBlocks = 64;
 constexpr int kLdsStack = 8;  // traversal stack entries per lane held in LDS (16 KB/workgroup)
 // kMiss: the ray left the domain and the policy replays paths (P::kReplay), so it gets a say
 // (P::miss) before the lane goes idle.
@@ -437,11 +442,12 @@ __device__ __forceinline__ void walk_trace(const P& pol, const RayQueue& q,
         if (st == kWHit) {
           ++nh;
           st = kWIdle;
-          unsigned at = kMaxTies;
-          if (T.tie) at = atomicAdd(q.n_ties, 1u);
-          if (at < kMaxTies) {
+          if (T.tie) {
             --nh;
-            q.ties[at] = make_uint2(pol.id(R), pol.earlier(R));
+            const unsigned at = atomicAdd(q.n_ties, 1u);
+            // (a load of n_ties with each claim took a quarter of a flux)
+            if (at == q.tie_stop) q.n_ties[1] = 1u + atomicExch(q.next, kQueueCut);
+            if (at < kTieList) q.ties[at] = make_uint2(pol.id(R), pol.earlier(R));
           } else {
             emit = pol.hit(R, Hit{T.face, T.face, T.t}, o, d, e, true);
             // a replayed path starts over from its source, not from this face
@@ -1270,19 +1276,22 @@ k_trace(P pol, RayQueue q, unsigned long long* __restrict__ hits) {
 }
 
 // The rays that a walk trace left to the tree, from their sources again: the same path up to the
-// tie, whose earlier hits are not deposited a second time. A handful per launch at most, so each
-// lane runs its ray to the end.
+// tie, whose earlier hits are not deposited a second time; then the rays that it did not take. A
+// handful per launch on a surface without coincident faces, so each lane runs its ray to the end.
 template <class P>
 __global__ void __launch_bounds__(kBS)
 k_trace_ties(P pol, RayQueue q, unsigned long long* __restrict__ hits) {
-  const unsigned n = min(*q.n_ties, kMaxTies);
+  const unsigned n = min(q.n_ties[0], kTieList), cut = q.n_ties[1];
+  const unsigned taken = cut ? min(cut - 1u, (unsigned)q.n) : (unsigned)q.n;
+  const unsigned end = n + ((unsigned)q.n - taken);
   unsigned nh = 0;
-  for (unsigned i = blockIdx.x * kBS + threadIdx.x; i < n; i += gridDim.x * kBS) {
+  for (unsigned i = blockIdx.x * kBS + threadIdx.x; i < end; i += gridDim.x * kBS) {
     typename P::Ray R;
     Emit e;
     Vec3 o;
-    pol.start(R, q.ties[i].x, o, e);
-    unsigned muted = q.ties[i].y;
+    const uint2 ray = i < n ? q.ties[i] : make_uint2(taken + (i - n), 0u);
+    pol.start(R, ray.x, o, e);
+    unsigned muted = ray.y;
     bool go = true;
     while (go) {
       const Vec3 d = emit_dir(e);
@@ -1547,6 +1556,7 @@ int make_queue(petch_ctx* ctx, int n, RayQueue& q) {
   q.next = (unsigned*)c;
   q.n = n;
   q.n_ties = (unsigned*)(c + 1);
+  q.tie_stop = kTieList;
   q.ties = (uint2*)(c + 2);
   PETCH_HIP(ctx, hipMemsetAsync(q.next, 0, 2 * sizeof(unsigned long long), ctx->stream));
   return PETCH_OK;
@@ -1554,13 +1564,17 @@ int make_queue(petch_ctx* ctx, int n, RayQueue& q) {
 
 // The grid of a walk trace and its wavefronts' shares of the rays.
 unsigned walk_share(petch_ctx* ctx, const void* kernel, RayQueue& q) {
-  const unsigned all = persistent_blocks(ctx, kernel, 0x7fffffff);
+  // (the list of ties has room for what all wavefronts hold: a ray a lane and a claim of ids)
+  const unsigned most = (kTieList - 1024) / (64 + kRayChunk) / (kBS / 64);
+  unsigned all = persistent_blocks(ctx, kernel, 0x7fffffff);
+  all = all < most ? all : most;
   const long long waves = (long long)all * (kBS / 64);
   const int per = (int)((q.n + waves - 1) / waves);
   q.lanes = per < kMinLanes ? kMinLanes : (per < 64 ? per : 64);
   q.chunk = per < 64 ? q.lanes : (per < 512 ? 64 : (int)kRayChunk);
   q.refill_at = q.lanes * kRefillAt / 64;
   const long long need = ((long long)q.n + q.lanes * (kBS / 64) - 1) / (q.lanes * (kBS / 64));
+  q.tie_stop = kTieList - (unsigned)waves * (64u + (unsigned)q.chunk);
   return (unsigned)(need < all ? need : all);
 }
 

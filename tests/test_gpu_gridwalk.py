@@ -220,3 +220,81 @@ def test_rays_at_vertices_edges_and_beside_planes_hit_as_on_the_tree(name, kind)
     assert int((fb >= 0).sum()) > 100000
     print(name, kind, int((fa != fb).sum()), int((ta != tb).sum()), flush=True)
     assert torch.equal(fa, fb) and torch.equal(ta, tb)
+
+
+def _doubled(mesh, phi, dx, share):
+    """mesh with the faces (a, b, c) of a share of its cells followed by (a, b, their centroid): the
+    verts and faces, and the walked and the plain tree over them. A ray that hits the added face
+    meets two at one distance, or an ulp apart."""
+    import torch
+    from petch import ops
+    dev = mesh.device
+    n = phi.numel()
+    cnt = mesh.grid[0][:n].long() & 15
+    gen = torch.Generator().manual_seed(4)
+    twice = (torch.rand(n, generator=gen).to(dev) < share) & (cnt <= 7)
+    new = torch.where(twice, 2 * cnt, cnt)
+    first = torch.cumsum(new, 0) - new
+    cells = torch.where(cnt > 0, (first << 4) | new, 0).to(torch.int32)
+    copies = torch.repeat_interleave(torch.where(twice, 2, 1), cnt)
+    faces = torch.repeat_interleave(mesh.faces, copies, dim=0)
+    at = torch.cumsum(copies, 0)[copies == 2] - 1
+    faces[at, 2] = mesh.nv + torch.arange(len(at), dtype=torch.int32, device=dev)
+    verts = torch.cat([mesh.verts, mesh.centroids[copies == 2]]).contiguous()
+    nx, ny, nz = phi.shape
+    walked = ops.Bvh(dev).build(verts, faces).set_grid(verts, faces, (cells, nx, ny, nz, dx))
+    assert walked.status() == 0
+    return verts, faces, walked, ops.Bvh(dev).build(verts, faces)
+
+
+# 3M rays: more ties than the list of a launch takes, so that the tree traces the rays left over
+@pytest.mark.parametrize("name,share,n", [("hole", 0.3, 40000), ("trench", 0.05, 40001),
+                                          ("flat", 0.5, 4097), ("noise", 0.2, 20000),
+                                          ("thin", 0.1, 63), ("rough", 1.0, 20000),
+                                          ("hole", 1.0, 3000000)])
+def test_rays_that_meet_two_faces_at_once_take_the_trees(name, share, n, det):
+    """A tied ray starts over on the tree and deposits what its walk had not: with coincident faces
+    ties come at every bounce, and the deterministic sums and the numbers of hits are the tree's to
+    the bit, in the batched launches too. (The adjoint's float sums: each adds at most 1e5 terms,
+    in any order, 1e5 * 2^-24 of their mass at the very most; 1e-5 of it.)"""
+    import torch
+    from petch import flux, ops
+    from petch.params import PAR
+    mesh, phi, dx, box, dev = _surface(name)
+    verts, faces, walked, tree = _doubled(mesh, phi, dx, share)
+    nf = int(faces.shape[0])
+    bare = torch.from_numpy(np.random.default_rng(3).uniform(0.05, 0.9, nf).astype(np.float32)).to(dev)
+    par = dict(PAR, ion_source="powcos", ion_exponent=20.0)
+    cen, area, nrm = ops.mesh_attrs(verts, faces)
+    gn = ops.gas_normals(phi, dx, cen, nrm)
+    src, isrc, ipar = flux.NEUTRAL_SOURCE, flux.ion_source(par), flux.ion_params(par)
+
+    def fluxes(b):
+        ops.trace_hit_counts(dev)
+        a, o = ops.trace_neutral_rr_pair(b, box, src, bare, 0.7, n, 5, 1.0, n // 2, 6)
+        out = [a.clone(), o.clone(), ops.trace_neutral_rr(b, box, src, bare, 0.3, n, 7).clone()]
+        out += [x.clone() for x in ops.trace_ion_yield(b, box, isrc, ipar, n, 8)]
+        out.append(ops.trace_neutral_cap(b, box, src, bare, 0.5, 4, n, 9).clone())
+        hits = tuple(int(x) for x in ops.trace_hit_counts(dev))
+        out.append(ops.trace_redeposition(b, cen, gn, area, bare, 0.5, n, 10).clone())
+        if n < 1000000:
+            out.append(ops.trace_ff(b, box, cen, gn, 24, 17).clone())
+            items = [dict(bvh=b, box=box, bare=bare, beta_a=0.7, n_a=n // (k + 1), seed_a=3 + k,
+                          beta_b=1.0, n_b=n // 2, seed_b=4) for k in range(3)]
+            for x, y in ops.trace_neutral_rr_batch(src, items):
+                out += [x.clone(), y.clone()]
+            items = [dict(bvh=b, box=box, src=isrc, ion=ipar, n=n // (k + 1), seed=3 + k)
+                     for k in range(3)]
+            for x in ops.trace_ion_yield_batch(items):
+                out += [y.clone() for y in x]
+            g = ops.trace_neutral_rr_pair_adjoint(b, box, src, bare, 0.7, n, 5, a, 1.0, n // 2, 6, o)
+        else:
+            g = None
+        assert b.status() == 0
+        return out, hits, g
+    (x, hx, gx), (y, hy, gy) = fluxes(walked), fluxes(tree)
+    assert hx == hy and hx[0] >= n // 4
+    for k, (p, q) in enumerate(zip(x, y)):
+        assert torch.equal(p, q), (k, float((p - q).abs().max()))
+    if gx is not None:
+        assert float((gx - gy).abs().sum()) <= 1e-5 * float(gy.abs().sum())
