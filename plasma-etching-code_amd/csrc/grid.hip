@@ -264,6 +264,8 @@ bool petch_grid_view(const petch_bvh* b, petch::GridView* v) {
   v->inv_dx = (float)(1.0 / b->grid_dx);
   v->eps = 1.0e-4f + 1.0e-6f * (float)max_axis(v->mx, v->my, v->mz);
   v->slack = 0.25f * v->eps * v->dx;
+  // (an ulp there is half of slack; it lies past the grid's length and past 100 cells)
+  v->reach = 4194304.f * v->slack;
   v->root = petch_bvh_view(b).root;
   return true;
 }

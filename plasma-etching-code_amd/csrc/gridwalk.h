@@ -28,7 +28,9 @@
 // crossing's own error along the ray) of a second plane, ahead or just left behind, and where it
 // ends just before a plane. (The check of each entry costs 1 to 3 % of a flux.) Each step leaves
 // its cell through a plane ahead, and a leap sets the other axes back by less than it gains, so a
-// walk ends after at most nx + ny + nz steps.
+// walk ends after at most nx + ny + nz steps. All this is about origins in the grid or some grid
+// lengths off; the rounding of a farther one grows with it, and its ray is left to the tree
+// (GridView::reach).
 #pragma once
 #include "bvh.h"
 
@@ -42,6 +44,7 @@ struct GridView {
   int mx, my, mz;      // cells per axis
   float dx, inv_dx, eps;  // eps in cells
   float slack;            // a quarter of eps in length units
+  float reach;            // largest coordinate of an origin that the walk takes
   const float* root;   // bounds of all triangles (lo xyz, hi xyz); null below two faces
 };
 
@@ -155,8 +158,8 @@ __device__ __forceinline__ WalkState walk_begin(const GridView& g, Walk& T, Vec3
                                                 const WalkRay& r, float tmax, int skip) {
   T.face = -1;
   T.skip = skip;
-  T.tie = false;
-  const float e = g.eps * g.dx;
+  const float far = fmaxf(fmaxf(fabsf(o.x), fabsf(o.y)), fabsf(o.z));
+  const float e = __builtin_fmaf(far, 9.53674316e-7f, g.eps * g.dx);  // and 8 ulps of the origin
   Vec3 lo = v3(0.f, 0.f, 0.f),
        hi = v3((float)g.mx * g.dx, (float)g.my * g.dx, (float)g.mz * g.dx);
   if (g.root) {
@@ -170,7 +173,13 @@ __device__ __forceinline__ WalkState walk_begin(const GridView& g, Walk& T, Vec3
   const float tf = fminf(fminf(((px ? hi.x + e : lo.x - e) - o.x) * r.inv.x,
                                ((py ? hi.y + e : lo.y - e) - o.y) * r.inv.y),
                          ((pz ? hi.z + e : lo.z - e) - o.z) * r.inv.z);
+  T.tie = false;
   if (!(tn <= tf)) return kWalkMiss;
+  // an origin so far off that its rounding nears eps: to the tree, as a tie
+  if (far > g.reach) {
+    T.tie = true;
+    return kWalkHit;
+  }
   T.t = fminf(tmax, tf);
   const float qx = grid_coord(g, o.x + tn * d.x, g.mx),
               qy = grid_coord(g, o.y + tn * d.y, g.my),

@@ -1609,6 +1609,13 @@ int launch_walk(petch_ctx* ctx, void (*kernel)(P, RayQueue, unsigned long long*)
   return PETCH_OK;
 }
 
+// Whether a surface has a grid whose walk takes the rays of a box's source plane and wraps (it
+// leaves an origin beyond the grid's reach to the tree, ray by ray).
+bool walk_grid(const petch_bvh* bvh, const Box& b, GridView* g) {
+  return petch_grid_view(bvh, g) &&
+         fmaxf(fmaxf(fabsf(b.lx), fabsf(b.ly)), fabsf(b.zsrc)) <= g->reach;
+}
+
 // Traces n rays on the surface of bvh: by its grid where it has one, else by its tree.
 // make(view) gives the policy for either view; Five picks k_trace5.
 template <bool Five, class Make>
@@ -1616,7 +1623,7 @@ int trace_surface(petch_ctx* ctx, const petch_bvh* bvh, Make make, int n,
                   unsigned long long* hits) {
   const auto tree = make(petch_bvh_view(bvh));
   GridView g;
-  const bool grid = petch_grid_view(bvh, &g);
+  const bool grid = walk_grid(bvh, tree.b, &g);
   const auto walk = make(g);
   using T = std::decay_t<decltype(tree)>;
   using W = std::decay_t<decltype(walk)>;
@@ -1750,7 +1757,7 @@ extern "C" int petch_trace_redeposition(petch_ctx* ctx, const petch_bvh* bvh,
     if (!q) return PETCH_E_HIP;
   }
   rc = trace_surface<true>(ctx, bvh, [&](auto view) {
-    return Redep<decltype(view)>{view, Box{1.f, 1.f, 1.f, 1.f, 0}, centroids, gas_normals, cum, nf,
+    return Redep<decltype(view)>{view, Box{0.f, 0.f, 0.f, 0.f, 0}, centroids, gas_normals, cum, nf,
                                  s_redep, q ? (float*)q : out, seed, q ? 1 : 0};
   }, n, nullptr);
   if (rc) return rc;
@@ -1929,8 +1936,8 @@ extern "C" int petch_trace_neutral_rr_batch(petch_ctx* ctx, const petch_source* 
     PETCH_ARG(ctx, a.n_a >= 0 && a.n_b >= 0, "trace_neutral_rr_batch: feature %d: n < 0", f);
     NeutralFeature& d = t[f];
     d.bv = petch_bvh_view(a.bvh);
-    if (a.bvh->nf > 0) grids = petch_grid_view(a.bvh, &d.gv) && grids;
     d.b = make_box(&a.box);
+    if (a.bvh->nf > 0) grids = walk_grid(a.bvh, d.b, &d.gv) && grids;
     d.bare = a.bare;
     d.beta[0] = a.beta_a;
     d.beta[1] = a.beta_b;
@@ -2004,8 +2011,8 @@ extern "C" int petch_trace_ion_yield_batch(petch_ctx* ctx, int nfeat,
     PETCH_ARG(ctx, a.n >= 0, "trace_ion_yield_batch: feature %d: n < 0", f);
     IonFeature& d = t[f];
     d.bv = petch_bvh_view(a.bvh);
-    if (a.bvh->nf > 0) grids = petch_grid_view(a.bvh, &d.gv) && grids;
     d.b = make_box(&a.box);
+    if (a.bvh->nf > 0) grids = walk_grid(a.bvh, d.b, &d.gv) && grids;
     d.src = make_source(&a.src);
     const petch_ion_params& ip = a.ip;
     d.P = IonParams{ip.meanE,  ip.sigmaE, ip.A_sp,   ip.Eth_sp,  ip.B_sp,   ip.A_ie,
@@ -2091,7 +2098,7 @@ extern "C" int petch_trace_ff(petch_ctx* ctx, const petch_bvh* bvh, const petch_
   PETCH_ARG(ctx, n < (1LL << 31), "trace_ff: nf*n_ff too large");
   if (n == 0) return PETCH_OK;
   GridView g;
-  if (petch_grid_view(bvh, &g))
+  if (walk_grid(bvh, make_box(box), &g))
     return trace_surface<false>(ctx, bvh, [&](auto view) {
       return FormFactor<decltype(view)>{view, make_box(box), centroids, gas_normals, n_ff, seed,
                                         hitface};

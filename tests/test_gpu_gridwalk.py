@@ -298,3 +298,41 @@ def test_rays_that_meet_two_faces_at_once_take_the_trees(name, share, n, det):
         assert torch.equal(p, q), (k, float((p - q).abs().max()))
     if gx is not None:
         assert float((gx - gy).abs().sum()) <= 1e-5 * float(gy.abs().sum())
+
+
+@pytest.mark.parametrize("name", NAMES)
+def test_rays_from_far_outside_hit_as_on_the_tree(name, det):
+    """The rounding of an origin grows with its distance; beyond the grid's reach (about 100 cells,
+    or the grid's own length where that is more) a ray is left to the tree: queries, rays that
+    start there within a trace, and launches whose source plane lies there."""
+    import torch
+    from petch import flux, ops
+    mesh, phi, dx, box, dev = _surface(name)
+    tree = ops.Bvh(dev).build(mesh.verts, mesh.faces)
+    g = torch.Generator().manual_seed(6)
+    n, L = 100000, max(phi.shape) * dx
+    for far in (2, 10, 100, 1000):
+        q = mesh.faces.cpu().long()[torch.randint(0, mesh.nf, (n,), generator=g)]
+        u = torch.rand((n, 3, 1), generator=g)
+        aim = (mesh.verts.cpu()[q] * (u / u.sum(1, keepdim=True))).sum(1)
+        d = torch.randn((n, 3), generator=g)
+        d = d / d.norm(dim=1, keepdim=True)
+        o = (aim - far * L * d).to(dev).contiguous()
+        fa, ta = mesh.bvh.query_ray(o, d.to(dev))
+        fb, tb = tree.query_ray(o, d.to(dev))
+        assert int((fb >= 0).sum()) > n // 2
+        print(name, far, int((fa != fb).sum()), int((ta != tb).sum()), flush=True)
+        assert torch.equal(fa, fb) and torch.equal(ta, tb), far
+    # form-factor rays from points up to 400 cells off, towards the surface
+    q = torch.randint(0, mesh.nf, (mesh.nf,), generator=g).to(dev)
+    d = torch.randn((mesh.nf, 3), generator=g).to(dev)
+    d = d / d.norm(dim=1, keepdim=True)
+    away = torch.linspace(0.0, 400.0, mesh.nf, device=dev)[:, None] * dx
+    cen = (mesh.centroids[q] - away * d).contiguous()
+    a, b = (ops.trace_ff(t, box, cen, d.contiguous(), 256, 3) for t in (mesh.bvh, tree))
+    assert int((b >= 0).sum()) > 100 and torch.equal(a, b)
+    bare = torch.full((mesh.nf,), 0.5, device=dev)
+    far_box = ops.make_box(*(s * dx for s in phi.shape[:2]), 1e4 * L, 300 * L, 1)
+    a, b = (ops.trace_neutral_rr(t, far_box, flux.NEUTRAL_SOURCE, bare, 0.5, 20000, 3)
+            for t in (mesh.bvh, tree))
+    assert float(b.sum()) > 0 and torch.equal(a, b)
