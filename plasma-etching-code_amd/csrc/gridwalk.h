@@ -101,13 +101,12 @@ __device__ __forceinline__ bool walk_tri(Vec3 o, const WalkRay& r, Vec3 p0, Vec3
 
 // State of one query. cell (cx, cy, cz) with its leap D; faces [cur, end) of the cell still to be
 // tested; amb: the neighbours still owed a test (two bits per axis: 1 the lower, 2 the upper
-// neighbour; bits 6..8 the subset of axes tested last); skip: the face the ray starts on, which it
-// cannot meet again.
+// neighbour; bits 6..8 the subset of axes tested last).
 struct Walk {
   float t;   // best hit so far, or the bound on t
   int face;  // its face, -1 none
   int cx, cy, cz, D;
-  int cur, end, amb, skip;
+  int cur, end, amb;
   bool tie;
 };
 
@@ -151,13 +150,13 @@ __device__ __forceinline__ WalkState walk_enter(Walk& T, uint32_t w, int amb) {
   return (n || amb) ? kWalkTri : kWalkOn;
 }
 
-// Starts the query of the ray (o, d) for hits with 0 < t < tmax, which does not meet the face
-// `skip` (-1 none). The walk covers the stretch of the ray within the bounds of the triangles, eps
-// wider: a ray that starts above the surface enters at its top, one that leaves upwards ends there.
+// Starts the query of the ray (o, d) for hits with 0 < t < tmax. The walk covers the stretch of the
+// ray within the bounds of the triangles, eps wider: a ray that starts above the surface enters at
+// its top, one that leaves upwards ends there. (The face that a ray starts on has its test as any
+// other: where the coordinates' rounding exceeds the origin's offset the ray meets it again.)
 __device__ __forceinline__ WalkState walk_begin(const GridView& g, Walk& T, Vec3 o, Vec3 d,
-                                                const WalkRay& r, float tmax, int skip) {
+                                                const WalkRay& r, float tmax) {
   T.face = -1;
-  T.skip = skip;
   const float far = fmaxf(fmaxf(fabsf(o.x), fabsf(o.y)), fabsf(o.z));
   const float e = __builtin_fmaf(far, 9.53674316e-7f, g.eps * g.dx);  // and 8 ulps of the origin
   Vec3 lo = v3(0.f, 0.f, 0.f),
@@ -279,7 +278,6 @@ __device__ __forceinline__ WalkState walk_step(const GridView& g, Walk& T, Vec3 
 // neighbour owed a test, or back to walking.
 __device__ __forceinline__ WalkState walk_test(const GridView& g, Walk& T, Vec3 o,
                                                const WalkRay& r) {
-  if (T.cur == T.skip) ++T.cur;
   if (T.cur < T.end) {
     const float4* q = g.tris + 3 * (long long)T.cur;
     const float4 q0 = q[0], q1 = q[1], q2 = q[2];
@@ -326,7 +324,7 @@ __device__ __forceinline__ Hit walk_closest_hit(const GridView& g, const BvhView
                                                 Vec3 d, float tmax) {
   const WalkRay r = walk_ray(d);
   Walk T;
-  WalkState s = walk_begin(g, T, o, d, r, tmax, -1);
+  WalkState s = walk_begin(g, T, o, d, r, tmax);
   while (s == kWalkOn || s == kWalkTri) {
     if (s == kWalkTri) s = walk_test(g, T, o, r);
     else s = walk_step(g, T, o, d, r);

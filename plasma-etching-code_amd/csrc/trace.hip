@@ -425,7 +425,7 @@ __device__ __forceinline__ void walk_trace(const P& pol, const RayQueue& q,
   typename P::Ray R;
   Vec3 o = v3(0.f, 0.f, 0.f), d = v3(0.f, 0.f, -1.f);
   petch::WalkRay rp;
-  int wraps = 0, skip = -1;
+  int wraps = 0;
   unsigned nh = 0;
   int st = kWIdle;
   bool exhausted = false;
@@ -450,14 +450,11 @@ __device__ __forceinline__ void walk_trace(const P& pol, const RayQueue& q,
             if (at < kTieList) q.ties[at] = make_uint2(pol.id(R), pol.earlier(R));
           } else {
             emit = pol.hit(R, Hit{T.face, T.face, T.t}, o, d, e, true);
-            // a replayed path starts over from its source, not from this face
-            skip = (!P::kReplay || e.mode == kLobe) ? T.face : -1;
           }
         }
         if constexpr (P::kReplay) {
           if (st == kWMiss) {
             emit = pol.miss(R, o, e);
-            skip = -1;
             st = kWIdle;
           }
         }
@@ -465,7 +462,6 @@ __device__ __forceinline__ void walk_trace(const P& pol, const RayQueue& q,
         unsigned ray;
         if (claim_some(q, st == kWIdle && !emit, q.lanes - busy, exhausted, pool, pool_end, ray)) {
           pol.start(R, ray, o, e);
-          skip = -1;
           emit = true;
         }
         if (emit) {
@@ -486,13 +482,12 @@ __device__ __forceinline__ void walk_trace(const P& pol, const RayQueue& q,
         if (b.periodic && wraps < kMaxWraps && !never_returns(g, o, d) &&
             wrap_ray(b, o, d, rp.inv)) {
           ++wraps;
-          skip = -1;
           st = kWBegin;
         } else {
           st = P::kReplay ? kWMiss : kWIdle;
         }
       }
-      if (st == kWBegin) st = petch::walk_begin(g, T, o, d, rp, 1.0e6f, skip);
+      if (st == kWBegin) st = petch::walk_begin(g, T, o, d, rp, 1.0e6f);
     } else if (nt >= nw) {
 #pragma unroll 1
       for (int k = 0; k < kTestsPerPhase; ++k)

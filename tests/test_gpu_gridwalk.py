@@ -336,3 +336,30 @@ def test_rays_from_far_outside_hit_as_on_the_tree(name, det):
     a, b = (ops.trace_neutral_rr(t, far_box, flux.NEUTRAL_SOURCE, bare, 0.5, 20000, 3)
             for t in (mesh.bvh, tree))
     assert float(b.sum()) > 0 and torch.equal(a, b)
+
+
+@pytest.mark.parametrize("name", ["hole", "trench"])
+def test_traces_in_large_units_equal_the_trees(name, det):
+    """With coordinates of thousands, re-emission points 1e-4 off the surface round onto it or below,
+    and the next query may meet the same face again, on the walk as on the tree."""
+    import torch
+    from petch import flux, ops
+    from petch.params import PAR
+    phi, dx, per = _phi(name)
+    dev, dx = torch.device("cuda", 0), dx * 1000.0
+    tphi = torch.from_numpy(np.ascontiguousarray(phi * 1000.0, np.float32)).to(dev)
+    mesh = flux.SurfaceMesh(dev).build(tphi, dx)
+    L = [n * dx for n in phi.shape]
+    box = ops.make_box(*L, L[2] - dx, per)
+    tree = ops.Bvh(dev).build(mesh.verts, mesh.faces)
+    bare = torch.full((mesh.nf,), 0.4, device=dev)
+    par = dict(PAR, ion_source="powcos", ion_exponent=20.0)
+
+    def run(b):
+        ops.trace_hit_counts(dev)
+        out = [ops.trace_neutral_rr(b, box, flux.NEUTRAL_SOURCE, bare, 0.5, 50000, 7).clone(),
+               ops.trace_ion_yield(b, box, flux.ion_source(par), flux.ion_params(par), 50000, 8)]
+        return out, ops.trace_hit_counts(dev)
+    (a, ha), (b, hb) = run(mesh.bvh), run(tree)
+    print(name, ha, hb, flush=True)
+    assert ha == hb and all(torch.equal(x, y) for x, y in zip(a, b))
