@@ -472,16 +472,22 @@ __device__ __forceinline__ float tie_lim(float m, float tb, float maxd2) {
 // chain of dependent node fetches, so the 4-wide nodes (half the binary tree's depth) and a stack
 // whose first entries are in LDS instead of scratch are what shortens it: one extension on an
 // AR-10 trench's surface 245 -> 219 us (183k queries of 18 nodes and 7 leaves); what is left is
-// the nodes' loads, 112 bytes a lane.
+// the nodes' loads, 112 bytes a lane. Returns false where an entry found no place on the stack: up
+// to three go on it a node, so a tree deeper than about 40 binary levels can run it over.
 template <class Stack, class Visit>
-__device__ __forceinline__ void point_walk(const BvhView& b, Vec3 p, float lim, Stack& stk,
+__device__ __forceinline__ bool point_walk(const BvhView& b, Vec3 p, float lim, Stack& stk,
                                            Visit visit) {
   int sp = 0, node = 0;
+  bool room = true;
+  auto push = [&](int c, float t) {
+    if (sp < kBvhStack) stk.put(sp++, c, t);
+    else room = false;
+  };
   const int max_steps = 2 * b.nf + 64;
   for (int steps = 0;; ++steps) {
     if (steps > max_steps || node < 0 || node >= b.nf - 1) {
       if (b.err) *b.err = 2;
-      return;
+      return room;
     }
     const BvhWide* N = b.wide + node;
     const float4 lx = N->lox, hx = N->hix, ly = N->loy, hy = N->hiy, lz = N->loz, hz = N->hiz;
@@ -511,25 +517,57 @@ __device__ __forceinline__ void point_walk(const BvhView& b, Vec3 p, float lim, 
     int next = -1;
     if (t3 <= lim && c3 >= 0) next = c3;
     if (t2 <= lim && c2 >= 0) {
-      if (next >= 0) push_far(b, stk, sp, next, t3);
+      if (next >= 0) push(next, t3);
       next = c2;
       t3 = t2;
     }
     if (t1 <= lim && c1 >= 0) {
-      if (next >= 0) push_far(b, stk, sp, next, t3);
+      if (next >= 0) push(next, t3);
       next = c1;
       t3 = t1;
     }
     if (t0 <= lim && c0 >= 0) {
-      if (next >= 0) push_far(b, stk, sp, next, t3);
+      if (next >= 0) push(next, t3);
       next = c0;
     }
     if (next < 0) {
       while (sp > 0 && !(stk.dist(sp - 1) <= lim)) --sp;
-      if (sp == 0) return;
+      if (sp == 0) return room;
       next = stk.node(--sp);
     }
     node = next;
+  }
+}
+
+// The same over the binary tree, one entry a node at most: the traversal of a query whose wide one
+// ran its stack over.
+template <class Stack, class Visit>
+__device__ __forceinline__ void point_walk_binary(const BvhView& b, Vec3 p, float lim, Stack& stk,
+                                                  Visit visit) {
+  int sp = 0, node = 0;
+  const int max_steps = 2 * b.nf + 64;
+  for (int steps = 0;; ++steps) {
+    if (steps > max_steps || node < 0 || node >= b.nf - 1) {
+      if (b.err) *b.err = 2;
+      return;
+    }
+    const BvhNode* N = b.nodes + node;
+    const float4 A = N->a, B = N->b, C = N->c;
+    int cn = N->d.x, cf = N->d.y;
+    float tn = box_dist2(p, A.x, A.y, A.z, A.w, B.x, B.y);
+    float tf = box_dist2(p, B.z, B.w, C.x, C.y, C.z, C.w);
+    sort2(tn, cn, tf, cf);
+    if (cn < 0 && tn <= lim && ~cn < b.nf) visit(~cn, lim);
+    if (cf < 0 && tf <= lim && ~cf < b.nf) visit(~cf, lim);
+    const bool hn = cn >= 0 && tn <= lim, hf = cf >= 0 && tf <= lim;
+    if (hn && hf) push_far(b, stk, sp, cf, tf);
+    if (hn || hf) {
+      node = hn ? cn : cf;
+      continue;
+    }
+    while (sp > 0 && !(stk.dist(sp - 1) <= lim)) --sp;
+    if (sp == 0) return;
+    node = stk.node(--sp);
   }
 }
 
@@ -549,7 +587,7 @@ struct PointTies {
 };
 
 template <class Stack>
-__device__ __forceinline__ void point_ties(const BvhView& b, Vec3 p, float maxd2, float tb,
+__device__ __forceinline__ bool point_ties(const BvhView& b, Vec3 p, float maxd2, float tb,
                                            Stack& stk, PointTies& T) {
   T.m = maxd2;
   T.ok = true;
@@ -558,7 +596,7 @@ __device__ __forceinline__ void point_ties(const BvhView& b, Vec3 p, float maxd2
     T.cf[j] = -1;
     T.cd[j] = INFINITY;
   }
-  point_walk(b, p, maxd2, stk, [&](int slot, float& lim) {
+  return point_walk(b, p, maxd2, stk, [&](int slot, float& lim) {
     int face;
     const float d2 = point_face_d2(b, p, slot, face);
     if (d2 < T.m) {
@@ -580,6 +618,29 @@ __device__ __forceinline__ void point_ties(const BvhView& b, Vec3 p, float maxd2
   });
 }
 
+// The whole query over the binary tree: the least squared distance m below maxd2, then the lowest
+// face id within the tie band of it.
+template <class Stack>
+__device__ __forceinline__ PointHit point_binary(const BvhView& b, Vec3 p, float maxd2, float tb,
+                                                 Stack& stk) {
+  PointHit t{-1, maxd2};
+  float m = maxd2, cut = maxd2;
+  for (int pass = 0; pass < 2; ++pass) {
+    point_walk_binary(b, p, cut, stk, [&](int slot, float& lim) {
+      int face;
+      const float d2 = point_face_d2(b, p, slot, face);
+      if (pass == 0) {
+        if (d2 < m) m = lim = d2;
+      } else if (d2 <= lim && (t.face < 0 || face < t.face)) {
+        t = PointHit{face, d2};
+      }
+    });
+    if (!(m < maxd2)) break;                      // no face below max_dist
+    cut = tie_lim(m, tb, maxd2);
+  }
+  return t;
+}
+
 // Closest face within max_dist (distance squared < max_dist^2), ties to the lowest face id. A
 // `hint` below max_dist, a distance within which the caller expects a face, bounds the traversal
 // from its first node; without a face (and its tie band) within it the query runs again without.
@@ -597,16 +658,16 @@ __device__ __forceinline__ PointHit bvh_closest_point(const BvhView& b, Vec3 p, 
   }
   const float tb = tie_band(p);
   PointTies T;
-  bool found = false;
+  bool found = false, room = true;
   if (hint < max_dist) {
     const float hint2 = hint * hint;
-    point_ties(b, p, hint2, tb, stk, T);
+    room = point_ties(b, p, hint2, tb, stk, T);
     found = T.m < hint2 && tie_lim(T.m, tb, maxd2) < hint2;
     if (found) maxd2 = hint2;
   }
   if (!found) {
-    point_ties(b, p, maxd2, tb, stk, T);
-    if (!(T.m < maxd2)) return h;                 // no face below max_dist
+    room = point_ties(b, p, maxd2, tb, stk, T) && room;
+    if (room && !(T.m < maxd2)) return h;         // no face below max_dist
   }
   const float lim = tie_lim(T.m, tb, maxd2);
   PointHit t{-1, T.m};
@@ -619,16 +680,16 @@ __device__ __forceinline__ PointHit bvh_closest_point(const BvhView& b, Vec3 p, 
       }
     }
   } else {
-    point_walk(b, p, lim, stk, [&](int slot, float&) {
+    room = point_walk(b, p, lim, stk, [&](int slot, float&) {
       int face;
       const float d2 = point_face_d2(b, p, slot, face);
       if (d2 <= lim && (t.face < 0 || face < t.face)) {
         t.face = face;
         t.d2 = d2;
       }
-    });
+    }) && room;
   }
-  return t;
+  return room ? t : point_binary(b, p, max_dist * max_dist, tb, stk);
 }
 
 }  // namespace petch
