@@ -14,6 +14,7 @@
 #include "fastdiv.h"
 #include "gridwalk.h"
 
+#include <algorithm>
 #include <vector>
 
 int* petch_bvh_err(const petch_bvh* b);
@@ -195,8 +196,8 @@ __global__ void k_grid_x_many(const GridBuild* __restrict__ t, int n) {
 
 int max_axis(int x, int y, int z) { return x > y ? (x > z ? x : z) : (y > z ? y : z); }
 
-// Checks an item and grows its BVH's buffers (twice the request, as the tree's own: a regrowth
-// waits for the stream).
+// Checks an item and grows its BVH's buffers (a regrowth waits for the stream). The BVH has no grid
+// until grid_done, so that a call that fails on the way leaves it to its tree.
 int grid_prepare(petch_ctx* ctx, const petch_grid_item& a, GridBuild& b) {
   PETCH_ARG(ctx, a.bvh && a.bvh->nf > 0 && a.verts && a.faces && a.cells,
             "bvh_set_grid: null pointer or no faces");
@@ -205,6 +206,7 @@ int grid_prepare(petch_ctx* ctx, const petch_grid_item& a, GridBuild& b) {
   PETCH_ARG(ctx, N < (1LL << 30) && (long long)a.nx * a.ny < (1LL << 24) && a.bvh->nf < (1 << 28),
             "bvh_set_grid: more than 2^30-1 nodes, 2^24-1 columns or 2^28-1 faces");
   petch_bvh* v = a.bvh;
+  v->grid_n[0] = 0;
   if (v->cells_cap < (size_t)N) {
     PETCH_HIP(ctx, hipStreamSynchronize(ctx->stream));
     if (v->cells) (void)hipFree(v->cells);
@@ -293,6 +295,12 @@ extern "C" int petch_bvh_set_grid(petch_ctx* ctx, const petch_grid_item* item) {
 extern "C" int petch_bvh_set_grid_batch(petch_ctx* ctx, int n, const petch_grid_item* items) {
   PETCH_ARG(ctx, ctx && n >= 0 && (n == 0 || items), "bvh_set_grid_batch: null pointer or n < 0");
   if (n == 0) return PETCH_OK;
+  // (a BVH twice: growing its buffers for the second would free the first's)
+  std::vector<const petch_bvh*> seen((size_t)n);
+  for (int k = 0; k < n; ++k) seen[k] = items[k].bvh;
+  std::sort(seen.begin(), seen.end());
+  PETCH_ARG(ctx, std::adjacent_find(seen.begin(), seen.end()) == seen.end(),
+            "bvh_set_grid_batch: a BVH is listed twice");
   std::vector<GridBuild> t((size_t)n);
   long long first = 0, rest = 0;
   size_t bytes = 0;

@@ -140,6 +140,8 @@ def test_batch_of_grids_equals_the_single_surfaces(det):
     assert m.bvh.status() == 0
     with pytest.raises(PetchError):
         m.bvh.set_grid(m.verts, m.faces, (cells, 1, ny, nz, dx))
+    with pytest.raises(PetchError, match="twice"):
+        ops.bvh_set_grid_batch([meshes[k].bvh_item() for k in (1, 0, 1)])
 
 
 @pytest.mark.parametrize("name", NAMES)
