@@ -1050,6 +1050,18 @@ def knudsen_face_flux(phi, dx, sub_top, trench, centroids, gas_normals, areas, b
     return outs
 
 
+class DdaPlan:
+    """dda_march's rays (their ends are nodes of its grid) and what they were marched for."""
+
+    def __init__(self, words, made_for):
+        self.words = words
+        self.made_for = made_for
+
+    @staticmethod
+    def key(phi, dx, F, n_dir, periodic_y):
+        return (*_shape3(phi), float(dx), int(F), int(n_dir), bool(periodic_y))
+
+
 def dda_march(phi, dx, centroids, gas_normals, n_dir=64, periodic_y=0):
     """The rays of dda_neutral_flux marched once (petch_dda_march), as a plan for any number of
     its calls on the same phi, dx, faces, n_dir and periodic_y."""
@@ -1062,7 +1074,7 @@ def dda_march(phi, dx, centroids, gas_normals, n_dir=64, periodic_y=0):
         _ctx(phi).call("petch_dda_march", ptr(phi, f32, "phi"), nx, ny, nz,
                        ptr(centroids, f32, "centroids"), ptr(gas_normals, f32, "gas_normals"), F,
                        ctypes_ref(p), ptr(plan))
-    return plan
+    return DdaPlan(plan, DdaPlan.key(phi, dx, F, n_dir, periodic_y))
 
 
 def dda_neutral_flux(phi, dx, centroids, gas_normals, areas, bare, betas, n_dir=64, n_reemit=12,
@@ -1076,6 +1088,9 @@ def dda_neutral_flux(phi, dx, centroids, gas_normals, areas, bare, betas, n_dir=
     betas = list(betas)
     if not 1 <= len(betas) <= 2:
         raise ValueError("dda_neutral_flux: one or two betas")
+    if plan is not None and plan.made_for != DdaPlan.key(phi, dx, F, n_dir, periodic_y):
+        raise ValueError("dda_neutral_flux: the plan is of another grid, number of faces, n_dir or "
+                         "period")
     outs = [torch.empty((F,), dtype=f32, device=phi.device) for _ in betas]
     p = DdaParams(float(dx), int(n_dir), int(n_reemit), int(bool(periodic_y)), float(betas[0]),
                   float(betas[-1]))
@@ -1084,9 +1099,7 @@ def dda_neutral_flux(phi, dx, centroids, gas_normals, areas, bare, betas, n_dir=
                 ptr(gas_normals, f32, "gas_normals"), ptr(areas, f32, "areas"),
                 ptr(bare, f32, "bare"), F, ctypes_ref(p)]
         if plan is not None:
-            if plan.numel() != 6 * int(n_dir) + F * (1 + 2 * int(n_dir)):
-                raise ValueError("dda_neutral_flux: the plan is of another surface or n_dir")
-            args.append(ptr(plan, i32, "plan"))
+            args.append(ptr(plan.words, i32, "plan"))
         _ctx(phi).call("petch_dda_neutral_flux" if plan is None else "petch_dda_reemit", *args,
                        ptr(outs[0]), ptr(outs[1]) if len(outs) > 1 else None)
     return outs

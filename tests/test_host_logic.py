@@ -115,3 +115,19 @@ def test_gpu_path_fails_loudly_without_gpu():
     with pytest.raises(RuntimeError, match="no CPU fallback"):
         Context(0)
 
+
+
+def test_dda_plan_of_another_grid_is_refused():
+    """The ends of a plan's rays are nodes of the grid it was marched on: on a smaller one of as many
+    faces they would lie outside."""
+    import torch
+    from petch import ops
+    big, small = torch.zeros(8, 9, 10), torch.zeros(8, 9, 9)
+    F, n_dir = 5, 4
+    face = [torch.zeros(F, 3), torch.zeros(F, 3), torch.zeros(F), torch.zeros(F)]
+    words = torch.zeros(6 * n_dir + F * (1 + 2 * n_dir), dtype=torch.int32)
+    plan = ops.DdaPlan(words, ops.DdaPlan.key(big, 0.25, F, n_dir, 0))
+    for phi, dx, nd, per in ((small, 0.25, n_dir, 0), (big, 0.5, n_dir, 0), (big, 0.25, 5, 0),
+                             (big, 0.25, n_dir, 1)):
+        with pytest.raises(ValueError, match="plan"):
+            ops.dda_neutral_flux(phi, dx, *face, (0.5, 1.0), nd, 2, per, plan=plan)
