@@ -433,7 +433,8 @@ int petch_trace_ion_yield_batch(petch_ctx* ctx, int nfeat, const petch_ion_featu
  * its own launch shapes): their grid is CUs x min(blocks_per_cu, the kernel's occupancy limit)
  * workgroups; 0 (the default) means the occupancy limit. The fluxes do not depend on it (a ray's
  * stream is keyed by its id, not by the wavefront that takes it). petch_trace_occupancy_limit
- * reports the limit of the neutral trace kernel. Used by petch.autotune. */
+ * reports the limit of the neutral trace on a surface with a grid (petch_bvh_set_grid). Used by
+ * petch.autotune. */
 int petch_set_trace_occupancy(petch_ctx* ctx, int blocks_per_cu);
 int petch_trace_occupancy_limit(petch_ctx* ctx, int* blocks_per_cu);
 

@@ -2115,7 +2115,7 @@ extern "C" int petch_set_trace_occupancy(petch_ctx* ctx, int blocks_per_cu) {
 extern "C" int petch_trace_occupancy_limit(petch_ctx* ctx, int* blocks_per_cu) {
   PETCH_ARG(ctx, ctx && blocks_per_cu, "trace_occupancy_limit: null pointer");
   int per_cu = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)k_trace5<NeutralRR<BvhView>>, kBS,
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)k_trace5<NeutralRR<GridView>>, kBS,
                                                    0) != hipSuccess)
     return petch_set_error(ctx, PETCH_E_HIP, "trace_occupancy_limit: occupancy query failed");
   *blocks_per_cu = per_cu;

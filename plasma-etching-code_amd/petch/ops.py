@@ -37,7 +37,8 @@ def set_trace_occupancy(blocks_per_cu, device=None):
 
 
 def trace_occupancy_limit(device=None):
-    """The neutral trace kernel's workgroups per CU at full occupancy (petch_trace_occupancy_limit)."""
+    """Workgroups per CU of the neutral trace on a surface with a grid at full occupancy
+    (petch_trace_occupancy_limit)."""
     import ctypes
     dev = torch.device("cuda", torch.cuda.current_device()) if device is None else torch.device(device)
     out = ctypes.c_int(0)
