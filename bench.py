@@ -29,7 +29,7 @@ for _p in (os.path.join(ROOT, "plasma-etching-code_amd"), ROOT):
 
 METRIC = "3D etch steps/s & rays/s (1 feature, 64-batch); fwd+adjoint / fwd cost ratio"
 HBM_PEAK_GBS = 8000.0
-# Each k_trace_neutral_rr launch carries the F and the O rays of one fixed-point iteration
+# Each neutral trace launch carries the F and the O rays of one fixed-point iteration
 # (2 x 8M primary rays); a ray-hit of either species reads its 36 B triangle and 4 B bare value
 # and read-modify-writes its 4 B accumulator.
 NEUTRAL_BYTES_PER_HIT = 48.0     # 36 B triangle + 4 B bare + 8 B accumulator read-modify-write
@@ -75,11 +75,11 @@ def build_loop(n_steps, timer=None, autotune=True):
     return loop, (nx, ny, nz)
 
 
-TRAFFIC_FILE = os.path.join(ROOT, "profiles", "k_trace_neutral_rr_trench_ar10_traffic.txt")
+TRAFFIC_FILE = os.path.join(ROOT, "profiles", "neutral_walk_trench_ar10_traffic.txt")
 
 
 def measured_traffic():
-    """HBM bytes per k_trace_neutral_rr launch from the rocprofv3 FETCH_SIZE / WRITE_SIZE runs
+    """HBM bytes per launch of the neutral walk from the rocprofv3 FETCH_SIZE / WRITE_SIZE runs
     summarised in profiles/ (KiB per dispatch, each scaled by what the same counter reads for
     a plain device copy of known size). None when no summary is present."""
     try:
@@ -620,7 +620,7 @@ def main(argv=None):
         "rays_per_s": rays_step * a.steps / wall,
         "ray_hits_per_s": (hits_n + hits_i) / wall,
         "stages_ms_per_step": {k: v / a.steps for k, v in sorted(timer.ms.items())},
-        "roofline": {"kernel": "k_trace_neutral_rr", "bound": "hbm", "achieved": achieved,
+        "roofline": {"kernel": "k_trace5<NeutralRR<GridView>>", "bound": "hbm", "achieved": achieved,
                      "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS,
                      "traffic": traffic, "traffic_source": traffic_src,
                      "avg_launch_ms": avg_launch_ms,

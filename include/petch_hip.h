@@ -279,9 +279,10 @@ int petch_bvh_build_batch(petch_ctx* ctx, int n, petch_bvh* const* bvhs_host,
 int petch_bvh_set_quality(petch_ctx* ctx, petch_bvh* bvh, int quality);
 /* Tells a built BVH that its mesh is the marching-cubes surface of an (nx, ny, nz) grid of spacing
  * dx: every triangle lies in one cell, whose word in `cells` (petch_marching_cubes_cells, the same
- * verts and faces) lists it. Ray traces and queries then walk the cells instead of the tree, with the
- * same hits; point queries keep the tree. The BVH keeps copies of all it needs; a new build
- * forgets the grid. A triangle outside its cell sets the guard flag (code 4). No reference
+ * verts and faces) lists it. Ray queries and the traces (all but petch_trace_legacy) then walk the
+ * cells instead of the tree, with the same hits; point queries keep the tree, and so do rays that
+ * meet two faces at one distance or start far outside the grid. The BVH keeps copies of all it
+ * needs; a new build forgets the grid, a call that fails leaves the BVH without one. A triangle outside its cell sets the guard flag (code 4). No reference
  * counterpart. */
 typedef struct petch_grid_item {
   petch_bvh* bvh;

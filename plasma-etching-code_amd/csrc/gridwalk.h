@@ -10,15 +10,15 @@
 // around it; in an occupied cell it tests the cell's triangles (ray_tri, the test of the BVH
 // leaves) and is done once its best hit lies before the cell's exit. Against the 4-wide tree this
 // takes about as many steps per query (6.6 and 3.1 triangle tests against 8.1 and 1.5, AR-10
-// trench), but a step is one dependent 4-byte load and 70 instructions instead of a 112-byte node
-// and 200, and the triangle tests of many lanes are batched. Whole fluxes: 6.97 -> 5.60 ms (hole,
-// 200k rays a species), 7.39 -> 5.17 ms (60x10x240 trench, 1M), one step of the AR-10 trench with
-// 88M rays 73.2 -> 62.4 ms; what bounds the small ones is the longest ray's chain of steps.
+// trench), but a step is one dependent 4-byte load instead of a 112-byte node and a third of its
+// instructions, and the triangle tests of many lanes are batched. Whole fluxes: 6.78 -> 5.60 ms
+// (hole, 200k rays a species), 6.98 -> 5.22 ms (60x10x240 trench, 1M), one step of the AR-10 trench
+// with 88M rays 73.3 -> 63.0 ms; what bounds the small ones is the longest ray's chain of steps.
 //
 // Hits are the tree's, by the same triangle test, but where a ray meets two faces at one distance
 // (an edge or a vertex, met exactly): there the tree takes the face that its traversal tests
 // first. A walk notes such a tie, and the caller leaves the ray to the tree; one query in ten
-// million ends so.
+// million ends so where faces don't coincide.
 //
 // Rounding. A plane crossing or a position is exact to a few ulps of the coordinates, 3e-5 of a
 // cell at 260 cells, and a triangle's vertices lie within as much of its cell; eps, 1e-4 of a cell

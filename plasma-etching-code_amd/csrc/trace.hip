@@ -5,8 +5,8 @@
 // divergent query lengths nor divergent bounce and wrap counts idle the wavefront for long.
 // Deposits go to per-face float accumulators with hardware float atomics.
 //
-//   k_trace_neutral_rr   _trace3d_cov_rr    threed.py:549-596 (RR-weighted neutral, <= 1024 bounces)
-//   k_trace_ion_yield    _trace3d_ion_yield threed.py:599-712 (faithful ion, 5 deposits per hit)
+//   NeutralRR            _trace3d_cov_rr    threed.py:549-596 (RR-weighted neutral, <= 1024 bounces)
+//   IonYield             _trace3d_ion_yield threed.py:599-712 (faithful ion, 5 deposits per hit)
 //   k_trace_legacy       _trace3d           threed.py:352-406 (sticking neutral / specular ion)
 //   k_trace_ff           _trace_ff          threed.py:908-920 (first hit of face-emitted rays)
 //   k_gen_source         _gen_source        threed.py:441-458 (same streams, for checking)
@@ -302,6 +302,10 @@ __device__ __forceinline__ bool claim_ray(const RayQueue& q, bool active, bool& 
 // comes from that ray's own Philox stream in a fixed order, so the result does not depend on
 // the schedule.
 constexpr int kRefillAt = 24;
+// The walk's: lanes a wavefront uses at least (4 / 8 / 16: the hole's flux of 200k rays a species
+// 5.5-5.8 / 5.6-5.7 / 5.6-5.8 ms), triangle tests and cell steps between two looks at what most
+// lanes wait for (1 and 3: 5.8-6.1 ms, 4 and 3, 2 and 1, 2 and 6: 5.6-5.8), workgroups of the ties'
+// launch (4 / 64: flat; for a launch that left many rays to the tree).
 constexpr int kMinLanes = 8;
 constexpr int kTestsPerPhase = 2, kStepsPerPhase = 3;
 constexpr int kTieBlocks = 64;

@@ -5,8 +5,10 @@ Two choices are tuned, per surface-size and ray-budget bucket (powers of two of 
 and of the rays per trace):
 - the BVH build (petch_bvh_set_quality): the Morton tree with the fixed 4-wide collapse (0),
   with the area-driven collapse (1), or the clustered (PLOC) tree with the area-driven collapse
-  (2). A better tree costs more to build and saves trace time; a run rebuilds its tree every
-  step, so a candidate's score is its build time plus its trace time;
+  (2). A better tree costs more to build and saves the time of traces on it (a surface's traces
+  walk its grid and leave the tree the ties, so there the builds differ by little but their own
+  time); a run rebuilds its tree every step, so a candidate's score is its build time plus its
+  trace time;
 - the persistent trace grid (petch_set_trace_occupancy): workgroups per CU, from the kernels'
   occupancy limit down by one and two (fewer resident rays share the caches among fewer).
 Every candidate gives the same fluxes: the tree only changes the order in which a query meets

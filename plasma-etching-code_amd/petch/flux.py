@@ -23,11 +23,14 @@ class SurfaceMesh:
     """The triangle surface of phi with everything the flux and extension stages need.
 
     Its ray traces walk the cells of phi's grid (Bvh.set_grid) and leave the tree the nearest-face
-    queries and the rays that meet two faces at once.
+    queries, the rays that meet two faces at once and the legacy trace.
 
-    rays_per_step (optional): the rays a step will trace on this surface. A clustered BVH
-    (slower build, faster traces) pays off from ~1000 rays per face; below that the fast
-    Morton build is used. Without it the BVH picks by mesh size."""
+    rays_per_step (optional): the rays a step will trace on this surface. From 1000 rays per face the
+    BVH is clustered, below that the fast Morton build is used; without it the BVH picks by mesh
+    size. The line dates from traces on the tree, which the clustered build made 4 % faster; with
+    the walk it costs build time (0.22 ms at 47k faces). It stays so that runs without the tuner
+    (petch.autotune, which picks by measurement) keep their trees, and with them the faces that
+    tied rays take."""
 
     def __init__(self, device, rays_per_step=None):
         self.device = device
