@@ -460,8 +460,8 @@ class EtchLoop:
     def begin_mesh(self, step, mc=None, bvh=True, staged=False):
         """Mesh + BVH of the step. Returns the device flag 'all centroids finite' that gates the
         warm start (threed.py:1699), or None when the step needs no warm start. mc: this step's
-        marching-cubes (verts, faces) when the caller already extracted them (the batched loop
-        meshes all features with one host read); bvh=False leaves the BVH to the caller (the
+        marching-cubes (verts, faces) when the caller already extracted them (they come without
+        their grid's cells, so rays are traced on the tree); bvh=False leaves the BVH to the caller (the
         batched loop builds all features' trees together); staged: the surface was built by
         stage_mesh and ops.surface_build_batch."""
         T, dx = self.timer, self.dx
