@@ -471,23 +471,22 @@ __device__ __forceinline__ float tie_lim(float m, float tb, float maxd2) {
 // `lim` of p (squared; visit(slot, lim) may lower it) and drops the rest unfetched. A query is a
 // chain of dependent node fetches, so the 4-wide nodes (half the binary tree's depth) and a stack
 // whose first entries are in LDS instead of scratch are what shortens it: one extension on an
-// AR-10 trench's surface 245 -> 219 us (183k queries of 18 nodes and 7 leaves); what is left is
+// AR-10 trench's surface 243 -> 220 us (183k queries of 18 nodes and 7 leaves); what is left is
 // the nodes' loads, 112 bytes a lane. Returns false where an entry found no place on the stack: up
 // to three go on it a node, so a tree deeper than about 40 binary levels can run it over.
 template <class Stack, class Visit>
 __device__ __forceinline__ bool point_walk(const BvhView& b, Vec3 p, float lim, Stack& stk,
                                            Visit visit) {
   int sp = 0, node = 0;
-  bool room = true;
   auto push = [&](int c, float t) {
     if (sp < kBvhStack) stk.put(sp++, c, t);
-    else room = false;
+    else lim = -1.f;   // nothing is in range any more
   };
   const int max_steps = 2 * b.nf + 64;
   for (int steps = 0;; ++steps) {
     if (steps > max_steps || node < 0 || node >= b.nf - 1) {
       if (b.err) *b.err = 2;
-      return room;
+      return true;
     }
     const BvhWide* N = b.wide + node;
     const float4 lx = N->lox, hx = N->hix, ly = N->loy, hy = N->hiy, lz = N->loz, hz = N->hiz;
@@ -532,7 +531,7 @@ __device__ __forceinline__ bool point_walk(const BvhView& b, Vec3 p, float lim, 
     }
     if (next < 0) {
       while (sp > 0 && !(stk.dist(sp - 1) <= lim)) --sp;
-      if (sp == 0) return room;
+      if (sp == 0) return lim >= 0.f;
       next = stk.node(--sp);
     }
     node = next;
